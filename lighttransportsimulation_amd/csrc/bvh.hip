@@ -30,7 +30,7 @@ constexpr int kBlock = 256;
 // of bounds.
 constexpr int kStatusClimb = 8;   // a climb took more steps than its bound
 constexpr int kStatusSort = 16;   // a radix scatter found inconsistent digit counts
-constexpr int kStatusTree = 32;   // packing found a child index outside the tree
+constexpr int kStatusTree = 32;   // packing or the render tree's check found a child index outside the tree
 
 __device__ __forceinline__ uint32_t order_key(float f) {
     uint32_t u = __float_as_uint(f);
@@ -538,7 +538,7 @@ struct TreeL1Fetch {
 __device__ __forceinline__ void tree_l1_fetch(TreeL1Fetch& f, const uint32_t* __restrict__ codes,
                                               const float* __restrict__ primBox, const int32_t* __restrict__ perm,
                                               int n, int mode, int chunk, int t) {
-    // every load is unconditional, at clamped in-range addresses (lanes past the end reload the last
+    // every load is unconditional, at clamped in range addresses (lanes past the end reload the last
     // entries), so no branch joins the loaded registers and nothing waits for them until they are used
     const int cs = chunk * kChunk, m = min(kChunk, n - cs);
     int pk[2] = {0, 0};
@@ -968,22 +968,17 @@ inline int bound_blocks(long n) { return std::min(blocks_for(n), 2048); }
 // ---------------------------------------------------------------- 4-wide render BVH
 constexpr int kScanBlock = 1024;
 
-// flag[i] = 1 when interior node i has even depth (the root has depth 0); maxDepth (when given)
-// receives the deepest level of a child, i.e. the tree depth counted in edges down to the leaves.
-__global__ __launch_bounds__(kBlock) void k_even_depth(const int32_t* __restrict__ parent, int n, int32_t* __restrict__ flag,
-                                                       int32_t* __restrict__ maxDepth) {
+// *maxDepth: the deepest level of a child, i.e. the tree depth counted in edges down to the leaves.
+__global__ __launch_bounds__(kBlock) void k_tree_depth(const int32_t* __restrict__ parent, int n, int32_t* __restrict__ maxDepth) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     int depth = -1;
     if (i < n - 1) {
         depth = 0;
         for (int node = i; node > 0 && depth < 2 * n; node = parent[node]) depth++;
-        flag[i] = (depth & 1) == 0;
     }
-    if (maxDepth) {
-        int d = depth + 1;
-        for (int o = 32; o > 0; o >>= 1) d = max(d, __shfl_xor(d, o));
-        if ((threadIdx.x & 63) == 0 && d > 0) atomicMax(maxDepth, d);
-    }
+    int d = depth + 1;
+    for (int o = 32; o > 0; o >>= 1) d = max(d, __shfl_xor(d, o));
+    if ((threadIdx.x & 63) == 0 && d > 0) atomicMax(maxDepth, d);
 }
 
 // In-place exclusive prefix sum of v[0, m) within blocks of kScanBlock; totals[block] = block sum.
@@ -1018,161 +1013,181 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_add(int32_t* __restrict__ v
     if (i < m) v[i] += totals[blockIdx.x];
 }
 
-// Smallest exponent e in [-126, 127] with qdecode(o, e, 255) >= hi.
-__device__ int q_exponent(float o, float hi) {
+// x - o without rounding, as s + err with s the nearest double (Knuth's two-sum): planes o + q 2^e are
+// compared with x as q 2^e (exact in fp64) against it.
+struct ExactGap { double s, err; };
+__device__ __forceinline__ ExactGap exact_gap(float x, float o) {
+    const double a = x, b = -(double)o, s = a + b, bb = s - a;
+    return ExactGap{s, (a - (s - bb)) + (b - bb)};
+}
+__device__ __forceinline__ bool plane_at_most(int q, double step, const ExactGap& g) {
+    const double p = q * step;
+    return p < g.s || (p == g.s && g.err >= 0);
+}
+__device__ __forceinline__ bool plane_at_least(int q, double step, const ExactGap& g) {
+    const double p = q * step;
+    return p > g.s || (p == g.s && g.err <= 0);
+}
+__device__ __forceinline__ double pow2(int e) { return __longlong_as_double((long long)(e + 1023) << 52); }
+
+// Smallest exponent e in [-126, 127] whose plane 255 reaches the gap.
+__device__ int q_exponent(const ExactGap& g) {
     int e = -126;
-    const float ext = hi - o;
-    if (ext > 0) {
+    if (g.s > 0) {
         int ee;
-        (void)frexpf(ext / 255.0f, &ee);  // ext / 255 < 2^ee
+        (void)frexp(g.s / 255.0, &ee);  // s / 255 < 2^ee
         e = max(-126, min(127, ee));
     }
-    while (e < 127 && !(qdecode(o, e, 255) >= hi)) e++;
-    while (e > -126 && qdecode(o, e - 1, 255) >= hi) e--;
+    while (e < 127 && !plane_at_least(255, pow2(e), g)) e++;
+    while (e > -126 && plane_at_least(255, pow2(e - 1), g)) e--;
     return e;
 }
 
-// Largest q with qdecode(o, e, q) <= lo (q = 0 always qualifies: o is the node's minimum).
-__device__ unsigned q_floor(float o, int e, float lo) {
-    const float d = (lo - o) / __int_as_float((e + 127) << 23);
-    int q = d > 0 ? (int)fminf(floorf(d), 255.0f) : 0;
-    while (q > 0 && qdecode(o, e, q) > lo) q--;
-    while (q < 255 && qdecode(o, e, q + 1) <= lo) q++;
+// Largest q whose plane does not pass the gap (0 qualifies: the origin is the node's minimum).
+__device__ unsigned q_floor(int e, const ExactGap& g) {
+    const double step = pow2(e);
+    int q = (int)fmin(fmax(floor(g.s * pow2(-e)), 0.0), 255.0);
+    while (q > 0 && !plane_at_most(q, step, g)) q--;
+    while (q < 255 && plane_at_most(q + 1, step, g)) q++;
     return (unsigned)q;
 }
 
-// Smallest q with qdecode(o, e, q) >= hi (q = 255 always qualifies by the choice of e).
-__device__ unsigned q_ceil(float o, int e, float hi) {
-    const float d = (hi - o) / __int_as_float((e + 127) << 23);
-    int q = d > 0 ? (int)fminf(ceilf(d), 255.0f) : 0;
-    while (q < 255 && qdecode(o, e, q) < hi) q++;
-    while (q > 0 && qdecode(o, e, q - 1) >= hi) q--;
+// Smallest q whose plane reaches the gap (255 qualifies by the choice of e).
+__device__ unsigned q_ceil(int e, const ExactGap& g) {
+    const double step = pow2(e);
+    int q = (int)fmin(fmax(ceil(g.s * pow2(-e)), 0.0), 255.0);
+    while (q < 255 && !plane_at_least(q, step, g)) q++;
+    while (q > 0 && plane_at_least(q - 1, step, g)) q--;
     return (unsigned)q;
 }
 
-// The quantized 4-wide node of `cnt` children with exact boxes mn / mx: the origin is the minimum
-// corner of their union, per axis the smallest exponent that reaches the maximum corner, then each
-// child's planes rounded outwards (q_floor / q_ceil).
-__device__ BvhQNode quantize_node(const int (&ch)[4], const float (&mn)[4][3], const float (&mx)[4][3], int cnt) {
-    BvhQNode o;
-    float org[3];
-    int ex[3];
+// The node record of `cnt` children with exact boxes mn / mx (TraceRec; the first child's number is
+// written by k_collapse_emit): the origin is the minimum corner of their union, per axis the smallest
+// exponent reaches the maximum corner, and each child's planes enclose its box in exact arithmetic
+// (the traversal's rounding margins are its own). A flat child at the minimum corner stays flat.
+__device__ TraceRec quantize_node(const bool (&leaf)[4], const float (&mn)[4][3], const float (&mx)[4][3], int cnt) {
+    TraceRec o;
+    uint32_t head = (uint32_t)cnt << 24;
     for (int a = 0; a < 3; a++) {
         float lo = mn[0][a], hi = mx[0][a];
         for (int k = 1; k < cnt; k++) { lo = fminf(lo, mn[k][a]); hi = fmaxf(hi, mx[k][a]); }
-        org[a] = lo;
-        ex[a] = q_exponent(lo, hi);
-    }
-    o.ox = org[0]; o.oy = org[1]; o.oz = org[2];
-    o.ex = (int8_t)ex[0]; o.ey = (int8_t)ex[1]; o.ez = (int8_t)ex[2];
-    o.count = (uint8_t)cnt;
-    for (int k = 0; k < 4; k++) {
-        const bool valid = k < cnt;
-        o.child[k] = valid ? ch[k] : 0;
-        for (int a = 0; a < 3; a++) {
-            o.qlo[a][k] = valid ? (uint8_t)q_floor(org[a], ex[a], mn[k][a]) : 0;
-            o.qhi[a][k] = valid ? (uint8_t)q_ceil(org[a], ex[a], mx[k][a]) : 0;
+        const int e = q_exponent(exact_gap(hi, lo));
+        o.w[a] = __float_as_uint(lo);
+        head |= ((uint32_t)e & 0xffu) << (8 * a);
+        uint32_t ql = 0, qh = 0;
+        for (int k = 0; k < cnt; k++) {
+            ql |= q_floor(e, exact_gap(mn[k][a], lo)) << (8 * k);
+            qh |= q_ceil(e, exact_gap(mx[k][a], lo)) << (8 * k);
         }
+        o.w[4 + a] = ql;
+        o.w[7 + a] = qh;
     }
-    o.pad[0] = o.pad[1] = 0;
+    for (int k = 0; k < cnt; k++)
+        if (leaf[k]) head |= 0x80000000u >> k;
+    o.w[3] = head;
+    o.w[10] = 0;
+    o.w[11] = 0xffffffffu;
     return o;
 }
 
-__global__ __launch_bounds__(kBlock) void k_build_bvh4(const BvhNode* __restrict__ nodes, const int32_t* __restrict__ flag,
-                                                       const int32_t* __restrict__ index4, int n, BvhQNode* __restrict__ out) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n - 1 || !flag[i]) return;
-    const BvhNode nd = nodes[i];
-    int ch[4];
-    float mn[4][3], mx[4][3];
-    int cnt = 0;
-    auto add = [&](int c, const float* lo, const float* hi) {
-        ch[cnt] = c >= n - 1 ? ~(c - (n - 1)) : index4[c];
-        for (int a = 0; a < 3; a++) { mn[cnt][a] = lo[a]; mx[cnt][a] = hi[a]; }
-        cnt++;
-    };
-    for (int side = 0; side < 2; side++) {
-        const int c = side ? nd.right : nd.left;
-        const float* lo = side ? nd.rmin : nd.lmin;
-        const float* hi = side ? nd.rmax : nd.lmax;
-        if (c >= n - 1) {
-            add(c, lo, hi);
-        } else {
-            const BvhNode g = nodes[c];  // odd depth: replaced by its two children
-            add(g.left, g.lmin, g.lmax);
-            add(g.right, g.rmin, g.rmax);
-        }
-    }
-    out[index4[i]] = quantize_node(ch, mn, mx, cnt);
-}
-
-// Greedy surface-area collapse, one level of the 4-wide tree per launch (breadth first). Frontier
-// entry t is binary interior node front[t]; it becomes 4-wide node levelStart + t, whose children
-// start as the binary node's two children, then the interior child of largest surface area is
-// replaced by its two children until there are four or only leaves are left. Leaf children are
-// stored as ~leaf; the interior ones are listed in tmp[4 t + slot] (-1 elsewhere) and counted in
-// cnt[t], and k_collapse_emit numbers them once cnt holds their exclusive prefix.
+// One level of the 4-wide tree per launch, breadth first. Frontier entry t (unified index of the binary
+// tree) becomes record levelStart + t. A leaf becomes its triangle's record. A node's children start as
+// the binary node's two; then, greedily, the interior child of largest surface area is replaced by its
+// two children until there are four or only leaves are left, or (even) each of the two that is interior
+// is replaced once. The children are listed in tmp[4 t ..] and counted in cnt[t]; k_collapse_emit
+// numbers them once cnt holds their exclusive prefix.
 __global__ __launch_bounds__(kBlock) void k_collapse_count(const int32_t* __restrict__ front, int count,
-                                                           const BvhNode* __restrict__ nodes, int n, int levelStart,
-                                                           int32_t* __restrict__ tmp, int32_t* __restrict__ cnt,
-                                                           BvhQNode* __restrict__ out) {
+                                                           const BvhNode* __restrict__ nodes, const TriLeaf* __restrict__ tris,
+                                                           int n, int levelStart, bool even, int32_t* __restrict__ tmp,
+                                                           int32_t* __restrict__ cnt, TraceRec* __restrict__ out) {
     const int t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= count) return;
-    const BvhNode nd = nodes[front[t]];
+    const int f = front[t];
+    if (f >= n - 1) {
+        const TriLeaf tl = tris[f - (n - 1)];
+        TraceRec r;
+        const float v[9] = {tl.p0x, tl.p0y, tl.p0z, tl.p1x, tl.p1y, tl.p1z, tl.p2x, tl.p2y, tl.p2z};
+        for (int q = 0; q < 9; q++) r.w[q] = __float_as_uint(v[q]);
+        r.w[9] = (uint32_t)tl.prim;
+        r.w[10] = 0;
+        r.w[11] = (uint32_t)(f - (n - 1));
+        out[levelStart + t] = r;
+        cnt[t] = 0;
+        return;
+    }
+    const BvhNode nd = nodes[f];
     int id[4];
     float mn[4][3], mx[4][3];
     auto put = [&](int k, int c, const float* lo, const float* hi) {
         id[k] = c;
         for (int a = 0; a < 3; a++) { mn[k][a] = lo[a]; mx[k][a] = hi[a]; }
     };
-    put(0, nd.left, nd.lmin, nd.lmax);
-    put(1, nd.right, nd.rmin, nd.rmax);
-    int c = 2;
-    while (c < 4) {
-        int best = -1;
-        float bestArea = -1.0f;
-        for (int k = 0; k < c; k++) {
-            if (id[k] >= n - 1) continue;
-            const float dx = mx[k][0] - mn[k][0], dy = mx[k][1] - mn[k][1], dz = mx[k][2] - mn[k][2];
-            const float area = dx * dy + dy * dz + dz * dx;
-            if (area > bestArea) { bestArea = area; best = k; }
-        }
-        if (best < 0) break;
-        const BvhNode g = nodes[id[best]];
-        put(best, g.left, g.lmin, g.lmax);
+    int c = 0;
+    auto open = [&](int k, int node) {
+        const BvhNode g = nodes[node];
+        put(k, g.left, g.lmin, g.lmax);
         put(c, g.right, g.rmin, g.rmax);
         c++;
+    };
+    put(0, nd.left, nd.lmin, nd.lmax);
+    put(1, nd.right, nd.rmin, nd.rmax);
+    c = 2;
+    if (even) {
+        if (nd.left < n - 1) open(0, nd.left);
+        if (nd.right < n - 1) open(1, nd.right);
+    } else {
+        while (c < 4) {
+            int best = -1;
+            float bestArea = -1.0f;
+            for (int k = 0; k < c; k++) {
+                if (id[k] >= n - 1) continue;
+                const float dx = mx[k][0] - mn[k][0], dy = mx[k][1] - mn[k][1], dz = mx[k][2] - mn[k][2];
+                const float area = dx * dy + dy * dz + dz * dx;
+                if (area > bestArea) { bestArea = area; best = k; }
+            }
+            if (best < 0) break;
+            open(best, id[best]);
+        }
     }
-    int ch[4];
-    int interior = 0;
+    bool leaf[4];
     for (int k = 0; k < 4; k++) {
-        const bool leaf = k < c && id[k] >= n - 1;
-        ch[k] = leaf ? ~(id[k] - (n - 1)) : 0;
-        const bool inner = k < c && !leaf;
-        tmp[4 * t + k] = inner ? id[k] : -1;
-        interior += inner;
+        leaf[k] = k < c && id[k] >= n - 1;
+        tmp[4 * (size_t)t + k] = k < c ? id[k] : -1;
     }
-    out[levelStart + t] = quantize_node(ch, mn, mx, c);
-    cnt[t] = interior;
+    out[levelStart + t] = quantize_node(leaf, mn, mx, c);
+    cnt[t] = c;
 }
 
-// Numbers the interior children of the level's nodes (cnt now holds exclusive offsets): the j-th
-// interior child of entry t becomes node nextStart + cnt[t] + j and frontier entry cnt[t] + j.
-__global__ __launch_bounds__(kBlock) void k_collapse_emit(int count, const int32_t* __restrict__ tmp,
-                                                          const int32_t* __restrict__ cnt, int levelStart, int nextStart,
-                                                          BvhQNode* __restrict__ out, int32_t* __restrict__ next) {
+// Numbers the children of the level's nodes (cnt now holds exclusive offsets): the k-th child of entry t
+// becomes record nextStart + cnt[t] + k and frontier entry cnt[t] + k.
+__global__ __launch_bounds__(kBlock) void k_collapse_emit(int count, const int32_t* __restrict__ front, int n,
+                                                          const int32_t* __restrict__ tmp, const int32_t* __restrict__ cnt,
+                                                          int levelStart, int nextStart, TraceRec* __restrict__ out,
+                                                          int32_t* __restrict__ next) {
     const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= count) return;
-    int j = cnt[t];
-    for (int k = 0; k < 4; k++) {
-        const int c = tmp[4 * t + k];
-        if (c < 0) continue;
-        out[levelStart + t].child[k] = nextStart + j;
-        next[j] = c;
-        j++;
-    }
+    if (t >= count || front[t] >= n - 1) return;
+    out[levelStart + t].w[10] = (uint32_t)kRecUnits * (uint32_t)(nextStart + cnt[t]);
+    for (int k = 0; k < 4 && tmp[4 * (size_t)t + k] >= 0; k++) next[cnt[t] + k] = tmp[4 * (size_t)t + k];
 }
 
+// What the traversal relies on instead of testing it at every step: the records under a node come
+// after it and lie among the m records (so every traversal ends), the node's triangle bits tell its
+// children's kinds, and triangles name leaves below n.
+__global__ __launch_bounds__(kBlock) void k_check_recs(const TraceRec* __restrict__ recs, int m, int n, int32_t* __restrict__ status) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= m) return;
+    const uint32_t kind = recs[i].w[11];
+    bool ok;
+    if (kind == 0xffffffffu) {
+        const uint32_t head = recs[i].w[3], unit = recs[i].w[10], cnt = (head >> 24) & 7u, first = unit / kRecUnits;
+        ok = cnt >= 2 && cnt <= 4 && unit % kRecUnits == 0 && first > (uint32_t)i && first + cnt <= (uint32_t)m;
+        for (uint32_t k = 0; ok && k < cnt; k++)
+            ok = ((head << k) >> 31) == (recs[first + k].w[11] != 0xffffffffu ? 1u : 0u);
+    } else {
+        ok = kind < (uint32_t)n;
+    }
+    if (!ok || (i == 0 && (kind == 0xffffffffu) != (n > 1))) atomicOr(status, kStatusTree);
+}
 
 // ---------------------------------------------------------------- PLOC render tree
 // Parallel locally-ordered clustering (Meister & Bittner, IEEE TVCG 2018) over the Morton-ordered
@@ -1335,7 +1350,6 @@ hipError_t bvh_reserve(BvhBuffers& b, int n) {
     TRY(dalloc(&b.segBase, (size_t)kBins * sort_segments(n)));
     TRY(dalloc(&b.left, n)); TRY(dalloc(&b.right, n));
     TRY(dalloc(&b.parent, 2 * (size_t)n));
-    TRY(dalloc(&b.flags, n));
     TRY(dalloc(&b.slots, n));
     TRY(dalloc(&b.chunkRoot, (n + kChunk - 1) / kChunk));
     TRY(dalloc(&b.pend, n));
@@ -1352,40 +1366,40 @@ hipError_t bvh_reserve(BvhBuffers& b, int n) {
     return hipSuccess;
 }
 
-// Greedy surface-area collapse (k_collapse_count / k_collapse_emit), level by level from the root.
-// Returns the number of 4-wide nodes in *nodes4, or 0 when the tree has more than kTraceStack / 3
-// levels (a 4-wide node leaves at most 3 entries on the traversal stack).
-static hipError_t collapse_greedy(BvhBuffers& b, hipStream_t s, int* nodes4) {
-    const int n = b.n, m = n - 1;
-    *nodes4 = 0;
-    int32_t *fa = nullptr, *fb = nullptr, *cnt = nullptr, *tmp = nullptr;
-    hipError_t e = dalloc(&fa, m);
-    if (e == hipSuccess) e = dalloc(&fb, m);
-    if (e == hipSuccess) e = dalloc(&cnt, m);
-    if (e == hipSuccess) e = dalloc(&tmp, 4 * (size_t)m);
-    const int32_t root = 0;
+// The collapse (k_collapse_count / k_collapse_emit), level by level from the root. Returns the number
+// of records in *total, or 0 when the tree has more than kMaxNodeLevels levels of nodes.
+static hipError_t collapse(BvhBuffers& b, bool even, hipStream_t s, int* total) {
+    const int n = b.n;
+    *total = 0;
+    int32_t *fa = nullptr, *fb = nullptr, *cnt = nullptr, *tmp = nullptr, *totals = nullptr;
+    hipError_t e = dalloc(&fa, n);
+    if (e == hipSuccess) e = dalloc(&fb, n);
+    if (e == hipSuccess) e = dalloc(&cnt, n);
+    if (e == hipSuccess) e = dalloc(&tmp, 4 * (size_t)n);
+    if (e == hipSuccess) e = dalloc(&totals, (size_t)(n + kScanBlock - 1) / kScanBlock + 1);
+    const int32_t root = 0;  // interior node 0, or the only leaf of a one-triangle scene
     if (e == hipSuccess) e = hipMemcpyAsync(fa, &root, sizeof(root), hipMemcpyHostToDevice, s);
-    int levelStart = 0, count = 1, levels = 0;
-    while (e == hipSuccess && count > 0) {
-        if (3 * ++levels > kTraceStack) { levelStart = 0; break; }
+    int levelStart = 0, count = 1;
+    for (int level = 0; e == hipSuccess && count > 0; level++) {
         const int lb = (count + kScanBlock - 1) / kScanBlock;
-        k_collapse_count<<<blocks_for(count), kBlock, 0, s>>>(fa, count, b.nodes, n, levelStart, tmp, cnt, b.nodes4);
-        k_scan_local<<<lb, kScanBlock, 0, s>>>(cnt, count, b.scanTotals);
-        k_scan_totals<<<1, 64, 0, s>>>(b.scanTotals, lb);
-        k_scan_add<<<lb, kScanBlock, 0, s>>>(cnt, count, b.scanTotals);
-        k_collapse_emit<<<blocks_for(count), kBlock, 0, s>>>(count, tmp, cnt, levelStart, levelStart + count, b.nodes4, fb);
+        k_collapse_count<<<blocks_for(count), kBlock, 0, s>>>(fa, count, b.nodes, b.tris, n, levelStart, even, tmp, cnt, b.recs);
+        k_scan_local<<<lb, kScanBlock, 0, s>>>(cnt, count, totals);
+        k_scan_totals<<<1, 64, 0, s>>>(totals, lb);
+        k_scan_add<<<lb, kScanBlock, 0, s>>>(cnt, count, totals);
+        k_collapse_emit<<<blocks_for(count), kBlock, 0, s>>>(count, fa, n, tmp, cnt, levelStart, levelStart + count, b.recs, fb);
         int32_t next = 0;
         e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(&next, b.scanTotals + lb, sizeof(next), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(&next, totals + lb, sizeof(next), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         levelStart += count;
+        if (next > 0 && level >= kMaxNodeLevels) { levelStart = 0; break; }
         count = next;
         std::swap(fa, fb);
     }
-    void* ps[] = {fa, fb, cnt, tmp};
+    void* ps[] = {fa, fb, cnt, tmp, totals};
     for (void* p : ps)
         if (p) (void)hipFree(p);
-    if (e == hipSuccess) *nodes4 = levelStart;
+    if (e == hipSuccess) *total = levelStart;
     return e;
 }
 
@@ -1393,51 +1407,33 @@ hipError_t bvh4_enqueue(BvhBuffers& b, hipStream_t s, int* depth, int* nodes4, b
     const int n = b.n;
     *depth = 0;
     *nodes4 = 0;
-    if (n < 2) return hipSuccess;
-    const int m = n - 1;
-    const int nb = (m + kScanBlock - 1) / kScanBlock;
-    if (b.cap4 < n) {
-        void* ps[] = {b.nodes4, b.index4, b.scanTotals};
-        for (void* p : ps)
-            if (p) (void)hipFree(p);
-        b.nodes4 = nullptr; b.index4 = nullptr; b.scanTotals = nullptr; b.cap4 = 0;
-        hipError_t e = dalloc(&b.nodes4, m);
-        if (e == hipSuccess) e = dalloc(&b.index4, m);
-        if (e == hipSuccess) e = dalloc(&b.scanTotals, (size_t)nb + 2);
+    const size_t most = 2 * (size_t)n - 1;  // at most n - 1 nodes and n triangles
+    if (b.recCap < most) {
+        if (b.recs) (void)hipFree(b.recs);
+        b.recs = nullptr; b.recCap = 0;
+        const hipError_t e = dalloc(&b.recs, most);
         if (e != hipSuccess) return e;
-        b.cap4 = n;
+        b.recCap = most;
     }
-    // the binary tree's depth (and its even-depth flags, for the fallback collapse)
-    int32_t* depthDev = b.scanTotals + nb + 1;
-    hipError_t e = hipMemsetAsync(depthDev, 0, sizeof(int32_t), s);
-    if (e != hipSuccess) return e;
-    k_even_depth<<<blocks_for(m), kBlock, 0, s>>>(b.parent, n, b.flags, depthDev);
-    e = hipMemcpyAsync(depth, depthDev, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    const int binaryDepth = *depth;
+    hipError_t e;
+    if (n > 1) {  // the binary tree's depth
+        int32_t* dev = reinterpret_cast<int32_t*>(b.sceneKeys) + 6;  // two spare words
+        if ((e = hipMemsetAsync(dev, 0, sizeof(int32_t), s)) != hipSuccess) return e;
+        k_tree_depth<<<blocks_for(n - 1), kBlock, 0, s>>>(b.parent, n, dev);
+        e = hipMemcpyAsync(depth, dev, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+    }
+    int total = 0;
     if (!*even) {
-        if ((e = collapse_greedy(b, s, nodes4)) != hipSuccess) return e;
-        if (*nodes4 > 0) return hipSuccess;
-        *even = true;
+        if ((e = collapse(b, false, s, &total)) != hipSuccess) return e;
+        *even = total == 0;
     }
-    // fallback: every interior node of even depth becomes a 4-wide node (ceil(depth / 2) levels)
-    // flags -> exclusive prefix in index4 -> 4-wide nodes
-    e = hipMemcpyAsync(b.index4, b.flags, (size_t)m * sizeof(int32_t), hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) return e;
-    k_scan_local<<<nb, kScanBlock, 0, s>>>(b.index4, m, b.scanTotals);
-    k_scan_totals<<<1, 64, 0, s>>>(b.scanTotals, nb);
-    k_scan_add<<<nb, kScanBlock, 0, s>>>(b.index4, m, b.scanTotals);
-    k_build_bvh4<<<blocks_for(m), kBlock, 0, s>>>(b.nodes, b.flags, b.index4, n, b.nodes4);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    int32_t total = 0;  // scanTotals[nb] = 4-wide node count
-    e = hipMemcpyAsync(&total, b.scanTotals + nb, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    *nodes4 = total;
-    *depth = binaryDepth;
-    return hipSuccess;
+    // an even-depth collapse of a tree that is too deep for the stack is refused by the caller (*depth)
+    if (*even && *depth <= kMaxRenderDepth && (e = collapse(b, true, s, &total)) != hipSuccess) return e;
+    *nodes4 = std::max(total - n, 0);
+    if (total > 0) k_check_recs<<<blocks_for(total), kBlock, 0, s>>>(b.recs, total, n, b.status);
+    return hipGetLastError();
 }
 
 
@@ -1486,7 +1482,7 @@ hipError_t ploc_enqueue(BvhBuffers& b, hipStream_t s, int maxDepth, int* depthOu
     if (created != n - 1) { cleanup(); return hipErrorUnknown; }
     // depth in edges down to the deepest leaf
     TRY(hipMemsetAsync(totals + 2, 0, sizeof(int32_t), s));
-    k_even_depth<<<blocks_for(n - 1), kBlock, 0, s>>>(parent, n, b.flags, totals + 2);
+    k_tree_depth<<<blocks_for(n - 1), kBlock, 0, s>>>(parent, n, totals + 2);
     TRY(hipGetLastError());
     TRY(hipMemcpyAsync(host + 2, totals + 2, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     TRY(hipStreamSynchronize(s));
@@ -1505,8 +1501,8 @@ hipError_t ploc_enqueue(BvhBuffers& b, hipStream_t s, int maxDepth, int* depthOu
 
 void bvh_release(BvhBuffers& b) {
     void* ps[] = {b.primBox, b.box, b.keysA, b.keysB, b.valsA, b.valsB, b.counts, b.segBase,
-                  b.left, b.right, b.parent, b.flags, b.sceneKeys, b.nodes, b.tris, b.slots, b.pend, b.chunkRoot, b.chunkRec, b.root2, b.rec2, b.partial,
-                  b.nodes4, b.index4, b.scanTotals, b.status};
+                  b.left, b.right, b.parent, b.sceneKeys, b.nodes, b.tris, b.slots, b.pend, b.chunkRoot, b.chunkRec, b.root2, b.rec2, b.partial,
+                  b.recs, b.status};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     b = BvhBuffers();

@@ -952,15 +952,16 @@ static int load_scene_impl(lts_ctx* c, const char* dir, const char* scene, const
     std::vector<ShadeTri> shadeLeaf(n);
     for (int k = 0; k < n; k++) shadeLeaf[k] = H.shade[perm[k]];
     HIPCHK(c, upload(&S.shade, shadeLeaf.data(), shadeLeaf.size(), s));
-    HIPCHK(c, launch_tri_materials(S.bvh.tris, S.shade, n, s));
+    HIPCHK(c, launch_tri_materials(S.bvh.tris, S.shade, n, S.bvh.recs, nodes4 + n, s));
     std::vector<LightDesc> lights = H.lights;
     for (LightDesc& L : lights)
         if (L.kind == 0) L.leaf = leafOf[L.prim];
     HIPCHK(c, upload(&S.lights, lights.data(), lights.size(), s));
     SceneView& v = S.view;
-    v.tris = S.bvh.tris; v.nodes = S.bvh.nodes; v.nodes4 = S.bvh.nodes4; v.shade = S.shade; v.mats = S.mats; v.texs = S.texs;
+    v.tris = S.bvh.tris; v.nodes = S.bvh.nodes; v.recs = S.bvh.recs; v.shade = S.shade; v.mats = S.mats; v.texs = S.texs;
     v.mips = S.mips; v.mipData = S.mipData; v.lights = S.lights; v.lfunc = S.lfunc; v.lcdf = S.lcdf;
     v.funcInt = H.funcInt; v.nLights = (int)H.lights.size(); v.nPrim = n; v.infiniteLight = H.infiniteLight;
+    v.root = n == 1 ? INT32_MIN : 0;
     v.perm = c->perm;
     v.cam = H.cam;
     std::memcpy(v.filter, H.filter, sizeof(v.filter));

@@ -78,10 +78,11 @@ LTS_D float absDot(V3 a, V3 b) { return fabsf(dot(a, b)); }
 LTS_D float lengthSq(V3 a) { return a.x * a.x + a.y * a.y + a.z * a.z; }
 LTS_D float length(V3 a) { return sqrtf(lengthSq(a)); }
 LTS_D V3 vabs(V3 a) { return v3(fabsf(a.x), fabsf(a.y), fabsf(a.z)); }
-// geometry/Geometry.cuh:77-83 (fp64 cross product)
+// geometry/Geometry.cuh:77-83 (fp64 cross product). A product of two floats is exact in fp64, so the
+// fused form rounds once, where the reference's subtraction does: same value, two operations a component.
 LTS_D V3 cross(V3 a, V3 b) {
     double ax = a.x, ay = a.y, az = a.z, bx = b.x, by = b.y, bz = b.z;
-    return v3((float)((ay * bz) - (az * by)), (float)((az * bx) - (ax * bz)), (float)((ax * by) - (ay * bx)));
+    return v3((float)__builtin_fma(ay, bz, -(az * by)), (float)__builtin_fma(az, bx, -(ax * bz)), (float)__builtin_fma(ax, by, -(ay * bx)));
 }
 LTS_D V3 normalize(V3 a) { return a * quake(lengthSq(a)); }
 LTS_D V3 faceTowards(V3 n, V3 v) { return (dot(n, v) < 0.0f) ? -n : n; }
@@ -143,11 +144,5 @@ struct Sampler {
         out[0] = u01(r.a); out[1] = u01(r.b); out[2] = u01(r.c); out[3] = u01(r.d);
     }
 };
-
-// Decoded plane of a quantized render-node box: origin + q * 2^e. The product is exact (q has 8
-// bits and e is at least -126), so the only rounding is the addition, and the fused form is one
-// instruction; the builder evaluates this same expression when it picks q, which keeps decoded
-// boxes conservative.
-LTS_D float qdecode(float origin, int e, unsigned q) { return __builtin_fmaf((float)q, __int_as_float((e + 127) << 23), origin); }
 
 }  // namespace lts

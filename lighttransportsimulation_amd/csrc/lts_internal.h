@@ -42,7 +42,6 @@ struct BvhBuffers {
     int32_t* left = nullptr;      // n-1
     int32_t* right = nullptr;     // n-1
     int32_t* parent = nullptr;    // 2n-1
-    int32_t* flags = nullptr;     // n-1 (4-wide collapse)
     int32_t* slots = nullptr;     // n-1 arrival slot per split of the bottom-up hierarchy
     ClimbRec* pend = nullptr;     // n-1: the node waiting at a split (written where a slot is set)
     int32_t* chunkRoot = nullptr; // per 512-leaf chunk: last leaf of the node its climbs handed on, or -1
@@ -54,21 +53,18 @@ struct BvhBuffers {
     int32_t* status = nullptr;    // failed bounded waits of the last build (bits; 0 = none)
     BvhNode* nodes = nullptr;     // n-1 (or 1 for n == 1)
     TriLeaf* tris = nullptr;      // n
-    BvhQNode* nodes4 = nullptr;   // 4-wide collapse for rendering (allocated by bvh4_enqueue)
-    int32_t* index4 = nullptr;    // n-1: 4-wide node of each even-depth interior node
-    int32_t* scanTotals = nullptr;
-    int cap4 = 0;
+    TraceRec* recs = nullptr;     // render tree: 4-wide nodes and triangles (allocated by bvh4_enqueue)
+    size_t recCap = 0;
     // results after the sort: sorted codes and permutation live in keysA / valsA
 };
 
 hipError_t bvh_reserve(BvhBuffers& b, int n);
 void bvh_release(BvhBuffers& b);
-// Collapses the packed tree of the last build (mode 1, pack) into the 4-wide render BVH: interior
-// nodes of even depth become 4-wide nodes (numbered in interior order, so the root is node 0) and
-// take the boxes of their children's children. Deterministic. Waits for the stream and returns
-// the tree's depth (edges down to the deepest leaf) and the 4-wide node count.
-// 4-wide render nodes of the binary tree in b (greedy surface-area collapse, or the even-depth
-// collapse when *even is set on entry or the greedy tree is too deep; *even tells which was used).
+// Render records of the packed tree of the last build (mode 1, pack): its binary tree collapsed into
+// 4-wide nodes level by level, greedily by surface area, or by opening both children once (the
+// even-depth collapse) when *even is set on entry or the greedy tree has too many levels (*even tells
+// which was used). Deterministic. Waits for the stream and returns the binary tree's depth (edges
+// down to the deepest leaf) and the 4-wide node count.
 hipError_t bvh4_enqueue(BvhBuffers& b, hipStream_t stream, int* depth, int* nodes4, bool* even);
 // Render tree of a scene: PLOC over the sorted leaves of the last bvh_enqueue (which must have run
 // with pack). When the PLOC tree is at most maxDepth deep it replaces b.nodes and b.parent (the
@@ -122,8 +118,9 @@ hipError_t launch_bdpt(const SceneView& sv, const RenderLaunch& rl, hipStream_t 
 hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);
 hipError_t launch_film_clear(float* film, int npix, hipStream_t stream);
 hipError_t launch_trace_rays(const SceneView& sv, const float* rays, int n, int32_t* prim, float* t, hipStream_t stream);
-// tris[k].mat = shade[k].mat for the n leaves of a loaded scene (shade is in leaf order).
-hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, hipStream_t stream);
+// The material of each of the n leaves of a loaded scene (shade is in leaf order) into its triangle and
+// its render record (nRecs records).
+hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t stream);
 hipError_t launch_get_render(const SceneView& sv, const float* film, float* rgb, hipStream_t stream);
 // plain copy of `bytes` (a multiple of 16) with 16-byte vector loads and stores
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
@@ -147,8 +144,9 @@ constexpr int kWfMaxSpp = 1 << (31 - kWfFlagBits);
 struct alignas(16) WfRay { float o[3]; float d[3]; int32_t scene; int32_t pad; };
 struct alignas(16) WfHit { int32_t leaf; float u, v, invDet; };
 struct alignas(16) WfNee { float nb[3]; float lpdf; float p1[3]; float p2[3]; int32_t used; int32_t pad; };
-struct alignas(16) WfShadow { float o[3]; float d[3]; int32_t path; int32_t scene; float c[3]; float pad2; };
-struct alignas(16) WfMis { float o[3]; float d[3]; int32_t path; int32_t light; float f[3]; float weight; float pdf; int32_t scene; int32_t pad[2]; };
+// A light sample's shadow ray or MIS-BSDF ray, at its path's index: the ray, the contribution c it
+// carries when nothing blocks it before tMax (MIS rays: nothing that beats leaf tieLeaf at tMax).
+struct alignas(16) WfLightRay { float o[3]; float d[3]; int32_t scene; int32_t tieLeaf; float c[3]; float tMax; };
 
 // Read by the kernels from device memory, so a captured pass graph can be replayed for every pass.
 struct WfParams {
@@ -209,8 +207,8 @@ struct WfBuffers {
     int32_t* shadowQ = nullptr;   // paths with a shadow ray (their records sit at the path index)
     int32_t* misQ = nullptr;      // paths with an MIS-BSDF ray (likewise)
     int32_t* bins = nullptr;      // material bin of each path's hit, written by the extend kernel
-    WfShadow* shadows = nullptr;  // per path
-    WfMis* mis = nullptr;         // per path
+    WfLightRay* shadows = nullptr;  // per path
+    WfLightRay* mis = nullptr;      // per path
     int32_t* counts = nullptr;
     // cached integrator (allocated by wf_reserve_cache)
     size_t cacheCap = 0;          // paths per pass covered by the query arrays

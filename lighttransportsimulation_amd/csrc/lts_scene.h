@@ -30,22 +30,23 @@ struct alignas(16) BvhNode {
     int32_t pad0, pad1;
 };
 
-// Node of the 4-wide render BVH: an interior node of even depth of the binary render tree, holding
-// the boxes of its children's children (a leaf child is kept as is). Child boxes are quantized to
-// 8 bits per plane against the node's own box: coordinate = origin + q * 2^e per axis, with qlo
-// rounded down and qhi rounded up so that the decoded box (computed exactly as the traversal does)
-// contains the child's box. child >= 0 is a 4-wide node, child < 0 the leaf ~child; `count`
-// children are valid. 64 bytes, four 16-byte loads.
-struct alignas(64) BvhQNode {
-    float ox, oy, oz;     // origin: minimum corner of the node's box
-    int8_t ex, ey, ez;    // per-axis scale exponents
-    uint8_t count;
-    int32_t child[4];
-    uint8_t qlo[3][4];    // [axis][child]
-    uint8_t qhi[3][4];
-    int32_t pad[2];
+// Record of the render tree, a 4-wide node or a triangle, so that one step of a traversal is three
+// 16-byte loads whatever it finds (the traversal's bound is the rate at which vector loads return).
+// The root is record 0 (the triangle of a one-triangle scene), levels follow breadth first, and the
+// children of a node are consecutive records. Node: the planes of its children's boxes are 8-bit
+// against its own box, coordinate = origin + q * 2^e per axis, and enclose the child's box.
+//   words 0-2   origin: minimum corner of the node's box (float)
+//   word 3      bytes 0-2: exponents e of x, y, z; bits 24-26: child count (2 to 4); bit 31 - k: child k
+//               is a triangle
+//   words 4-6   lower planes of x, y, z (byte k: child k), words 7-9 upper planes
+//   word 10     first child, in units of 16 bytes (3 per record)
+//   word 11     -1
+// Triangle: words 0-8 vertices, word 9 primitive number, word 10 material, word 11 leaf (>= 0).
+struct alignas(16) TraceRec {
+    uint32_t w[12];
 };
-static_assert(sizeof(BvhQNode) == 64, "BvhQNode layout");
+static_assert(sizeof(TraceRec) == 48, "TraceRec layout");
+constexpr int kRecUnits = 3;  // 16-byte units of a record
 
 struct alignas(16) ShadeTri {
     float n[9];    // vertex normals (valid when hasN)
@@ -111,7 +112,7 @@ struct CameraDesc {
 struct SceneView {
     const TriLeaf* tris;
     const BvhNode* nodes;
-    const BvhQNode* nodes4;  // 4-wide collapse of `nodes`, root at 0 (used by the traversal)
+    const TraceRec* recs;    // 4-wide collapse of `nodes` with its triangles, root at 0 (used by the traversal)
     const ShadeTri* shade;   // per BVH leaf: shade[k] belongs to the triangle tris[k]
     const MatDesc* mats;
     const TexDesc* texs;
@@ -125,14 +126,16 @@ struct SceneView {
     int32_t nLights;
     int32_t nPrim;
     int32_t infiniteLight;
+    int32_t root;  // the traversal's first stack entry: record 0, marked as a triangle in a one-triangle scene
     CameraDesc cam;
     float filter[256];
 };
 
-// Traversal stack entries per lane of the 4-wide traversal. A 4-wide node leaves at most 3 entries
-// on the stack, and a leaf at depth D of the binary tree lies under ceil(D / 2) 4-wide nodes, so a
-// render tree is accepted only when it is at most kMaxRenderDepth deep.
+// Traversal stack entries per lane of the 4-wide traversal: an end marker, and at most 3 for each
+// level of 4-wide nodes. A leaf at depth D of the binary tree lies under ceil(D / 2) even-collapsed
+// nodes, so a render tree is accepted only when it is at most kMaxRenderDepth deep.
 constexpr int kTraceStack = 128;
-constexpr int kMaxRenderDepth = 2 * (kTraceStack / 3);
+constexpr int kMaxNodeLevels = (kTraceStack - 1) / 3;
+constexpr int kMaxRenderDepth = 2 * kMaxNodeLevels;
 
 }  // namespace lts

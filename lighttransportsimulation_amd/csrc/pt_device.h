@@ -35,6 +35,7 @@ typedef float GlobalF4 __attribute__((ext_vector_type(4)));
 typedef unsigned GlobalU4 __attribute__((ext_vector_type(4)));
 LTS_D GlobalF4 load_global_f4(const void* p, int i) { return ((const __attribute__((address_space(1))) GlobalF4*)p)[i]; }
 LTS_D GlobalU4 load_global_u4(const void* p, int i) { return ((const __attribute__((address_space(1))) GlobalU4*)p)[i]; }
+LTS_D float word_f(unsigned w) { return __uint_as_float(w); }
 
 LTS_D void load_tri(const TriLeaf* __restrict__ tris, int k, V3& p0, V3& p1, V3& p2, int& prim) {
     const GlobalF4 a = load_global_f4(tris + k, 0), b = load_global_f4(tris + k, 1), c = load_global_f4(tris + k, 2);
@@ -53,8 +54,10 @@ constexpr float kOneMinusEpsF = 0x1.fff2e4p-1f;  // largest float <= 1.0 - (doub
 constexpr float kOnePlusEpsF = 0x1.00068cp+0f;   // largest float <= 1.0 + (double)SHADOW_EPS
 
 // Triangle::intersect hit test (shapes/Triangle.cu:94-128) without its distance test: true when
-// the ray meets the triangle inside the barycentric margins, at distance t of either sign.
-LTS_D bool tri_mt(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float& v, float& invDetOut) {
+// the ray meets the triangle inside the barycentric margins [SHADOW_EPS, limit], at distance t of either
+// sign. Triangle::simpleIntersect (shapes/Triangle.cu:50-84) is the same test with p1 and p2 exchanged
+// and limit 1 + SHADOW_EPS.
+LTS_D bool tri_mt(V3 p0, V3 p1, V3 p2, const Ray& r, float limit, float& t, float& u, float& v, float& invDetOut) {
     V3 edge1 = p1 - p0, edge2 = p2 - p0;
     V3 pVec = cross(r.d, edge2);
     float det = dot(edge1, pVec);
@@ -62,10 +65,10 @@ LTS_D bool tri_mt(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float& 
     float invDet = 1.0f / det;
     V3 tVec = r.o - p0;
     u = invDet * dot(tVec, pVec);
-    if (u < SHADOW_EPS || u > kOneMinusEpsF) return false;
+    if (u < SHADOW_EPS || u > limit) return false;
     V3 qVec = cross(tVec, edge1);
     v = invDet * dot(r.d, qVec);
-    if (v < SHADOW_EPS || u + v > kOneMinusEpsF) return false;
+    if (v < SHADOW_EPS || u + v > limit) return false;
     t = invDet * dot(edge2, qVec);
     invDetOut = invDet;
     return true;
@@ -73,7 +76,7 @@ LTS_D bool tri_mt(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float& 
 
 // Triangle::intersect hit test (shapes/Triangle.cu:94-128): t in (0, tMax).
 LTS_D bool tri_hit(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float& v, float& invDetOut) {
-    return tri_mt(p0, p1, p2, r, t, u, v, invDetOut) && t > 0 && t < r.tMax;
+    return tri_mt(p0, p1, p2, r, kOneMinusEpsF, t, u, v, invDetOut) && t > 0 && t < r.tMax;
 }
 
 // The closest-hit acceptance of leaf `leaf` against the current closest hit (distance r.tMax, leaf
@@ -83,24 +86,13 @@ LTS_D bool tri_hit(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float&
 // this rule gives the same winner in any visiting order.
 LTS_D bool tri_hit_closest(V3 p0, V3 p1, V3 p2, const Ray& r, int leaf, int best, float& t, float& u, float& v,
                            float& invDetOut) {
-    return tri_mt(p0, p1, p2, r, t, u, v, invDetOut) && t > 0 && (t < r.tMax || (t == r.tMax && leaf < best));
+    return tri_mt(p0, p1, p2, r, kOneMinusEpsF, t, u, v, invDetOut) && t > 0 && (t < r.tMax || (t == r.tMax && leaf < best));
 }
 
 // Triangle::simpleIntersect (shapes/Triangle.cu:50-84)
 LTS_D bool tri_occludes(V3 p0, V3 p1, V3 p2, const Ray& r) {
-    V3 edge1 = p1 - p0, edge2 = p2 - p0;
-    V3 pVec = cross(r.d, edge1);
-    float det = dot(edge2, pVec);
-    if (det == 0) return false;
-    float invDet = 1.0f / det;
-    V3 tVec = r.o - p0;
-    float u = invDet * dot(tVec, pVec);
-    if (u < SHADOW_EPS || u > kOnePlusEpsF) return false;
-    V3 qVec = cross(tVec, edge2);
-    float v = invDet * dot(r.d, qVec);
-    if (v < SHADOW_EPS || u + v > kOnePlusEpsF) return false;
-    float t = invDet * dot(edge1, qVec);
-    return t > 0 && t < r.tMax;
+    float t, u, v, invDet;
+    return tri_mt(p0, p2, p1, r, kOnePlusEpsF, t, u, v, invDet) && t > 0 && t < r.tMax;
 }
 
 // Bounds3::simpleIntersect (geometry/Bound.cuh:200-227); also returns the entry distance.
@@ -125,11 +117,24 @@ LTS_D bool box_hit(const float* mn, const float* mx, const Ray& r, V3 inv, int n
     return (tMin < r.tMax) && (tMax > 0);
 }
 
+// The reference's leaf-box test for a shadow ray (its inverse direction, BVH.cuh:336, and the
+// triangle's bounds).
+LTS_D bool leaf_box_passes(V3 p0, V3 p1, V3 p2, const Ray& r) {
+    const V3 inv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
+    const float mn[3] = {fminf(fminf(p0.x, p1.x), p2.x), fminf(fminf(p0.y, p1.y), p2.y), fminf(fminf(p0.z, p1.z), p2.z)};
+    const float mx[3] = {fmaxf(fmaxf(p0.x, p1.x), p2.x), fmaxf(fmaxf(p0.y, p1.y), p2.y), fmaxf(fmaxf(p0.z, p1.z), p2.z)};
+    float tEnter;
+    return box_hit(mn, mx, r, inv, inv.x < 0, inv.y < 0, inv.z < 0, tEnter);
+}
+
 constexpr int kStack = kTraceStack;
-// Stack entries kept in LDS; deeper entries go to private memory. 22 entries of a 256-lane block
-// (22528 B) plus the 256 B material histogram let 7 trace blocks (7 waves per SIMD) share a CU's
-// 160 KB of LDS.
+// Stack entries kept in LDS (the first is the end marker); deeper entries go to private memory. 22
+// entries of a 256-lane block (22528 B) plus the 256 B material histogram let 7 trace blocks (7
+// waves per SIMD) share a CU's 160 KB of LDS.
 constexpr int kShortStack = 22;
+// A stack entry is a record's offset in 16-byte units, with the sign bit set for a triangle.
+constexpr int kTraceLeaf = INT32_MIN;
+constexpr int kTraceDone = -1;  // bottom of the stack: the traversal has ended
 
 // Traversal stack of one lane: entries [0, kShortStack) in LDS (entry e at lds[e * stride], so the
 // lanes of a wave touch consecutive words), deeper entries in a private array that only deep
@@ -143,226 +148,214 @@ struct TraceStack {
 // LDS stack of thread `tid` in a block-wide array __shared__ int[kShortStack * blockSize].
 LTS_D TraceStack lds_stack(int* shared, int tid, int blockSize) { return TraceStack{shared + tid, blockSize}; }
 
-// Child boxes of a 4-wide node: hit distance per slot (INFINITY for a miss or an empty slot). The
-// quantized boxes are decoded with qdecode, as the builder did, and contain the exact child boxes;
-// the slab test is monotone in the planes, so a ray that passes an exact box passes its decoded box.
-// The ray's direction signs pick the near and far plane bytes once per axis for all four children,
-// so only those planes are decoded. The slab test is box_hit's in closed form: its pairwise
-// comparisons pass exactly when the largest near distance is at most the smallest far distance
-// (rounding is monotone, so scaling the minimum equals the minimum of the scaled values), then the
-// entry lies before tMax and the exit after 0. A NaN slab distance (a zero direction component with
-// the origin exactly on a plane) is ignored here on every axis, where box_hit culls on x only.
-// The inverse direction comes from the hardware reciprocal (at most 1 ulp, ray_inverse), so a slab
-// distance (p - o) * inv carries at most about 4 roundings instead of box_hit's 3, and the far
-// distances are scaled by 1 + 2 gamma(4) = (1 + 4u) / (1 - 4u) instead of 1 + 2 gamma(3): every box
-// the exact arithmetic passes still passes, so the test stays conservative.
-LTS_D void node4_hits(const BvhQNode* nodes4, int cur, const Ray& r, V3 inv, int nx, int ny, int nz, float (&t)[4],
-                      int (&c)[4], int& count) {
-    const GlobalU4 h = load_global_u4(nodes4 + cur, 0), ch = load_global_u4(nodes4 + cur, 1), lo = load_global_u4(nodes4 + cur, 2),
-                   hi = load_global_u4(nodes4 + cur, 3);
-    const float ox = __uint_as_float(h.x), oy = __uint_as_float(h.y), oz = __uint_as_float(h.z);
-    const int ex = (int)(int8_t)(h.w & 0xffu), ey = (int)(int8_t)((h.w >> 8) & 0xffu), ez = (int)(int8_t)((h.w >> 16) & 0xffu);
-    count = (int)(h.w >> 24);
-    // lo = (qlo x, qlo y, qlo z, qhi x), hi = (qhi y, qhi z, pad, pad); byte k belongs to child k
-    const unsigned nearX = nx ? lo.w : lo.x, farX = nx ? lo.x : lo.w;
-    const unsigned nearY = ny ? hi.x : lo.y, farY = ny ? lo.y : hi.x;
-    const unsigned nearZ = nz ? hi.y : lo.z, farZ = nz ? lo.z : hi.y;
-    const float g4 = 1 + 2 * gammaN(4);
-    const int cc[4] = {(int)ch.x, (int)ch.y, (int)ch.z, (int)ch.w};
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const unsigned s = 8 * k;
-        const float txMin = (qdecode(ox, ex, (nearX >> s) & 0xffu) - r.o.x) * inv.x;
-        const float txMax = (qdecode(ox, ex, (farX >> s) & 0xffu) - r.o.x) * inv.x;
-        const float tyMin = (qdecode(oy, ey, (nearY >> s) & 0xffu) - r.o.y) * inv.y;
-        const float tyMax = (qdecode(oy, ey, (farY >> s) & 0xffu) - r.o.y) * inv.y;
-        const float tzMin = (qdecode(oz, ez, (nearZ >> s) & 0xffu) - r.o.z) * inv.z;
-        const float tzMax = (qdecode(oz, ez, (farZ >> s) & 0xffu) - r.o.z) * inv.z;
-        const float tMin = fmaxf(fmaxf(txMin, tyMin), tzMin);
-        const float tMax = fminf(fminf(txMax, tyMax), tzMax) * g4;
-        const bool hit = k < count && tMin <= tMax && tMin <= r.tMax && tMax > 0;
-        t[k] = hit ? tMin : INFINITY;
-        c[k] = cc[k];
-    }
-}
-
-// 1 / d per component by v_rcp_f32 (within 1 ulp; 1 / ±0 = ±inf), for the 4-wide node test only.
-LTS_D V3 ray_inverse(V3 d) { return v3(__builtin_amdgcn_rcpf(d.x), __builtin_amdgcn_rcpf(d.y), __builtin_amdgcn_rcpf(d.z)); }
-
-LTS_D void cswap(float& ta, int& ca, float& tb, int& cb) {
-    if (tb < ta) {
-        const float t = ta; ta = tb; tb = t;
-        const int c = ca; ca = cb; cb = c;
-    }
-}
-
-// Closest hit (BVH::intersect, acceleration/BVH.cuh:365-398) over the 4-wide collapse of the render
-// tree (PLOC or the LBVH itself, over the same sorted leaves), children visited nearest first. A
-// 4-wide node tests the boxes of the binary tree's grandchildren and skips the children's boxes,
-// which never prunes a candidate a binary traversal would keep (a ray that passes a box passes its
-// ancestors' boxes). Every triangle whose box the ray passes before the current closest distance
-// is tested, so the reported hit is the reference traversal's, except for exactly equal distances.
 // Render-node fetches and triangle tests of one lane's traversals (counting launches only; the
 // timed kernels are instantiated without it).
 struct TraceTally {
     unsigned long long nodes = 0, tris = 0;
 };
 
-LTS_D Hit trace_closest(const SceneView& sv, Ray& r, TraceStack ts, unsigned long long* nodeCount, unsigned long long* triCount,
-                        TraceTally* tally = nullptr) {
-    Hit h; h.leaf = -1; h.t = h.u = h.v = h.invDet = 0;
-    const int n = sv.nPrim;
-    const V3 inv = ray_inverse(r.d);
-    int nx = inv.x < 0, ny = inv.y < 0, nz = inv.z < 0;
-    unsigned long long nodes = 0, tests = 0;
-    if (n == 1) {
-        V3 p0, p1, p2; int prim;
-        load_tri(sv.tris, 0, p0, p1, p2, prim);
-        float t, u, v, id;
-        tests++;
-        if (tri_hit_closest(p0, p1, p2, r, 0, h.leaf, t, u, v, id)) { r.tMax = t; h.leaf = 0; h.t = t; h.u = u; h.v = v; h.invDet = id; }
-    } else {
-        int spill[kStack - kShortStack];
-        int sp = 0;
-        int cur = 0;  // the 4-wide root; entries < 0 are leaves (~leaf)
-        // every node and leaf is entered at most once; the step bound and the index checks keep a
-        // malformed node array from running away
-        for (unsigned steps = 0; steps < 2u * (unsigned)n + 64u; steps++) {
-            if (cur >= 0) {
-                if (cur >= n - 1) break;
-                float t[4];
-                int c[4], count;
-                node4_hits(sv.nodes4, cur, r, inv, nx, ny, nz, t, c, count);
-                nodes++;
-                cswap(t[0], c[0], t[1], c[1]);
-                cswap(t[2], c[2], t[3], c[3]);
-                cswap(t[0], c[0], t[2], c[2]);
-                cswap(t[1], c[1], t[3], c[3]);
-                cswap(t[1], c[1], t[2], c[2]);
+// 1 / d by v_rcp_f32 (within 1 ulp) with its magnitude held to 2^100, for the node test only: a
+// zero direction component gives slab distances that are hugely negative or positive, never NaN.
+LTS_D float slab_inverse(float d) { return __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(d), -0x1p100f, 0x1p100f); }
+
+// The traversal of one lane. A ray's slab constants, then the stack (entry e in LDS below kShortStack,
+// else in `spill`) and the record to visit next.
+struct TraceLane {
+    V3 o, inv;
+    bool nx, ny, nz;
+    int cur, sp;
+};
+
+// Whether a ray has an infinite or NaN component: it then passes no triangle test.
+LTS_D bool ray_degenerate(V3 o, V3 d) { return !(0 * o.x + 0 * o.y + 0 * o.z + 0 * d.x + 0 * d.y + 0 * d.z == 0); }
+
+LTS_D void trace_begin(TraceLane& l, V3 o, V3 d, int root, TraceStack ts) {
+    l.o = o;
+    l.inv = v3(slab_inverse(d.x), slab_inverse(d.y), slab_inverse(d.z));
+    l.nx = l.inv.x < 0; l.ny = l.inv.y < 0; l.nz = l.inv.z < 0;
+    ts.lds[0] = kTraceDone;
+    l.sp = 1;
+    l.cur = ray_degenerate(o, d) ? kTraceDone : root;
+}
+
+LTS_D void trace_pop(TraceLane& l, TraceStack ts, const int* spill) {
+    --l.sp;
+    if (__builtin_expect(__any(l.sp >= kShortStack), 0)) l.cur = l.sp < kShortStack ? ts.lds[l.sp * ts.stride] : spill[l.sp - kShortStack];
+    else l.cur = ts.lds[l.sp * ts.stride];
+}
+
+// One node of the 4-wide render tree (BVH::intersect / BVH::simpleIntersect, acceleration/BVH.cuh:331-398):
+// tests the boxes of its children, goes on to the nearest one hit and stacks the others. Every triangle
+// whose box the ray passes before its current tMax is reached, so the closest hit is the reference
+// traversal's in any order of visits (tri_hit_closest settles equal distances).
+//
+// A child's planes are origin + q * 2^e with 8-bit q, and the builder encloses the child's box between
+// the exact planes (quantize_node). Their slab distances come as one fused multiply-add each,
+// t = q * (2^e inv) + (origin - o) inv: 2^e inv is exact, so a distance is off by the rounding of
+// origin - o and of its product, at most 2.01 u |B| with B = (origin - o) inv, by the final rounding
+// (1 u) and by the reciprocal's 2 u, a factor common to the axis. Near distances take B - 4u|B| and far
+// ones B + 4u|B|, the far minimum is scaled by 1 + 2 gamma(4) > 1 + 6u, and tBox exceeds tMax by 2^-20
+// of it: the test passes every box that exact arithmetic passes, boxes entered exactly at tMax included
+// (a tie there may go to a lower leaf). A zero direction component (inv = +-2^100) passes exactly the
+// slabs that hold the origin, but for a flat one at the node's minimum with the ray in its plane, whose
+// triangles the ray is parallel to (det = 0).
+constexpr float kTieScale = 1 + 0x1p-20f;
+
+LTS_D void trace_node(TraceLane& l, const TraceRec* recs, float tMax, TraceStack ts, int* spill) {
+    const void* rec = reinterpret_cast<const char*>(recs) + ((size_t)(unsigned)l.cur << 4);
+    const GlobalU4 hd = load_global_u4(rec, 0), lo = load_global_u4(rec, 1), hi = load_global_u4(rec, 2);
+    const float ax = __builtin_amdgcn_ldexpf(l.inv.x, (int)(int8_t)(hd.w & 0xffu));
+    const float ay = __builtin_amdgcn_ldexpf(l.inv.y, (int)(int8_t)((hd.w >> 8) & 0xffu));
+    const float az = __builtin_amdgcn_ldexpf(l.inv.z, (int)(int8_t)((hd.w >> 16) & 0xffu));
+    const int count = (int)((hd.w >> 24) & 7u);
+    const float bx = (word_f(hd.x) - l.o.x) * l.inv.x, by = (word_f(hd.y) - l.o.y) * l.inv.y, bz = (word_f(hd.z) - l.o.z) * l.inv.z;
+    constexpr float k4u = 0x1p-22f;
+    const float bxn = __builtin_fmaf(fabsf(bx), -k4u, bx), bxf = __builtin_fmaf(fabsf(bx), k4u, bx);
+    const float byn = __builtin_fmaf(fabsf(by), -k4u, by), byf = __builtin_fmaf(fabsf(by), k4u, by);
+    const float bzn = __builtin_fmaf(fabsf(bz), -k4u, bz), bzf = __builtin_fmaf(fabsf(bz), k4u, bz);
+    // lo = (qlo x, qlo y, qlo z, qhi x), hi = (qhi y, qhi z, first child, -1); byte k belongs to child k
+    const unsigned nearX = l.nx ? lo.w : lo.x, farX = l.nx ? lo.x : lo.w;
+    const unsigned nearY = l.ny ? hi.x : lo.y, farY = l.ny ? lo.y : hi.x;
+    const unsigned nearZ = l.nz ? hi.y : lo.z, farZ = l.nz ? lo.z : hi.y;
+    const float g4 = 1 + 2 * gammaN(4), tBox = tMax * kTieScale;
+    float t[4];
 #pragma unroll
-                for (int k = 3; k >= 1; k--) {
-                    if (t[k] < INFINITY && sp < kStack) {
-                        if (sp < kShortStack) ts.lds[sp * ts.stride] = c[k];
-                        else spill[sp - kShortStack] = c[k];
-                        sp++;
-                    }
-                }
-                if (t[0] < INFINITY) { cur = c[0]; continue; }
+    for (int k = 0; k < 4; k++) {
+        const unsigned s = 8 * k;
+        const float tn = fmaxf(fmaxf(__builtin_fmaf((float)((nearX >> s) & 0xffu), ax, bxn),
+                                     __builtin_fmaf((float)((nearY >> s) & 0xffu), ay, byn)),
+                               __builtin_fmaf((float)((nearZ >> s) & 0xffu), az, bzn));
+        const float tf = fminf(fminf(__builtin_fmaf((float)((farX >> s) & 0xffu), ax, bxf),
+                                     __builtin_fmaf((float)((farY >> s) & 0xffu), ay, byf)),
+                               __builtin_fmaf((float)((farZ >> s) & 0xffu), az, bzf));
+        const float enter = fmaxf(tn, 0.0f), leave = fminf(tf * g4, tBox);
+        t[k] = enter <= leave && (k < 2 || k < count) ? enter : INFINITY;  // a node has two children at least
+    }
+    // the nearest child next, the other three stacked with the nearer pair's loser on top
+    const unsigned first = hi.z, leafBit = 0x80000000u;
+    const int c0 = (int)(first | (hd.w & leafBit)), c1 = (int)((first + kRecUnits) | ((hd.w << 1) & leafBit)),
+              c2 = (int)((first + 2 * kRecUnits) | ((hd.w << 2) & leafBit)),
+              c3 = (int)((first + 3 * kRecUnits) | ((hd.w << 3) & leafBit));
+    const bool sa = t[1] < t[0], sb = t[3] < t[2];
+    const float ta = fminf(t[0], t[1]), tb = fminf(t[2], t[3]), ua = fmaxf(t[0], t[1]), ub = fmaxf(t[2], t[3]);
+    const int ca = sa ? c1 : c0, da = sa ? c0 : c1, cb = sb ? c3 : c2, db = sb ? c2 : c3;
+    const bool sw = tb < ta;
+    const float tw = fminf(ta, tb), tl = fmaxf(ta, tb);
+    const int cw = sw ? cb : ca, cl = sw ? ca : cb;
+    if (__builtin_expect(__any(l.sp > kShortStack - 3), 0)) {
+        const float pt[3] = {ua, ub, tl};
+        const int pc[3] = {da, db, cl};
+        for (int k = 0; k < 3; k++) {
+            if (pt[k] < INFINITY) {
+                if (l.sp < kShortStack) ts.lds[l.sp * ts.stride] = pc[k];
+                else spill[l.sp - kShortStack] = pc[k];
+                l.sp++;
+            }
+        }
+    } else {
+        // written whether or not the box was hit: an entry above the top is never read
+        ts.lds[l.sp * ts.stride] = da;
+        l.sp += ua < INFINITY;
+        ts.lds[l.sp * ts.stride] = db;
+        l.sp += ub < INFINITY;
+        ts.lds[l.sp * ts.stride] = cl;
+        l.sp += tl < INFINITY;
+    }
+    if (tw < INFINITY) l.cur = cw;
+    else trace_pop(l, ts, spill);
+}
+
+// The triangle record at the lane's current entry.
+struct TraceTri {
+    V3 p0, p1, p2;
+    int mat, leaf;
+};
+LTS_D TraceTri trace_triangle(const TraceLane& l, const TraceRec* recs) {
+    const void* rec = reinterpret_cast<const char*>(recs) + ((size_t)((unsigned)l.cur & 0x7fffffffu) << 4);
+    const GlobalU4 a = load_global_u4(rec, 0), b = load_global_u4(rec, 1), c = load_global_u4(rec, 2);
+    TraceTri t;
+    t.p0 = v3(word_f(a.x), word_f(a.y), word_f(a.z));
+    t.p1 = v3(word_f(a.w), word_f(b.x), word_f(b.y));
+    t.p2 = v3(word_f(b.z), word_f(b.w), word_f(c.x));
+    t.mat = (int)c.z;
+    t.leaf = (int)c.w;
+    return t;
+}
+
+// What a traversal does at a triangle.
+enum TraceKind {
+    kTraceClosest,  // Triangle::intersect: keep the closest hit
+    kTraceShadow,   // Triangle::simpleIntersect within the leaf's box: any triangle ends the traversal
+    kTraceBeats     // Triangle::intersect: any triangle that would win the closest hit against `best` at r.tMax
+};
+
+// A whole traversal by every lane of the wave that calls it. The wave runs either the node step or the
+// triangle step: lanes that hold a triangle wait until kLeafGate of them do or no lane holds a node, so
+// the triangle test (fp64 cross products) runs for several lanes at once. The records were checked when
+// the scene was loaded (k_check_recs): children lie in range and after their node, so each traversal
+// ends, and no accepted tree needs more than kStack entries.
+constexpr int kLeafGate = 8;
+
+template <int kKind>
+LTS_D Hit traverse(const TraceRec* recs, int root, Ray& r, TraceStack ts, int best, TraceTally* tally) {
+    Hit h;
+    h.leaf = -1; h.t = h.u = h.v = h.invDet = 0;
+    int spill[kStack - kShortStack];
+    TraceLane l;
+    trace_begin(l, r.o, r.d, root, ts);
+    while (l.cur != kTraceDone) {
+        const bool leafStep = l.cur < 0;
+        const unsigned long long waiting = __ballot(leafStep), walking = __ballot(!leafStep);
+        if (walking != 0 && __popcll(waiting) < kLeafGate) {
+            if (!leafStep) {
+                if (tally) tally->nodes++;
+                trace_node(l, recs, r.tMax, ts, spill);
+            }
+        } else if (leafStep) {
+            const TraceTri tr = trace_triangle(l, recs);
+            if (tally) tally->tris++;
+            float t, u, v, id;
+            if constexpr (kKind == kTraceShadow) {
+                if (tri_occludes(tr.p0, tr.p1, tr.p2, r) && leaf_box_passes(tr.p0, tr.p1, tr.p2, r)) { h.leaf = tr.leaf; break; }
+            } else if constexpr (kKind == kTraceBeats) {
+                if (tri_hit_closest(tr.p0, tr.p1, tr.p2, r, tr.leaf, best, t, u, v, id)) { h.leaf = tr.leaf; break; }
             } else {
-                const int k = ~cur;
-                if (k >= n) break;
-                V3 p0, p1, p2; int prim;
-                load_tri(sv.tris, k, p0, p1, p2, prim);
-                float t, u, v, id;
-                tests++;
-                if (tri_hit_closest(p0, p1, p2, r, k, h.leaf, t, u, v, id)) {
-                    r.tMax = t; h.leaf = k; h.t = t; h.u = u; h.v = v; h.invDet = id;
+                if (tri_hit_closest(tr.p0, tr.p1, tr.p2, r, tr.leaf, h.leaf, t, u, v, id)) {
+                    r.tMax = t;
+                    h.leaf = tr.leaf; h.t = t; h.u = u; h.v = v; h.invDet = id;
                 }
             }
-            if (sp == 0) break;
-            --sp;
-            cur = sp < kShortStack ? ts.lds[sp * ts.stride] : spill[sp - kShortStack];
+            trace_pop(l, ts, spill);
         }
     }
-    if (nodeCount) { atomicAdd(nodeCount, nodes); atomicAdd(triCount, tests); }
-    if (tally) { tally->nodes += nodes; tally->tris += tests; }
     return h;
 }
 
-// The reference's leaf-box test for a shadow ray (its inverse direction, BVH.cuh:336, and the
-// triangle's bounds), out of line: it runs once per occluded shadow ray.
-static __device__ __attribute__((noinline)) bool leaf_box_passes(V3 p0, V3 p1, V3 p2, Ray r) {
-    const V3 inv = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
-    const float mn[3] = {fminf(fminf(p0.x, p1.x), p2.x), fminf(fminf(p0.y, p1.y), p2.y), fminf(fminf(p0.z, p1.z), p2.z)};
-    const float mx[3] = {fmaxf(fmaxf(p0.x, p1.x), p2.x), fmaxf(fmaxf(p0.y, p1.y), p2.y), fmaxf(fmaxf(p0.z, p1.z), p2.z)};
-    float tEnter;
-    return box_hit(mn, mx, r, inv, inv.x < 0, inv.y < 0, inv.z < 0, tEnter);
+// Closest hit (BVH::intersect, acceleration/BVH.cuh:365-398); r.tMax becomes its distance.
+LTS_D Hit trace_closest(const SceneView& sv, Ray& r, TraceStack ts, unsigned long long* nodeCount, unsigned long long* triCount,
+                        TraceTally* tally = nullptr) {
+    if (nodeCount) {
+        TraceTally own;
+        const Hit h = traverse<kTraceClosest>(sv.recs, sv.root, r, ts, -1, &own);
+        atomicAdd(nodeCount, own.nodes);
+        atomicAdd(triCount, own.tris);
+        return h;
+    }
+    return traverse<kTraceClosest>(sv.recs, sv.root, r, ts, -1, tally);
 }
 
-// The triangle test of an any-hit traversal: Triangle::simpleIntersect for shadow rays (with
-// kLeafBox, only when the leaf-box test passes too), or the closest-hit test (Triangle::intersect)
-// when the question is whether leaf `leaf` would win the closest hit against leaf `tieLeaf` at
-// distance r.tMax (nearer, or as near with a lower index).
-template <bool kHitTest, bool kLeafBox>
-LTS_D bool leaf_blocks(V3 p0, V3 p1, V3 p2, const Ray& r, int leaf, int tieLeaf) {
-    if constexpr (kHitTest) {
-        float t, u, v, id;
-        return tri_hit_closest(p0, p1, p2, r, leaf, tieLeaf, t, u, v, id);
-    } else if constexpr (kLeafBox) {
-        return tri_occludes(p0, p1, p2, r) && leaf_box_passes(p0, p1, p2, r);
-    } else {
-        return tri_occludes(p0, p1, p2, r);
-    }
-}
-
-// Any hit (BVH::simpleIntersect, acceleration/BVH.cuh:331-363) over the 4-wide tree: leaf children
-// are tested as soon as their box is hit, interior children are stacked. Returns the first leaf
-// whose test passes, or -1.
-template <bool kHitTest, bool kLeafBox>
-LTS_D int any_hit_leaf(int n, const BvhQNode* nodes4, const TriLeaf* tris, const Ray& r, TraceStack ts, TraceTally* tally,
-                       int tieLeaf) {
-    const V3 inv = ray_inverse(r.d);
-    int nx = inv.x < 0, ny = inv.y < 0, nz = inv.z < 0;
-    if (n == 1) {
-        V3 p0, p1, p2; int prim;
-        load_tri(tris, 0, p0, p1, p2, prim);
-        if (tally) tally->tris++;
-        return leaf_blocks<kHitTest, kLeafBox>(p0, p1, p2, r, 0, tieLeaf) ? 0 : -1;
-    }
-    int spill[kStack - kShortStack];
-    int sp = 0;
-    int cur = 0;
-    for (unsigned steps = 0; steps < 2u * (unsigned)n + 64u; steps++) {
-        if (cur < 0 || cur >= n - 1) return -1;
-        float t[4];
-        int c[4], count;
-        node4_hits(nodes4, cur, r, inv, nx, ny, nz, t, c, count);
-        if (tally) tally->nodes++;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (t[k] < INFINITY) {
-                if (c[k] < 0) {
-                    const int leaf = ~c[k];
-                    if (leaf >= n) return -1;
-                    V3 p0, p1, p2; int prim;
-                    load_tri(tris, leaf, p0, p1, p2, prim);
-                    if (tally) tally->tris++;
-                    if (leaf_blocks<kHitTest, kLeafBox>(p0, p1, p2, r, leaf, tieLeaf)) return leaf;
-                } else if (sp < kStack) {
-                    if (sp < kShortStack) ts.lds[sp * ts.stride] = c[k];
-                    else spill[sp - kShortStack] = c[k];
-                    sp++;
-                }
-            }
-        }
-        if (sp == 0) return -1;
-        --sp;
-        cur = sp < kShortStack ? ts.lds[sp * ts.stride] : spill[sp - kShortStack];
-    }
-    return -1;
-}
-
-// kHitTest: the closest-hit question of an MIS ray, whether any leaf beats tieLeaf at r.tMax.
+// Any hit (BVH::simpleIntersect, acceleration/BVH.cuh:331-363), whether the ray is blocked before
+// r.tMax. kHitTest: the closest-hit question of an MIS ray, whether any leaf beats tieLeaf at r.tMax.
 // Otherwise a shadow ray. Triangle::simpleIntersect accepts points up to SHADOW_EPS outside the
 // triangle's edges, and the reference reaches a triangle only through its leaf's box test
 // (BVH.cuh:343-348: the leaf node's bounds, the primitive's own bounds). The render tree's quantized
 // boxes are wider than that leaf box, so a triangle the enlarged test accepts is also put to the
-// leaf-box test; when that fails (a ray passing just outside a triangle's edge and its bounds, rare),
-// the ray is traversed again with the leaf-box test on every triangle hit. The common path keeps the
-// plain loop. (The closest-hit test accepts only points inside the triangle shrunk by SHADOW_EPS,
+// leaf-box test. (The closest-hit test accepts only points inside the triangle shrunk by SHADOW_EPS,
 // which lie inside its bounds.)
 template <bool kHitTest = false>
-LTS_D bool trace_any(const SceneView& sv, const Ray& r, TraceStack ts, TraceTally* tally = nullptr, int tieLeaf = -1) {
-    if constexpr (kHitTest) {
-        return any_hit_leaf<true, false>(sv.nPrim, sv.nodes4, sv.tris, r, ts, tally, tieLeaf) >= 0;
-    } else {
-        const int leaf = any_hit_leaf<false, false>(sv.nPrim, sv.nodes4, sv.tris, r, ts, tally, -1);
-        if (leaf < 0) return false;
-        V3 p0, p1, p2; int prim;
-        load_tri(sv.tris, leaf, p0, p1, p2, prim);
-        if (leaf_box_passes(p0, p1, p2, r)) return true;
-        return any_hit_leaf<false, true>(sv.nPrim, sv.nodes4, sv.tris, r, ts, tally, -1) >= 0;
-    }
+LTS_D bool trace_any(const SceneView& sv, const Ray& ray, TraceStack ts, TraceTally* tally = nullptr, int tieLeaf = -1) {
+    Ray r = ray;
+    return traverse<kHitTest ? kTraceBeats : kTraceShadow>(sv.recs, sv.root, r, ts, tieLeaf, tally).leaf >= 0;
 }
 
 // Triangle::intersect interaction part + SurfaceInteraction constructor / setShaddingGeometry
@@ -923,25 +916,32 @@ LTS_D int sample_light(const SceneView& sv, float u, float* pdf) {
 // The light test of the MIS-BSDF ray (IntegratorHelper.cuh:103-122): whether the closest hit of r
 // (spawned with tMax = infinity) is light li's triangle, seen from its emitting side, or for the
 // infinite light whether r escapes. The closest-hit traversal is not needed for that. A ray that
-// misses the light's triangle, or meets its back, contributes nothing whatever lies in front. A ray
-// that meets its front at t reaches it unless some triangle would win the closest hit against it
-// (nearer, or at exactly t with a lower leaf index, tri_hit_closest), which an any-hit traversal
-// bounded at t answers; the same t, u, v and 1/det come out of the triangle test whatever tMax is.
-LTS_D bool mis_reaches_light(const SceneView& sv, const LightDesc& L, int li, Ray r, TraceStack ts,
-                             TraceTally* tally = nullptr) {
-    if (L.kind == 0) {
-        if (L.leaf < 0 || sv.shade[L.leaf].light != li) return false;
-        V3 p0, p1, p2; int prim;
-        load_tri(sv.tris, L.leaf, p0, p1, p2, prim);
-        if (tally) tally->tris++;
-        float t, u, v, id;
-        if (!tri_hit(p0, p1, p2, r, t, u, v, id)) return false;
-        const SurfacePoint lt = make_surface(sv, L.leaf, r, u, v, id);
-        if (!(dot(lt.n, -r.d) > 0.f)) return false;
-        r.tMax = t;
-        return !trace_any<true>(sv, r, ts, tally, L.leaf);
-    }
-    return !trace_any<true>(sv, r, ts, tally, -1);
+// misses the light's triangle, or meets its back, contributes nothing whatever lies in front
+// (mis_target is false). A ray that meets its front at t reaches it unless some triangle would win the
+// closest hit against it (nearer, or at exactly t with a lower leaf index, tri_hit_closest), which an
+// any-hit traversal bounded at t answers; the same t, u, v and 1/det come out of the triangle test
+// whatever tMax is. tMax and tieLeaf receive that traversal's bound.
+LTS_D bool mis_target(const SceneView& sv, const LightDesc& L, int li, const Ray& r, float& tMax, int& tieLeaf) {
+    tMax = INFINITY;
+    tieLeaf = -1;
+    if (L.kind != 0) return true;
+    if (L.leaf < 0 || sv.shade[L.leaf].light != li) return false;
+    V3 p0, p1, p2; int prim;
+    load_tri(sv.tris, L.leaf, p0, p1, p2, prim);
+    float t, u, v, id;
+    if (!tri_hit(p0, p1, p2, r, t, u, v, id)) return false;
+    const SurfacePoint lt = make_surface(sv, L.leaf, r, u, v, id);
+    if (!(dot(lt.n, -r.d) > 0.f)) return false;
+    tMax = t;
+    tieLeaf = L.leaf;
+    return true;
+}
+LTS_D bool mis_reaches_light(const SceneView& sv, const LightDesc& L, int li, Ray r, TraceStack ts) {
+    int tieLeaf;
+    float tMax;
+    if (!mis_target(sv, L, li, r, tMax, tieLeaf)) return false;
+    r.tMax = tMax;
+    return !trace_any<true>(sv, r, ts, nullptr, tieLeaf);
 }
 
 // estimateDirect (intergrators/IntegratorHelper.cuh:51-125)

@@ -71,9 +71,14 @@ LTS_D Spec radiance(const SceneView& sv, int px, int py, int sample, const Rende
     return L;
 }
 
-__global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tris, const ShadeTri* __restrict__ shade, int n) {
+__global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tris, const ShadeTri* __restrict__ shade, int n,
+                                                       TraceRec* __restrict__ recs, int nRecs) {
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k < n) tris[k].mat = shade[k].mat;
+    if (k < nRecs) {
+        const uint32_t leaf = recs[k].w[11];
+        if (leaf < (uint32_t)n) recs[k].w[10] = (uint32_t)shade[leaf].mat;
+    }
 }
 
 // Latency-bound: five waves per SIMD (the compiler spills the rest of the path state to scratch)
@@ -193,9 +198,10 @@ hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipSt
     return hipGetLastError();
 }
 
-hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, hipStream_t s) {
+hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t s) {
     if (n < 1) return hipSuccess;
-    k_tri_materials<<<(n + 255) / 256, 256, 0, s>>>(tris, shade, n);
+    const int m = nRecs > n ? nRecs : n;
+    k_tri_materials<<<(m + 255) / 256, 256, 0, s>>>(tris, shade, n, recs, nRecs);
     return hipGetLastError();
 }
 

@@ -2,12 +2,12 @@
 //
 // The reference integrator (intergrators/PathTracingIntegrator.cuh:38-104 with estimateDirect,
 // IntegratorHelper.cuh:51-125) is cut at its three ray casts:
-//   extend   closest hit of every live path ray                     (persistent, wave-batched)
+//   extend   closest hit of every live path ray                     (persistent)
 //   sort     optional counting sort of the hit queue by material
 //   shade    emission, BSDF, light sample + MIS-BSDF sample (NEE set-up), continuation, roulette;
 //            appends one shadow ray and one MIS ray per path at most
-//   shadow   any hit of the shadow rays                             (persistent, wave-batched)
-//   mis      closest hit of the MIS-BSDF rays, light identity test  (persistent, wave-batched)
+//   shadow   any hit of the shadow rays                             (persistent, in extend's launch)
+//   mis      whether an MIS-BSDF ray reaches its light              (persistent, in extend's launch)
 //   finalize L += beta * ((Ld_light + Ld_bsdf) / p_pick), the reference's order of additions;
 //            terminated paths write their radiance
 // Each path's arithmetic is the megakernel's, so the image does not depend on queue order.
@@ -93,46 +93,6 @@ __global__ __launch_bounds__(256) void k_wf_generate(const SceneView* __restrict
         r.scene = sc; r.pad = 0;
         rays[k] = r;
         queue[k] = (int)k;
-    }
-}
-
-// Wave-batched work fetch (lane 0 takes 64 items at a time) over kWfWorkSegments contiguous segments of segLen items (a multiple of
-// 64), one counter each. Workgroups are dealt to the 8 XCDs round robin, so the waves of XCD
-// blockIdx % 8 start on their own segment and keep neighbouring rays in one L2; a wave whose
-// segment has run dry moves on to the next ones. Returns the item of this lane, with `j` (uniform
-// over the wave) advanced past the segments found empty; j == kWfWorkSegments means no work is left.
-LTS_D int wave_fetch_segmented(int32_t* work, int segLen, int& j) {
-    const int lane = threadIdx.x & 63;
-    const int home = blockIdx.x % kWfWorkSegments;
-    while (j < kWfWorkSegments) {
-        const int seg = (home + j) % kWfWorkSegments;
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&work[kWfWorkStride * seg], 64);
-        base = __shfl(base, 0);
-        if (base < segLen) return seg * segLen + base + lane;
-        j++;
-    }
-    return 0;
-}
-
-// Closest hit of path ray `pi`; with `hist` set, the hit is also filed under its material bin
-// (misses in the last bin) for the counting sort: bins[path] and the block histogram lh.
-LTS_D void extend_item(const SceneView* scenes, const WfRay* rays, WfHit* hits, int pi,
-                       TraceStack ts, int32_t* bins, int32_t* lh, bool filing, int nBins, TraceTally* tally = nullptr) {
-    const WfRay rr = rays[pi];
-    Ray r;
-    r.o = v3(rr.o[0], rr.o[1], rr.o[2]);
-    r.d = v3(rr.d[0], rr.d[1], rr.d[2]);
-    r.tMax = INFINITY;
-    const SceneView& sv = scenes[rr.scene];
-    Hit h = trace_closest(sv, r, ts, nullptr, nullptr, tally);
-    WfHit o;
-    o.leaf = h.leaf; o.u = h.u; o.v = h.v; o.invDet = h.invDet;
-    hits[pi] = o;
-    if (filing) {
-        const int bin = h.leaf < 0 ? nBins - 1 : min(sv.tris[h.leaf].mat, nBins - 2);
-        bins[pi] = bin;
-        atomicAdd(&lh[bin], 1);
     }
 }
 
@@ -232,8 +192,8 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                                                           const WfHit* __restrict__ hits, WfNee* __restrict__ nee,
                                                           const int32_t* __restrict__ queue, const int32_t* __restrict__ count,
                                                           int32_t* __restrict__ nextQueue, int32_t* __restrict__ nextCount,
-                                                          WfShadow* __restrict__ shadows, int32_t* __restrict__ shadowCount,
-                                                          WfMis* __restrict__ misRays, int32_t* __restrict__ misCount,
+                                                          WfLightRay* __restrict__ shadows, int32_t* __restrict__ shadowCount,
+                                                          WfLightRay* __restrict__ misRays, int32_t* __restrict__ misCount,
                                                           float* __restrict__ qRaw, NrcQuery* __restrict__ qMeta,
                                                           int32_t* __restrict__ qCount,
                                                           WfTrainRec* __restrict__ tRec, float* __restrict__ tRaw,
@@ -262,8 +222,7 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
         const bool active = k < n;
         const int pi = active ? queue[k] : 0;
         bool wantShadow = false, wantMis = false, wantNext = false, wantQuery = false, wantDone = false;
-        WfShadow sh;
-        WfMis ms;
+        WfLightRay sh;
         if (active) {
             const WfParams P = *prm;
             WfPath p;
@@ -390,7 +349,7 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                             V3 d = target - origin;
                             sh.o[0] = origin.x; sh.o[1] = origin.y; sh.o[2] = origin.z;
                             sh.d[0] = d.x; sh.d[1] = d.y; sh.d[2] = d.z;
-                            sh.path = pi; sh.scene = scene;
+                            sh.scene = scene; sh.tieLeaf = -1; sh.tMax = 1 - SHADOW_EPS;
                             sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
                             wantShadow = true;
                             shadows[pi] = sh;  // per path; the queue below lists the paths
@@ -409,15 +368,18 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                             if (lightPdf == 0) cast = false;
                             else weight = power_heuristic(scatteringPdf, lightPdf);
                         }
-                        if (cast) {
-                            Ray mr = spawn_ray(si, wi);
-                            ms.o[0] = mr.o.x; ms.o[1] = mr.o.y; ms.o[2] = mr.o.z;
-                            ms.d[0] = wi.x; ms.d[1] = wi.y; ms.d[2] = wi.z;
-                            ms.path = pi; ms.light = li; ms.scene = scene;
-                            ms.f[0] = f2.r; ms.f[1] = f2.g; ms.f[2] = f2.b;
-                            ms.weight = weight; ms.pdf = scatteringPdf;
-                            wantMis = true;
-                            misRays[pi] = ms;
+                        const Spec Li2 = light_le(Lt);
+                        if (cast && !isBlack(Li2)) {
+                            const Ray mr = spawn_ray(si, wi);
+                            if (mis_target(sv, Lt, li, mr, sh.tMax, sh.tieLeaf)) {
+                                const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
+                                sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
+                                sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
+                                sh.scene = scene;
+                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
+                                wantMis = true;
+                                misRays[pi] = sh;
+                            }
                         }
                     }
                 }
@@ -586,54 +548,32 @@ __global__ __launch_bounds__(kCollectBlock) void k_wf_nrc_scatter(const WfParams
     }
 }
 
-// Any hit of the shadow ray of path k: the light sample's contribution when the segment is free.
-LTS_D void shadow_item(const SceneView* scenes, const WfShadow* shadows, WfNee* nee, int k,
-                       TraceStack ts, TraceTally* tally = nullptr) {
-    const WfShadow s = shadows[k];
-    Ray r;
-    r.o = v3(s.o[0], s.o[1], s.o[2]);
-    r.d = v3(s.d[0], s.d[1], s.d[2]);
-    r.tMax = 1 - SHADOW_EPS;
-    if (!trace_any(scenes[s.scene], r, ts, tally)) {
-        nee[s.path].p1[0] = s.c[0];
-        nee[s.path].p1[1] = s.c[1];
-        nee[s.path].p1[2] = s.c[2];
-    }
-}
-
-// The MIS-BSDF ray of path k: does it reach the light it was cast for (IntegratorHelper.cuh:103-122).
-LTS_D void mis_item(const SceneView* scenes, const WfMis* misRays, WfNee* nee, int k, TraceStack ts,
-                    TraceTally* tally = nullptr) {
-    const WfMis m = misRays[k];
-    const SceneView& sv = scenes[m.scene];
-    const LightDesc& Lt = sv.lights[m.light];
-    Ray r;
-    r.o = v3(m.o[0], m.o[1], m.o[2]);
-    r.d = v3(m.d[0], m.d[1], m.d[2]);
-    r.tMax = INFINITY;
-    const Spec Li2 = mis_reaches_light(sv, Lt, m.light, r, ts, tally) ? light_le(Lt) : spec(0.f);
-    if (!isBlack(Li2)) {
-        Spec c = spec(m.f[0], m.f[1], m.f[2]) * Li2 * spec(1.0f) * m.weight / m.pdf;
-        nee[m.path].p2[0] = c.r;
-        nee[m.path].p2[1] = c.g;
-        nee[m.path].p2[2] = c.b;
-    }
-}
-
 // One persistent launch traces every ray that is ready: the path rays of the next bounce (queue
 // `ext`), then the shadow rays and the MIS rays of the bounce just shaded. The three sets do not
 // depend on each other, so one work counter over their concatenation balances long rays against
 // short ones and leaves one tail per bounce instead of three. Counts may be null (empty set).
-// The launch asks for 7 waves per SIMD (at most 72 VGPRs): enough waves to cover the load latency
-// of the traversal, which then runs at the VALU issue limit; at 8 the 64-register cap spills.
+//
+// A wave's rays differ in length by a factor of ten, so a wave that traced 64 rays to their ends ran its
+// steps with 26 % of its lanes. Instead a lane whose ray has ended takes the next one as soon as half of
+// the wave's lanes are free (refilling at a quarter measured the same, at three quarters 8 % slower), and
+// the lanes that hold a triangle wait until they are half as many as those that hold a node
+// (kGateRatio; 29.5 ms of tracing per 64-spp frame of the 1M-triangle displaced sphere at 1920x1080,
+// 30.5 at a ratio of 1, 29.8 at 3, 31.1 at 6 and 38.0 without waiting; 43 ms before both). The lanes carry
+// rays of any kind: a shadow ray's triangle test (Triangle::simpleIntersect) is the closest-hit test with
+// the triangle's second and third corners exchanged and wider margins.
+// The launch asks for 7 waves per SIMD (at most 72 VGPRs).
 // kCount: the counting instantiation, which also adds every lane's render-node fetches and
 // triangle tests per ray kind (path, shadow, MIS) to traceCounts[0..5] (nodes, tests per kind).
+constexpr int kGateRatio = 2;
+// fewest lanes of a wave that carry rays
+constexpr int kMinWidth = 4;
+
 template <int BS, bool kCount>
 __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict__ scenes, const WfRay* __restrict__ rays, WfHit* __restrict__ hits,
                                                  const int32_t* __restrict__ ext, const int32_t* __restrict__ extCount,
                                                  int32_t* __restrict__ bins, int32_t* __restrict__ hist, int nBins,
-                                                 const WfShadow* __restrict__ shadows, const int32_t* __restrict__ shadowCount,
-                                                 const WfMis* __restrict__ misRays, const int32_t* __restrict__ misCount,
+                                                 const WfLightRay* __restrict__ shadows, const int32_t* __restrict__ shadowCount,
+                                                 const WfLightRay* __restrict__ misRays, const int32_t* __restrict__ misCount,
                                                  const int32_t* __restrict__ shadowQueue, const int32_t* __restrict__ misQueue,
                                                  WfNee* __restrict__ nee, int32_t* __restrict__ work,
                                                  unsigned long long* __restrict__ traceCounts) {
@@ -650,21 +590,134 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
     const int nM = misCount ? *misCount : 0;
     const int n = nE + nS + nM;
     const int segLen = ((n + kWfWorkSegments - 1) / kWfWorkSegments + 63) / 64 * 64;
-    int j = 0;
-    TraceTally tally[3];
+    // lanes of a wave that carry rays: 64, or fewer in a small launch so that every wave gets some (a step
+    // takes as long as the slowest of its lanes, and a wave with few lanes alternates less between node
+    // and triangle steps: 1.61 against 1.74 ms of tracing for one sample of an 853x479 frame)
+    const int waves = (int)gridDim.x * (BS / 64);
+    int width = 64;
+    while (width > kMinWidth && (long)width * waves > 2L * n) width >>= 1;
+    const int spare = 64 - width, refill = spare + width / 2;
+    int seg = 0;             // segments found empty so far
+    int next = 0, end = 0;   // items of the wave's current chunk that no lane has taken yet
+    unsigned long long tally[6] = {0, 0, 0, 0, 0, 0};
+    int spill[kStack - kShortStack];
+    // the lane's ray: path, kind (-1: none), direction, bound and hit
+    TraceLane l;
+    l.cur = kTraceDone; l.sp = 1; l.o = l.inv = v3(0, 0, 0); l.nx = l.ny = l.nz = false;
+    const TraceRec* recs = nullptr;
+    int path = 0, kind = -1, best = -1, mat = 0;
+    V3 d = v3(0, 0, 0);
+    float tMax = 0, hu = 0, hv = 0, hInvDet = 0;
     for (;;) {
-        const int k = wave_fetch_segmented(work, segLen, j);
-        if (j >= kWfWorkSegments) break;
-        if (k >= n) continue;
-        if (k < nE) extend_item(scenes, rays, hits, ext[k], ts, bins, lh, filing, nBins, kCount ? &tally[0] : nullptr);
-        else if (k < nE + nS) shadow_item(scenes, shadows, nee, shadowQueue[k - nE], ts, kCount ? &tally[1] : nullptr);
-        else mis_item(scenes, misRays, nee, misQueue[k - nE - nS], ts, kCount ? &tally[2] : nullptr);
+        const unsigned long long idle = __ballot(l.cur == kTraceDone);
+        const bool dry = seg >= kWfWorkSegments && next >= end;
+        if (idle == ~0ull || (!dry && __popcll(idle) >= refill)) {
+            if (l.cur == kTraceDone && kind >= 0) {
+                if (kind == 0) {
+                    WfHit o;
+                    o.leaf = best; o.u = hu; o.v = hv; o.invDet = hInvDet;
+                    hits[path] = o;
+                    if (filing) {
+                        // the hit is also filed under its material bin (misses in the last) for the counting sort
+                        const int bin = best < 0 ? nBins - 1 : min(mat, nBins - 2);
+                        bins[path] = bin;
+                        atomicAdd(&lh[bin], 1);
+                    }
+                } else if (mat == 0) {  // nothing blocked the light ray
+                    const float4 c = reinterpret_cast<const float4*>((kind == 1 ? shadows : misRays) + path)[2];
+                    float* p = kind == 1 ? nee[path].p1 : nee[path].p2;
+                    p[0] = c.x; p[1] = c.y; p[2] = c.z;
+                }
+                kind = -1;
+            }
+            if (next >= end) {
+                // workgroups are dealt to the 8 XCDs round robin: the waves of XCD blockIdx % 8 start on
+                // their own segment and keep neighbouring rays in one L2, then move on to the others
+                while (seg < kWfWorkSegments) {
+                    const int s = (blockIdx.x + seg) % kWfWorkSegments;
+                    int base = 0;
+                    if ((threadIdx.x & 63) == 0) base = atomicAdd(&work[kWfWorkStride * s], width);
+                    base = __builtin_amdgcn_readfirstlane(base);
+                    if (base < segLen) {
+                        next = s * segLen + base;
+                        end = min(next + width, n);
+                        if (next < end) break;
+                    }
+                    seg++;
+                }
+                if (seg >= kWfWorkSegments) {
+                    next = end = 0;
+                    if (idle == ~0ull) break;
+                    continue;
+                }
+            }
+            const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0));
+            const int k = next + rank;
+            const int give = min((int)__popcll(idle) - spare, end - next);
+            if (l.cur == kTraceDone && rank < give) {
+                const float4* src;
+                if (k < nE) {
+                    kind = 0;
+                    path = ext[k];
+                    src = reinterpret_cast<const float4*>(rays + path);
+                } else if (k < nE + nS) {
+                    kind = 1;
+                    path = shadowQueue[k - nE];
+                    src = reinterpret_cast<const float4*>(shadows + path);
+                } else {
+                    kind = 2;
+                    path = misQueue[k - nE - nS];
+                    src = reinterpret_cast<const float4*>(misRays + path);
+                }
+                const float4 a = src[0], b = src[1];
+                best = -1;
+                tMax = INFINITY;
+                if (kind > 0) {
+                    tMax = src[2].w;
+                    best = __float_as_int(b.w);
+                }
+                const SceneView& sv = scenes[__float_as_int(b.z)];
+                recs = sv.recs;
+                d = v3(a.w, b.x, b.y);
+                mat = 0;
+                hu = hv = hInvDet = 0;
+                trace_begin(l, v3(a.x, a.y, a.z), d, sv.root, ts);
+            }
+            next += give;
+            continue;
+        }
+        const bool done = l.cur == kTraceDone, leafStep = l.cur < 0 && !done;
+        const unsigned long long waiting = __ballot(leafStep), walking = __ballot(l.cur >= 0);
+        if (walking != 0 && kGateRatio * __popcll(waiting) < __popcll(walking)) {
+            if (l.cur >= 0) {
+                if (kCount) tally[0] += kind == 0, tally[2] += kind == 1, tally[4] += kind == 2;
+                trace_node(l, recs, tMax, ts, spill);
+            }
+        } else if (leafStep) {
+            if (kCount) tally[1] += kind == 0, tally[3] += kind == 1, tally[5] += kind == 2;
+            const TraceTri tr = trace_triangle(l, recs);
+            Ray r;
+            r.o = l.o; r.d = d; r.tMax = tMax;
+            const bool shadow = kind == 1;
+            const V3 p1 = shadow ? tr.p2 : tr.p1, p2 = shadow ? tr.p1 : tr.p2;
+            const float limit = shadow ? kOnePlusEpsF : kOneMinusEpsF;
+            float t, u, v, id;
+            bool over = false;
+            if (tri_mt(tr.p0, p1, p2, r, limit, t, u, v, id) && t > 0 && (t < tMax || (t == tMax && !shadow && tr.leaf < best))) {
+                if (kind == 0) {
+                    tMax = t;
+                    best = tr.leaf; mat = tr.mat; hu = u; hv = v; hInvDet = id;
+                } else if (!shadow || leaf_box_passes(tr.p0, tr.p1, tr.p2, r)) {
+                    mat = 1;  // blocked
+                    over = true;
+                }
+            }
+            if (over) l.cur = kTraceDone;
+            else trace_pop(l, ts, spill);
+        }
     }
     if constexpr (kCount) {
-        for (int q = 0; q < 3; q++) {
-            atomicAdd(&traceCounts[2 * q], tally[q].nodes);
-            atomicAdd(&traceCounts[2 * q + 1], tally[q].tris);
-        }
+        for (int q = 0; q < 6; q++) atomicAdd(&traceCounts[q], tally[q]);
     }
     if (filing) {
         __syncthreads();

@@ -151,7 +151,7 @@ LTS_D bool visible(const SceneView& sv, const BVertex& a, const BVertex& b, Trac
 }
 
 // A surface vertex from a closest hit.
-LTS_D void surface_vertex(const SceneView& sv, BVertex& v, const SurfacePoint& si, const int* perm) {
+LTS_D void surface_vertex(const SceneView& sv, BVertex& v, const SurfacePoint& si, const NoiseTables& perm) {
     v.kind = kVSurface;
     v.p = si.p; v.n = si.n; v.sn = si.sn; v.pError = si.pError; v.wo = si.wo;
     v.light = sv.shade[si.leaf].light;
@@ -163,7 +163,7 @@ LTS_D void surface_vertex(const SceneView& sv, BVertex& v, const SurfacePoint& s
 // or an absorbed sample. pdfDir is the solid-angle density the ray's direction was sampled with.
 // Camera walks record an escape as a vertex of the infinite light.
 LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool importance, BVertex* path, int k0,
-               int maxVerts, const Sampler& smp, uint32_t block, TraceStack ts, const int* perm, const CamRays* cr) {
+               int maxVerts, const Sampler& smp, uint32_t block, TraceStack ts, const NoiseTables& perm, const CameraSample* cs, int spp) {
     int k = k0;
     while (k < maxVerts) {
         Hit h = trace_closest(sv, ray, ts, nullptr, nullptr);
@@ -184,7 +184,7 @@ LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool impor
             break;
         }
         SurfacePoint si = make_surface(sv, h.leaf, ray, h.u, h.v, h.invDet);
-        if (cr && k == 1) differentials(si, *cr, uv_derivative_scale(sv, h.leaf, h.invDet));
+        if (cs && k == 1) camera_footprint(sv, si, *cs, spp, ray, h.invDet);
         surface_vertex(sv, v, si, perm);
         v.beta = beta;
         v.pdfFwd = to_area(pdfDir, prev, v);
@@ -227,7 +227,7 @@ LTS_D SurfacePoint light_point(const SceneView& sv, const LightDesc& L, V2 u) {
 }
 
 LTS_D int light_subpath(const SceneView& sv, BVertex* path, const Sampler& smp, int maxVerts, TraceStack ts,
-                        const int* perm) {
+                        const NoiseTables& perm) {
     if (sv.nLights == 0 || maxVerts < 1) return 0;
     float u0[4], u1[4];
     smp.block(kBlockLightStart, u0);
@@ -260,7 +260,7 @@ LTS_D int light_subpath(const SceneView& sv, BVertex* path, const Sampler& smp, 
     r.o = offsetRayOrigin(lp.p, lp.pError, lp.n, w);
     r.d = w;
     r.tMax = INFINITY;
-    return walk(sv, r, beta, pdfDir, true, path, 1, maxVerts, smp, kBlockLightWalk, ts, perm, nullptr);
+    return walk(sv, r, beta, pdfDir, true, path, 1, maxVerts, smp, kBlockLightWalk, ts, perm, nullptr, 0);
 }
 
 LTS_D float remap0(float f) { return f != 0 ? f : 1.0f; }
@@ -364,17 +364,18 @@ LTS_D Spec connect(const SceneView& sv, const BVertex* lp, const BVertex* cp, in
 }
 
 LTS_D Spec bdpt_radiance(const SceneView& sv, int px, int py, int sample, const RenderLaunch& rl, TraceStack ts,
-                         const int* perm) {
+                         const NoiseTables& perm) {
     Sampler smp;
     smp.seed = rl.seed;
     smp.pixel = (uint32_t)(py * sv.cam.width + px);
     smp.sample = (uint32_t)sample;
     const int maxBounce = rl.maxBounce;
     BVertex cp[kCamVerts], lp[kLightVerts];
-    CamRays cr = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
+    const CameraSample cs = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
+    const Ray camRay = camera_ray(sv, cs);
     BVertex& c0 = cp[0];
     c0.kind = kVCamera;
-    c0.p = cr.r.o;
+    c0.p = camRay.o;
     c0.n = c0.sn = c0.pError = c0.wo = v3(0, 0, 0);
     c0.beta = spec(1.0f);
     c0.pdfFwd = c0.pdfRev = 0.0f;
@@ -382,7 +383,7 @@ LTS_D Spec bdpt_radiance(const SceneView& sv, int px, int py, int sample, const 
     c0.delta = false;
     c0.bsdf.kind = -1;
     // pdfDir of the camera ray only feeds the t = 1 strategies, which are not used
-    const int nCam = walk(sv, cr.r, spec(1.0f), 0.0f, false, cp, 1, maxBounce + 2, smp, kBlockCamWalk, ts, perm, &cr);
+    const int nCam = walk(sv, camRay, spec(1.0f), 0.0f, false, cp, 1, maxBounce + 2, smp, kBlockCamWalk, ts, perm, &cs, rl.spp);
     const int nLight = light_subpath(sv, lp, smp, maxBounce + 1, ts, perm);
     Spec L = spec(0.0f);
     for (int t = 2; t <= nCam; t++)
@@ -397,8 +398,8 @@ LTS_D Spec bdpt_radiance(const SceneView& sv, int px, int py, int sample, const 
 // 1920x1080, against 38.0 ms at the three waves its natural 165 VGPRs allow and 34.3 ms at five.
 __global__ __launch_bounds__(256, 4) void k_bdpt(SceneView sv, RenderLaunch rl) {
     __shared__ int stk[kShortStack * 256];
-    __shared__ int perm[512];
-    for (int i = threadIdx.x; i < 512; i += 256) perm[i] = sv.perm[i];
+    __shared__ NoiseTables perm;
+    noise_tables(perm, sv.perm, threadIdx.x, 256);
     __syncthreads();
     const int W = sv.cam.width, H = sv.cam.height;
     const int tilesX = (W + kTileSide - 1) / kTileSide;

@@ -18,11 +18,43 @@ constexpr float SHADOW_EPS = 0.0001f;                 // core/ErrorHelper.cuh:40
 
 // Transcendentals: evaluated in fp64 and rounded once, a last-bit-stable definition of the fp32
 // function shared by every code path.
-LTS_D float f_sin(float x) { return (float)sin((double)x); }
-LTS_D float f_cos(float x) { return (float)cos((double)x); }
-LTS_D float f_acos(float x) { return (float)acos((double)x); }
-LTS_D float f_log2(float x) { return (float)log2((double)x); }
-LTS_D float f_log(float x) { return (float)log((double)x); }
+// The rarely taken ones stay out of line: inlined, their fp64 constants are hoisted out of a kernel's
+// loop and hold registers across it.
+#define LTS_D_CALL static __device__ __attribute__((noinline))
+LTS_D_CALL float f_sin(float x) { return (float)sin((double)x); }
+LTS_D_CALL float f_sin_acos(float x) { return (float)sin((double)(float)acos((double)x)); }
+LTS_D_CALL float f_log2(float x) { return (float)log2((double)x); }
+
+// sin and cos of an angle in [0, 2 pi], the range of every sampled azimuth: one reduction by multiples
+// of pi / 2 (two-part constant, fused) and the Taylor series of both on [-pi/4, pi/4] in fp64, to terms
+// below 1e-17. Rounded to float it equals f_sin and f_cos at all 2^24 azimuths 2 pi k / 2^24 the sampler
+// can draw; about 30 fp64 operations where the two library calls take some 130 and a rarely taken
+// branch each.
+__device__ __constant__ const double kSinCos[18] = {
+    1.0 / 355687428096000.0, -1.0 / 1307674368000.0, 1.0 / 6227020800.0, -1.0 / 39916800.0, 1.0 / 362880.0, -1.0 / 5040.0,
+    1.0 / 120.0, -1.0 / 6.0,  // sin: 1 / 17! .. 1 / 3!
+    -1.0 / 6402373705728000.0, 1.0 / 20922789888000.0, -1.0 / 87178291200.0, 1.0 / 479001600.0, -1.0 / 3628800.0,
+    1.0 / 40320.0, -1.0 / 720.0, 1.0 / 24.0, -0.5, 1.0};  // cos: 1 / 18! .. 1
+LTS_D void f_sincos(float x, float& sinOut, float& cosOut) {
+    const double k = rint((double)x * 0x1.45f306dc9c883p-1);
+    const double r = __builtin_fma(k, -0x1.1a62633145c07p-54, __builtin_fma(k, -0x1.921fb54442d18p+0, (double)x));
+    const double z = r * r;
+    // the coefficients are read where they are used: hoisted out of a kernel's loop they would hold 36
+    // registers across it
+    const double* t = kSinCos;
+    asm volatile("" : "+s"(t));
+    double s = t[0], c = t[8];
+#pragma unroll
+    for (int i = 1; i < 8; i++) s = __builtin_fma(s, z, t[i]);
+#pragma unroll
+    for (int i = 9; i < 18; i++) c = __builtin_fma(c, z, t[i]);
+    s = __builtin_fma(s * z, r, r);
+    const int q = (int)k;
+    const float sf = (float)s, cf = (float)c;
+    const float a = (q & 1) ? cf : sf, b = (q & 1) ? sf : cf;
+    sinOut = (q & 2) ? -a : a;
+    cosOut = ((q + 1) & 2) ? -b : b;
+}
 
 LTS_D uint32_t fbits(float f) { return __float_as_uint(f); }
 LTS_D float bitsf(uint32_t u) { return __uint_as_float(u); }

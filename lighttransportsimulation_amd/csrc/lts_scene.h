@@ -75,7 +75,7 @@ struct MatDesc {
     float extra;     // roughness (matte, microfacet) or eta (glass)
     float onA, onB;  // Oren-Nayar A, B (matte with roughness != 0)
     float alpha;     // Trowbridge-Reitz alpha (microfacet)
-    int32_t pad;
+    int32_t footprint;  // 1: a texture of the material reads the hit's differentials
 };
 
 struct MipLevelDesc {

@@ -419,7 +419,9 @@ LTS_D Ray spawn_ray(const SurfacePoint& it, V3 d) {
 LTS_D V2 uniform_disk(V2 u) {
     float r = sqrtf(u.x);
     float theta = 2 * PI_F * u.y;
-    return v2(r * f_cos(theta), r * f_sin(theta));
+    float sn, cs;
+    f_sincos(theta, sn, cs);
+    return v2(r * cs, r * sn);
 }
 LTS_D V3 cosine_hemisphere(V2 u) {
     V2 d = uniform_disk(u);
@@ -430,7 +432,9 @@ LTS_D V3 uniform_hemisphere(V2 u) {
     float z = u.x;
     float r = sqrtf(fmaxf(0.0f, 1.0f - z * z));
     float phi = 2 * PI_F * u.y;
-    return v3(r * f_cos(phi), r * f_sin(phi), z);
+    float sn, cs;
+    f_sincos(phi, sn, cs);
+    return v3(r * cs, r * sn, z);
 }
 LTS_D float power_heuristic(float fPdf, float gPdf) {
     float f = 1 * fPdf, g = 1 * gPdf;
@@ -500,8 +504,10 @@ LTS_D void tr_sample11(float cosTheta, float U1, float U2, float* sx, float* sy)
     if ((double)cosTheta > .9999) {
         float r = sqrtf(U1 / (1 - U1));
         float phi = (float)(6.28318530718 * (double)U2);
-        *sx = r * f_cos(phi);
-        *sy = r * f_sin(phi);
+        float sn, cs;
+        f_sincos(phi, sn, cs);
+        *sx = r * cs;
+        *sy = r * sn;
         return;
     }
     float sinTheta = sqrtf(fmaxf(0.0f, 1.0f - cosTheta * cosTheta));
@@ -665,60 +671,94 @@ LTS_D float smooth_step(float mn, float mx, float val) {
     float v = clampf((val - mn) / (mx - mn), 0, 1);
     return v * v * (-2 * v + 3);
 }
-LTS_D float grad(const int* __restrict__ perm, int x, int y, int z, float dx, float dy, float dz) {
-    int h = perm[perm[perm[x] + y] + z];
-    h &= 15;
-    float u = h < 8 || h == 12 || h == 13 ? dx : dy;
-    float v = h < 4 || h == 12 || h == 13 ? dy : dz;
-    return ((h & 1) ? -u : u) + ((h & 2) ? -v : v);
+// The noise's tables in LDS: the permutation, whose three chained lookups a kernel's lanes make eight
+// times per noise value, and for each entry the gradient its last lookup selects (x, y, z in {-1, 0, 1}
+// as fp16 pairs): the reference's choice of two coordinates and their signs (Procedural.cuh grad) as a
+// dot product of three mixed-precision fused operations, exact but for the one rounding of the sum of
+// its two nonzero terms, as the reference's addition rounds.
+struct NoiseTables {
+    int perm[512];
+    uint2 grad[512];
+};
+LTS_D void noise_tables(NoiseTables& t, const int* __restrict__ perm, int tid, int threads) {
+    for (int i = tid; i < 512; i += threads) {
+        const int w = perm[i], h = w & 15;
+        const unsigned one = 0x3c00u, su = (h & 1) ? 0x8000u : 0u, sv = (h & 2) ? 0x8000u : 0u;
+        const bool ux = h < 8 || h == 12 || h == 13, vy = h < 4 || h == 12 || h == 13;
+        const unsigned gx = ux ? one | su : 0u, gy = (ux ? 0u : one | su) | (vy ? one | sv : 0u), gz = vy ? 0u : one | sv;
+        t.perm[i] = w;
+        t.grad[i] = make_uint2(gx | (gy << 16), gz);
+    }
 }
-LTS_D float perlin(const int* __restrict__ P, V3 p) {
+LTS_D float grad(const NoiseTables& t, int i, float dx, float dy, float dz) {
+    typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+    const uint2 g = t.grad[i];
+    const Half2 xy = __builtin_bit_cast(Half2, g.x), z = __builtin_bit_cast(Half2, g.y);
+    return __builtin_fmaf((float)xy.x, dx, __builtin_fmaf((float)xy.y, dy, __builtin_fmaf((float)z.x, dz, 0.0f)));
+}
+LTS_D float perlin(const NoiseTables& t, V3 p) {
     int ix = (int)floorf(p.x), iy = (int)floorf(p.y), iz = (int)floorf(p.z);
     float dx = p.x - ix, dy = p.y - iy, dz = p.z - iz;
     ix &= 255; iy &= 255; iz &= 255;
-    float w000 = grad(P, ix, iy, iz, dx, dy, dz);
-    float w100 = grad(P, ix + 1, iy, iz, dx - 1, dy, dz);
-    float w010 = grad(P, ix, iy + 1, iz, dx, dy - 1, dz);
-    float w001 = grad(P, ix, iy, iz + 1, dx, dy, dz - 1);
-    float w110 = grad(P, ix + 1, iy + 1, iz, dx - 1, dy - 1, dz);
-    float w011 = grad(P, ix, iy + 1, iz + 1, dx, dy - 1, dz - 1);
-    float w101 = grad(P, ix + 1, iy, iz + 1, dx - 1, dy, dz - 1);
-    float w111 = grad(P, ix + 1, iy + 1, iz + 1, dx - 1, dy - 1, dz - 1);
+    const int p0 = t.perm[ix] + iy, p1 = t.perm[ix + 1] + iy;
+    const int p00 = t.perm[p0] + iz, p01 = t.perm[p0 + 1] + iz, p10 = t.perm[p1] + iz, p11 = t.perm[p1 + 1] + iz;
+    float w000 = grad(t, p00, dx, dy, dz);
+    float w100 = grad(t, p10, dx - 1, dy, dz);
+    float w010 = grad(t, p01, dx, dy - 1, dz);
+    float w001 = grad(t, p00 + 1, dx, dy, dz - 1);
+    float w110 = grad(t, p11, dx - 1, dy - 1, dz);
+    float w011 = grad(t, p01 + 1, dx, dy - 1, dz - 1);
+    float w101 = grad(t, p10 + 1, dx - 1, dy, dz - 1);
+    float w111 = grad(t, p11 + 1, dx - 1, dy - 1, dz - 1);
     float wx = noise_weight(dx), wy = noise_weight(dy), wz = noise_weight(dz);
     float x00 = lerpf(wx, w000, w100), x10 = lerpf(wx, w010, w110);
     float x01 = lerpf(wx, w001, w101), x11 = lerpf(wx, w011, w111);
     float y0 = lerpf(wy, x00, x10), y1 = lerpf(wy, x01, x11);
     return lerpf(wz, y0, y1);
 }
-LTS_D float fbm(const int* P, V3 p, V3 dpdx, V3 dpdy, float omega, int maxOct) {
+// Octaves of a footprint: clamp(-1 - log2(len2) / 2, 0, maxOct). At or below 2^(-2 maxOct - 2) (every
+// hit after the first bounce, which has no footprint, and most first ones) it is maxOct: rounding is
+// monotone, so the rounded logarithm is at most -2 maxOct - 2.
+LTS_D float noise_octaves(V3 dpdx, V3 dpdy, int maxOct) {
     float len2 = fmaxf(lengthSq(dpdx), lengthSq(dpdy));
-    float n = clampf(-1 - 0.5f * f_log2(len2), 0, (float)maxOct);
-    int nInt = (int)floorf(n);
+    if (maxOct >= 0 && len2 <= __builtin_amdgcn_ldexpf(1.0f, -2 * maxOct - 2)) return (float)maxOct;
+    return clampf(-1 - 0.5f * f_log2(len2), 0, (float)maxOct);
+}
+// fbm (turb false) or turbulence over n = noise_octaves octaves: the whole ones, then the fraction, with
+// one copy of the noise code for all of them (every inlined copy is 1.5 KB of instructions, and the
+// shading kernels once held thirty). The fraction is skipped where its weight is 0 (a whole number of
+// octaves): one noise value in seven at six octaves.
+LTS_D float noise_sum(const NoiseTables& T, V3 p, float n, float omega, int maxOct, bool turb) {
+    const int nInt = (int)floorf(n);
+    const float part = smooth_step(0.3f, 0.7f, n - nInt);
+    const int count = nInt + (part != 0);
     float sum = 0, lambda = 1, o = 1;
-    for (int i = 0; i < nInt; i++) { sum += o * perlin(P, p * lambda); lambda *= 1.99f; o *= omega; }
-    float nPartial = n - nInt;
-    sum += o * smooth_step(0.3f, 0.7f, nPartial) * perlin(P, p * lambda);
+#pragma unroll 1
+    for (int i = 0; i < count; i++) {
+        float v = perlin(T, p * lambda);
+        if (turb) v = fabsf(v);
+        if (i < nInt) {
+            sum += o * v;
+            lambda *= 1.99f;
+            o *= omega;
+        } else {
+            sum += turb ? o * lerpf(part, 0.2f, v) : o * part * v;
+        }
+    }
+    if (turb) {
+        if (part == 0) sum += o * 0.2f;
+#pragma unroll 1
+        for (int i = nInt; i < maxOct; i++) { sum += o * 0.2f; o *= omega; }
+    }
     return sum;
 }
-LTS_D float turbulence(const int* P, V3 p, V3 dpdx, V3 dpdy, float omega, int maxOct) {
-    float len2 = fmaxf(lengthSq(dpdx), lengthSq(dpdy));
-    float n = clampf(-1 - 0.5f * f_log2(len2), 0, (float)maxOct);
-    int nInt = (int)floorf(n);
-    float sum = 0, lambda = 1, o = 1;
-    for (int i = 0; i < nInt; i++) { sum += o * fabsf(perlin(P, p * lambda)); lambda *= 1.99f; o *= omega; }
-    float nPartial = n - nInt;
-    sum += o * lerpf(smooth_step(0.3f, 0.7f, nPartial), 0.2f, fabsf(perlin(P, p * lambda)));
-    for (int i = nInt; i < maxOct; i++) { sum += o * 0.2f; o *= omega; }
-    return sum;
-}
-LTS_D Spec marble_tex(const int* P, const TexDesc& X, V3 p, V3 dpdx, V3 dpdy) {
+// MarbleTexture's colour at m = p.y + variation * fbm
+LTS_D Spec marble_colour(float m) {
     // MarbleTexture colours (Procedural.cuh:278-282); the zero row stands in for the read past the
     // table at t == 1, where its weight is exactly 0
     const float C[10][3] = {{.58f, .58f, .6f}, {.58f, .58f, .6f}, {.58f, .58f, .6f}, {.5f, .5f, .5f},
                             {.6f, .59f, .58f}, {.58f, .58f, .6f}, {.58f, .58f, .6f}, {.2f, .2f, .33f},
                             {.58f, .58f, .6f}, {0, 0, 0}};
-    p = p * X.scale;
-    float m = p.y + X.variation * fbm(P, p, dpdx * X.scale, dpdy * X.scale, X.omega, X.octaves);
     float t = 0.5f + 0.5f * f_sin(m);
     int first = (int)floorf(t * 6.0f);
     first = first < 0 ? 0 : (first > 6 ? 6 : first);  // t is in [0, 1]; the clamp only fences NaN
@@ -767,7 +807,7 @@ LTS_D Spec mip_triangle(const SceneView& sv, const MipDesc& m, int l, V2 st) {
 // width of the lookup and reads the top level correctly (the reference swaps texel's arguments
 // there: texel (levels - 1, 0) of level 0).
 LTS_D Spec mip_lookup(const SceneView& sv, const MipDesc& m, V2 st, float width) {
-    float levels = m.filtered ? (float)(m.levels - 1) + (float)log2((double)fmaxf(width, (float)1e-8)) : m.lookupLevel;
+    float levels = m.filtered ? (float)(m.levels - 1) + f_log2(fmaxf(width, (float)1e-8)) : m.lookupLevel;
     if (levels < 0) return mip_triangle(sv, m, 0, st);
     if (levels >= m.levels - 1) return m.filtered ? mip_texel(sv, m, 0, 0, m.levels - 1) : mip_texel(sv, m, m.levels - 1, 0, 0);
     int iLevel = (int)floorf(levels);
@@ -775,26 +815,25 @@ LTS_D Spec mip_lookup(const SceneView& sv, const MipDesc& m, V2 st, float width)
     return lerpS(delta, mip_triangle(sv, m, iLevel, st), mip_triangle(sv, m, iLevel + 1, st));
 }
 
-// `perm` is the Perlin permutation (sv.perm or a copy of it in LDS).
-LTS_D Spec eval_tex(const SceneView& sv, int ti, const SurfacePoint& s, const int* perm) {
+LTS_D Spec eval_tex(const SceneView& sv, int ti, const SurfacePoint& s, const NoiseTables& noise) {
     const TexDesc& X = sv.texs[ti];
-    switch (X.type) {
-        case TEX_CONST: return spec(X.c[0], X.c[1], X.c[2]);
-        case TEX_IMAGE: {
-            // filtered pipeline: PBRT's isotropic width 2 max(|ds/dx|, |dt/dx|, |ds/dy|, |dt/dy|) of
-            // UVMapping2D (st = uv, Mapping.cuh:19-37); the reference's lookup ignores it
-            const float width = 2 * fmaxf(fmaxf(fabsf(s.dudx), fabsf(s.dvdx)), fmaxf(fabsf(s.dudy), fabsf(s.dvdy)));
-            return mip_lookup(sv, sv.mips[X.img], v2(1 * s.uv.x + 0, 1 * s.uv.y + 0), width);
-        }
-        case TEX_FBM: return spec(fbm(perm, identityMap(s.p), identityMap(s.dpdx), identityMap(s.dpdy), X.omega, X.octaves));
-        case TEX_WRINKLED: return spec(turbulence(perm, identityMap(s.p), identityMap(s.dpdx), identityMap(s.dpdy), X.omega, X.octaves));
-        case TEX_MARBLE: return marble_tex(perm, X, identityMap(s.p), identityMap(s.dpdx), identityMap(s.dpdy));
+    if (X.type == TEX_CONST) return spec(X.c[0], X.c[1], X.c[2]);
+    if (X.type == TEX_IMAGE) {
+        // filtered pipeline: PBRT's isotropic width 2 max(|ds/dx|, |dt/dx|, |ds/dy|, |dt/dy|) of
+        // UVMapping2D (st = uv, Mapping.cuh:19-37); the reference's lookup ignores it
+        const float width = 2 * fmaxf(fmaxf(fabsf(s.dudx), fabsf(s.dvdx)), fmaxf(fabsf(s.dudy), fabsf(s.dvdy)));
+        return mip_lookup(sv, sv.mips[X.img], v2(1 * s.uv.x + 0, 1 * s.uv.y + 0), width);
     }
-    return spec(0.0f);
+    const bool marble = X.type == TEX_MARBLE;
+    if (!marble && X.type != TEX_FBM && X.type != TEX_WRINKLED) return spec(0.0f);
+    V3 p = identityMap(s.p), dx = identityMap(s.dpdx), dy = identityMap(s.dpdy);
+    if (marble) { p = p * X.scale; dx = dx * X.scale; dy = dy * X.scale; }
+    const float v = noise_sum(noise, p, noise_octaves(dx, dy, X.octaves), X.omega, X.octaves, X.type == TEX_WRINKLED);
+    return marble ? marble_colour(p.y + X.variation * v) : spec(v);
 }
 
 // Material::computeScatteringFunctions (materials/Material.cuh:31-130)
-LTS_D Bsdf make_bsdf(const SceneView& sv, const SurfacePoint& s, const int* perm) {
+LTS_D Bsdf make_bsdf(const SceneView& sv, const SurfacePoint& s, const NoiseTables& noise) {
     Bsdf b;
     b.ns = s.sn; b.ng = s.n;
     b.ss = normalize(s.sdpdu);
@@ -803,30 +842,19 @@ LTS_D Bsdf make_bsdf(const SceneView& sv, const SurfacePoint& s, const int* perm
     b.R = b.T = spec(0.0f);
     b.A = b.B = b.eta = b.alpha = 0;
     const MatDesc& M = sv.mats[sv.shade[s.leaf].mat];
+    Spec r = spec(0.0f), t = spec(0.0f);
+#pragma unroll 1
+    for (int k = 0; k < (M.type == MAT_GLASS ? 2 : 1); k++) {  // one copy of the texture code
+        t = eval_tex(sv, k ? M.tex1 : M.tex0, s, noise);
+        if (k == 0) r = t;
+    }
+    if (isBlack(r) && (M.type != MAT_GLASS || isBlack(t))) return b;
+    b.R = r;
     switch (M.type) {
-        case MAT_MATTE: {
-            Spec kd = eval_tex(sv, M.tex0, s, perm);
-            if (!isBlack(kd)) { b.R = kd; b.type = B_REFL | B_DIFF; b.kind = M.extra == 0 ? 0 : 1; b.A = M.onA; b.B = M.onB; }
-            break;
-        }
-        case MAT_GLASS: {
-            Spec r = eval_tex(sv, M.tex0, s, perm), t = eval_tex(sv, M.tex1, s, perm);
-            if (isBlack(r) && isBlack(t)) break;
-            b.kind = 3; b.type = B_REFL | B_TRANS | B_SPEC; b.R = r; b.T = t; b.eta = M.extra;
-            break;
-        }
-        case MAT_MIRROR: {
-            Spec r = eval_tex(sv, M.tex0, s, perm);
-            if (isBlack(r)) break;
-            b.kind = 2; b.type = B_REFL | B_SPEC; b.R = r;
-            break;
-        }
-        case MAT_MICROFACET: {
-            Spec r = eval_tex(sv, M.tex0, s, perm);
-            if (isBlack(r)) break;
-            b.kind = 4; b.type = B_REFL | B_GLOSSY; b.R = r; b.alpha = M.alpha;
-            break;
-        }
+        case MAT_MATTE: b.type = B_REFL | B_DIFF; b.kind = M.extra == 0 ? 0 : 1; b.A = M.onA; b.B = M.onB; break;
+        case MAT_GLASS: b.kind = 3; b.type = B_REFL | B_TRANS | B_SPEC; b.T = t; b.eta = M.extra; break;
+        case MAT_MIRROR: b.kind = 2; b.type = B_REFL | B_SPEC; break;
+        case MAT_MICROFACET: b.kind = 4; b.type = B_REFL | B_GLOSSY; b.alpha = M.alpha; break;
     }
     return b;
 }
@@ -852,19 +880,27 @@ LTS_D LightPoint tri_sample(const SceneView& sv, const LightDesc& L, V2 u) {
     return lp;
 }
 
-// Triangle::Pdf(it, wi) (shapes/Triangle.cu:211-225)
-LTS_D float tri_pdf(const SceneView& sv, const LightDesc& L, const SurfacePoint& it, V3 wi) {
-    Ray r = spawn_ray(it, wi);
+// Where a ray r spawned from `it` meets the triangle of area light L: the distance, whether it meets
+// the emitting side, and Triangle::Pdf(it, r.d) (shapes/Triangle.cu:211-225). False for a miss.
+struct LightHit {
+    float t, pdf;
+    bool front;
+};
+LTS_D bool light_hit(const SceneView& sv, const LightDesc& L, const SurfacePoint& it, const Ray& r, LightHit& h) {
     V3 p0, p1, p2; int prim;
     load_tri(sv.tris, L.leaf, p0, p1, p2, prim);
     float t, u, v, id;
-    if (!tri_hit(p0, p1, p2, r, t, u, v, id)) return 0;
+    h.pdf = 0;
+    if (!tri_hit(p0, p1, p2, r, t, u, v, id)) return false;
     SurfacePoint is = make_surface(sv, L.leaf, r, u, v, id);
-    return lengthSq(it.p - is.p) / (absDot(is.n, -wi) * L.area);
+    h.t = t;
+    h.front = dot(is.n, -r.d) > 0.f;
+    h.pdf = lengthSq(it.p - is.p) / (absDot(is.n, -r.d) * L.area);
+    return true;
 }
 
 LTS_D float inf_pdf(V3 wi) {
-    float sinTheta = f_sin(f_acos(clampf(wi.z, -1.0f, 1.0f)));
+    float sinTheta = f_sin_acos(clampf(wi.z, -1.0f, 1.0f));
     return (0.5f * INV_PI_F) / (2 * PI_F * PI_F * sinTheta);
 }
 
@@ -874,7 +910,9 @@ LTS_D Spec sample_li(const SceneView& sv, const LightDesc& L, const SurfacePoint
     if (L.kind == 0) {
         LightPoint ps = tri_sample(sv, L, u);
         *wi = normalize(ps.p - it.p);
-        *pdf = tri_pdf(sv, L, it, *wi);
+        LightHit lh;
+        light_hit(sv, L, it, spawn_ray(it, *wi), lh);
+        *pdf = lh.pdf;
         *target = ps;
         return dot(ps.n, -*wi) > 0.f ? light_le(L) : spec(0.0f);
     }
@@ -913,35 +951,35 @@ LTS_D int sample_light(const SceneView& sv, float u, float* pdf) {
     return off;
 }
 
-// The light test of the MIS-BSDF ray (IntegratorHelper.cuh:103-122): whether the closest hit of r
-// (spawned with tMax = infinity) is light li's triangle, seen from its emitting side, or for the
-// infinite light whether r escapes. The closest-hit traversal is not needed for that. A ray that
-// misses the light's triangle, or meets its back, contributes nothing whatever lies in front
-// (mis_target is false). A ray that meets its front at t reaches it unless some triangle would win the
-// closest hit against it (nearer, or at exactly t with a lower leaf index, tri_hit_closest), which an
-// any-hit traversal bounded at t answers; the same t, u, v and 1/det come out of the triangle test
-// whatever tMax is. tMax and tieLeaf receive that traversal's bound.
-LTS_D bool mis_target(const SceneView& sv, const LightDesc& L, int li, const Ray& r, float& tMax, int& tieLeaf) {
+// The MIS-BSDF ray r = spawn_ray(si, wi) toward light li (IntegratorHelper.cuh:96-122): false when it
+// contributes nothing whatever lies in its way; else the weight of its contribution, and the any-hit
+// traversal that is left to do. The reference finds the closest hit and asks whether it is the light's
+// triangle seen from its emitting side, or for the infinite light whether the ray escapes. A ray that
+// misses the light's triangle, or meets its back, never contributes. A ray that meets its front at t
+// reaches it unless some triangle would win the closest hit against it (nearer, or at exactly t with a
+// lower leaf index, tri_hit_closest), which an any-hit traversal bounded at tMax = t with tieLeaf
+// answers; the same t, u, v and 1/det come out of the triangle test whatever tMax is.
+LTS_D bool mis_ray(const SceneView& sv, const LightDesc& L, int li, const SurfacePoint& si, const Ray& r, bool sampledSpecular,
+                   float scatteringPdf, float& weight, float& tMax, int& tieLeaf) {
+    weight = 1;
     tMax = INFINITY;
     tieLeaf = -1;
-    if (L.kind != 0) return true;
-    if (L.leaf < 0 || sv.shade[L.leaf].light != li) return false;
-    V3 p0, p1, p2; int prim;
-    load_tri(sv.tris, L.leaf, p0, p1, p2, prim);
-    float t, u, v, id;
-    if (!tri_hit(p0, p1, p2, r, t, u, v, id)) return false;
-    const SurfacePoint lt = make_surface(sv, L.leaf, r, u, v, id);
-    if (!(dot(lt.n, -r.d) > 0.f)) return false;
-    tMax = t;
-    tieLeaf = L.leaf;
+    if (L.kind == 0) {
+        LightHit lh;
+        const bool hit = light_hit(sv, L, si, r, lh);
+        if (!sampledSpecular) {
+            if (lh.pdf == 0) return false;
+            weight = power_heuristic(scatteringPdf, lh.pdf);
+        }
+        if (!hit || !lh.front || sv.shade[L.leaf].light != li) return false;
+        tMax = lh.t;
+        tieLeaf = L.leaf;
+    } else if (!sampledSpecular) {
+        const float lightPdf = inf_pdf(r.d);
+        if (lightPdf == 0) return false;
+        weight = power_heuristic(scatteringPdf, lightPdf);
+    }
     return true;
-}
-LTS_D bool mis_reaches_light(const SceneView& sv, const LightDesc& L, int li, Ray r, TraceStack ts) {
-    int tieLeaf;
-    float tMax;
-    if (!mis_target(sv, L, li, r, tMax, tieLeaf)) return false;
-    r.tMax = tMax;
-    return !trace_any<true>(sv, r, ts, nullptr, tieLeaf);
 }
 
 // estimateDirect (intergrators/IntegratorHelper.cuh:51-125)
@@ -968,16 +1006,15 @@ LTS_D Spec estimate_direct(const SceneView& sv, const SurfacePoint& si, const Bs
     int sampledType = 0;
     Spec f = bsdf.sampleF(si.wo, &wi, uScatter, &scatteringPdf, flags, &sampledType);
     f = f * absDot(wi, si.sn);
-    bool sampledSpecular = (sampledType & B_SPEC) != 0;
-    if (!isBlack(f) && scatteringPdf > 0) {
-        float weight = 1;
-        if (!sampledSpecular) {
-            lightPdf = L.kind == 0 ? tri_pdf(sv, L, si, wi) : inf_pdf(wi);
-            if (lightPdf == 0) return Ld;
-            weight = power_heuristic(scatteringPdf, lightPdf);
-        }
-        const Spec Li2 = mis_reaches_light(sv, L, li, spawn_ray(si, wi), ts) ? light_le(L) : spec(0.f);
-        if (!isBlack(Li2)) Ld = Ld + f * Li2 * spec(1.0f) * weight / scatteringPdf;
+    const bool sampledSpecular = (sampledType & B_SPEC) != 0;
+    const Spec Li2 = light_le(L);
+    if (!isBlack(f) && scatteringPdf > 0 && !isBlack(Li2)) {
+        Ray mr = spawn_ray(si, wi);
+        float weight;
+        int tieLeaf;
+        if (mis_ray(sv, L, li, si, mr, sampledSpecular, scatteringPdf, weight, mr.tMax, tieLeaf) &&
+            !trace_any<true>(sv, mr, ts, nullptr, tieLeaf))
+            Ld = Ld + f * Li2 * spec(1.0f) * weight / scatteringPdf;
     }
     return Ld;
 }
@@ -999,8 +1036,7 @@ LTS_D V2 film_sample(int px, int py, int sample, int spp, int stratified, const 
 
 // ---------------------------------------------------------------- camera (rendering/Camera.cu:51-81)
 struct CamRays {
-    Ray r;
-    V3 rxO, rxD, ryO, ryD;
+    V3 rxO, rxD, ryO, ryD;  // the differential rays
 };
 
 LTS_D void camera_ray(const CameraDesc& c, V2 pf, V2 lens, V3* o, V3* d) {
@@ -1013,32 +1049,43 @@ LTS_D void camera_ray(const CameraDesc& c, V2 pf, V2 lens, V3* o, V3* d) {
                    v3(c.up[0], c.up[1], c.up[2]) * pr.y - co - offset);
 }
 
-// generateDifferentialRay + Ray::scaleDifferentials(rsqrt(spp)) (Camera.cu:67-81, Ray.cuh:35-40)
-LTS_D CamRays camera_rays(const CameraDesc& c, V2 pFilm, V2 lens, int spp) {
-    CamRays cr;
-    camera_ray(c, pFilm, lens, &cr.r.o, &cr.r.d);
-    camera_ray(c, pFilm + v2(1, 0), lens, &cr.rxO, &cr.rxD);
-    camera_ray(c, pFilm + v2(0, 1), lens, &cr.ryO, &cr.ryD);
-    cr.r.tMax = INFINITY;
-    float sc = quake((float)spp);
-    cr.rxO = cr.r.o + (cr.rxO - cr.r.o) * sc;
-    cr.ryO = cr.r.o + (cr.ryO - cr.r.o) * sc;
-    cr.rxD = cr.r.d + (cr.rxD - cr.r.d) * sc;
-    cr.ryD = cr.r.d + (cr.ryD - cr.r.d) * sc;
-    return cr;
-}
-
-// Camera rays of one (pixel, sample): film sample from dims 0-1, lens sample from dims 2-3.
-LTS_D CamRays camera_sample(const SceneView& sv, int px, int py, int sample, int spp, int stratified, uint32_t seed) {
+// Film position and lens sample of one (pixel, sample): dims 0-1 and 2-3. A pinhole (lens radius 0,
+// the only camera the scene files describe) has no use for the lens sample.
+struct CameraSample {
+    V2 film, lens;
+};
+LTS_D CameraSample camera_sample(const SceneView& sv, int px, int py, int sample, int spp, int stratified, uint32_t seed) {
     Sampler smp;
     smp.seed = seed;
     smp.pixel = (uint32_t)(py * sv.cam.width + px);
     smp.sample = (uint32_t)sample;
     float d[4];
     smp.block(0, d);
-    V2 pFilm = film_sample(px, py, sample, spp, stratified, d);
-    V2 lens = uniform_disk(v2(d[2], d[3]));
-    return camera_rays(sv.cam, pFilm, lens, spp);
+    CameraSample cs;
+    cs.film = film_sample(px, py, sample, spp, stratified, d);
+    cs.lens = v2(0, 0);
+    if (sv.cam.lensRadius != 0) cs.lens = uniform_disk(v2(d[2], d[3]));
+    return cs;
+}
+LTS_D Ray camera_ray(const SceneView& sv, const CameraSample& cs) {
+    Ray r;
+    camera_ray(sv.cam, cs.film, cs.lens, &r.o, &r.d);
+    r.tMax = INFINITY;
+    return r;
+}
+
+// generateDifferentialRay + Ray::scaleDifferentials(rsqrt(spp)) (Camera.cu:67-81, Ray.cuh:35-40): the
+// differential rays of the camera ray (o, d) of a sample.
+LTS_D CamRays camera_differentials(const CameraDesc& c, const CameraSample& cs, int spp, V3 o, V3 d) {
+    CamRays cr;
+    camera_ray(c, cs.film + v2(1, 0), cs.lens, &cr.rxO, &cr.rxD);
+    camera_ray(c, cs.film + v2(0, 1), cs.lens, &cr.ryO, &cr.ryD);
+    float sc = quake((float)spp);
+    cr.rxO = o + (cr.rxO - o) * sc;
+    cr.ryO = o + (cr.ryO - o) * sc;
+    cr.rxD = d + (cr.rxD - d) * sc;
+    cr.ryD = d + (cr.ryD - d) * sc;
+    return cr;
 }
 
 // invDet * determinant of a hit: Triangle::intersect scales dpdu and dpdv by the ray's invDet where
@@ -1082,6 +1129,13 @@ LTS_D void differentials(SurfacePoint& s, const CamRays& cr, float k) {
     solve(c(px, d0) - c(s.p, d0), c(px, d1) - c(s.p, d1), s.dudx, s.dvdx);
     solve(c(py, d0) - c(s.p, d0), c(py, d1) - c(s.p, d1), s.dudy, s.dvdy);
     s.dudx *= k; s.dvdx *= k; s.dudy *= k; s.dvdy *= k;
+}
+
+// The footprint of a camera hit, for the materials whose textures read it (procedural and filtered
+// image textures).
+LTS_D void camera_footprint(const SceneView& sv, SurfacePoint& si, const CameraSample& cs, int spp, const Ray& r, float invDet) {
+    if (sv.mats[sv.shade[si.leaf].mat].footprint)
+        differentials(si, camera_differentials(sv.cam, cs, spp, r.o, r.d), uv_derivative_scale(sv, si.leaf, invDet));
 }
 
 }  // namespace lts

@@ -15,13 +15,13 @@ constexpr int kTileSide = 16;
 
 // One camera sample of PathTracingIntegrator::evaluate.
 LTS_D Spec radiance(const SceneView& sv, int px, int py, int sample, const RenderLaunch& rl, unsigned long long* cnt,
-                     TraceStack ts, const int* perm) {
+                     TraceStack ts, const NoiseTables& perm) {
     Sampler smp;
     smp.seed = rl.seed;
     smp.pixel = (uint32_t)(py * sv.cam.width + px);
     smp.sample = (uint32_t)sample;
-    CamRays cr = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
-    Ray r = cr.r;
+    const CameraSample cs = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
+    Ray r = camera_ray(sv, cs);
     Spec L = spec(0.0f), beta = spec(1.0f);
     bool specularBounce = false;
     for (int bounce = 0; bounce < rl.maxBounce; bounce++) {
@@ -43,7 +43,7 @@ LTS_D Spec radiance(const SceneView& sv, int px, int py, int sample, const Rende
         }
         if (h.leaf < 0) break;
         SurfacePoint si = make_surface(sv, h.leaf, r, h.u, h.v, h.invDet);
-        if (bounce == 0) differentials(si, cr, uv_derivative_scale(sv, h.leaf, h.invDet));
+        if (bounce == 0) camera_footprint(sv, si, cs, rl.spp, r, h.invDet);
         Bsdf bsdf = make_bsdf(sv, si, perm);
         float u0[4], u1[4];
         smp.block(1 + 2 * bounce, u0);
@@ -86,8 +86,8 @@ __global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tri
 // waves its natural register count allows.
 __global__ __launch_bounds__(256, 5) void k_megakernel(SceneView sv, RenderLaunch rl) {
     __shared__ int stk[kShortStack * 256];
-    __shared__ int perm[512];  // the procedural textures' permutation lookups chain three deep
-    for (int i = threadIdx.x; i < 512; i += 256) perm[i] = sv.perm[i];
+    __shared__ NoiseTables perm;
+    noise_tables(perm, sv.perm, threadIdx.x, 256);
     __syncthreads();
     const int W = sv.cam.width, H = sv.cam.height;
     const int tilesX = (W + kTileSide - 1) / kTileSide;

@@ -378,6 +378,7 @@ bool load_scene_files(const MeshTransformFn& transform, const std::string& dir, 
                     default: err = std::string("unsupported texture type '") + tt + "'"; return false;
                 }
                 if (td.type == TEX_IMAGE && (td.img < 0 || td.img >= (int)S.mips.size())) { err = "image index out of range"; return false; }
+                if (td.type != TEX_CONST && (td.type != TEX_IMAGE || filteredTextures)) md.footprint = 1;
                 (t == 0 ? md.tex0 : md.tex1) = (int)S.texs.size();
                 S.texs.push_back(td);
             }

@@ -83,13 +83,13 @@ __global__ __launch_bounds__(256) void k_wf_generate(const SceneView* __restrict
         const SceneView& sv = scenes[sc];
         const WfSceneSlot& sl = slots[sc];
         const int px = pixel % sv.cam.width, py = pixel / sv.cam.width;
-        CamRays cr = camera_sample(sv, px, py, sample, sl.spp, sl.stratified, sl.seed);
+        const Ray cr = camera_ray(sv, camera_sample(sv, px, py, sample, sl.spp, sl.stratified, sl.seed));
         const int ts = train_slot(P, sl, sc, pixel, sample);
         if (ts >= 0)
             for (int b = 0; b < P.maxBounce; b++) tRec[(size_t)ts * kWfMaxBounce + b].valid = 0;
         WfRay r;
-        r.o[0] = cr.r.o.x; r.o[1] = cr.r.o.y; r.o[2] = cr.r.o.z;
-        r.d[0] = cr.r.d.x; r.d[1] = cr.r.d.y; r.d[2] = cr.r.d.z;
+        r.o[0] = cr.o.x; r.o[1] = cr.o.y; r.o[2] = cr.o.z;
+        r.d[0] = cr.d.x; r.d[1] = cr.d.y; r.d[2] = cr.d.z;
         r.scene = sc; r.pad = 0;
         rays[k] = r;
         queue[k] = (int)k;
@@ -202,15 +202,13 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
     const int n = *count;
     const int maxBounce = prm->maxBounce, rrStart = prm->rrStart, queryBounce = prm->queryBounce;
     constexpr bool cached = kCached;
-    // the procedural textures' permutation lookups chain three deep: served from LDS (every scene
-    // view points at its context's one table)
-    __shared__ int perm[512];
+    __shared__ NoiseTables perm;  // every scene view points at its context's one permutation
     __shared__ int32_t appendLds[2][5 * (kShadeBlock / 64) + 5];
     // a query's raw record (4 float4) and its NrcQuery (3 float4), held by the thread that makes it
     // until the round's append gives the query its compact slot
     constexpr int kStage = 7;
     __shared__ float4 qStage[kCached ? kShadeBlock * kStage : 1];
-    for (int i = threadIdx.x; i < 512; i += kShadeBlock) perm[i] = scenes[0].perm[i];
+    noise_tables(perm, scenes[0].perm, threadIdx.x, kShadeBlock);
     __syncthreads();
     const int stride = gridDim.x * kShadeBlock;
     const int rounds = (n + stride - 1) / stride;  // uniform trip count: the appends below are wave-collective
@@ -245,13 +243,13 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
             const WfSceneSlot& sl = slots[scene];
             const int trainSlot = cached ? train_slot(P, sl, scene, pixel, sample) : -1;
             Ray r;
-            CamRays cam;
+            CameraSample cam;
             if (kFirst) {
-                // the camera ray and its differentials, drawn again as the generate kernel drew
-                // them (a path that escapes needs neither)
+                // the camera ray, drawn again as the generate kernel drew it (a path that escapes has no
+                // need of it)
                 if (hh.leaf >= 0) {
                     cam = camera_sample(sv, pixel % sv.cam.width, pixel / sv.cam.width, sample, sl.spp, sl.stratified, sl.seed);
-                    r = cam.r;
+                    r = camera_ray(sv, cam);
                 }
             } else {
                 const WfRay rr = rays[pi];
@@ -293,7 +291,7 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                 alive = false;
             } else {
                 SurfacePoint si = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
-                if (kFirst) differentials(si, cam, uv_derivative_scale(sv, hh.leaf, hh.invDet));
+                if (kFirst) camera_footprint(sv, si, cam, sl.spp, r, hh.invDet);
                 Bsdf bsdf = make_bsdf(sv, si, perm);
                 const int slot = (sample - sl.s0) * sl.width * sl.height + pixel;  // sample index of the path
                 if (cached && (bsdf.kind == 0 || bsdf.kind == 1 || bsdf.kind == 4)) {
@@ -360,26 +358,18 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                     Spec f2 = bsdf.sampleF(si.wo, &wi, v2(u0[3], u1[0]), &scatteringPdf, flags, &sampledType);
                     f2 = f2 * absDot(wi, si.sn);
                     const bool sampledSpecular = (sampledType & B_SPEC) != 0;
-                    if (!isBlack(f2) && scatteringPdf > 0) {
-                        float weight = 1;
-                        bool cast = true;
-                        if (!sampledSpecular) {
-                            lightPdf = Lt.kind == 0 ? tri_pdf(sv, Lt, si, wi) : inf_pdf(wi);
-                            if (lightPdf == 0) cast = false;
-                            else weight = power_heuristic(scatteringPdf, lightPdf);
-                        }
-                        const Spec Li2 = light_le(Lt);
-                        if (cast && !isBlack(Li2)) {
-                            const Ray mr = spawn_ray(si, wi);
-                            if (mis_target(sv, Lt, li, mr, sh.tMax, sh.tieLeaf)) {
-                                const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
-                                sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
-                                sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
-                                sh.scene = scene;
-                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
-                                wantMis = true;
-                                misRays[pi] = sh;
-                            }
+                    const Spec Li2 = light_le(Lt);
+                    if (!isBlack(f2) && scatteringPdf > 0 && !isBlack(Li2)) {
+                        const Ray mr = spawn_ray(si, wi);
+                        float weight;
+                        if (mis_ray(sv, Lt, li, si, mr, sampledSpecular, scatteringPdf, weight, sh.tMax, sh.tieLeaf)) {
+                            const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
+                            sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
+                            sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
+                            sh.scene = scene;
+                            sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
+                            wantMis = true;
+                            misRays[pi] = sh;
                         }
                     }
                 }

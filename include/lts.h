@@ -72,7 +72,7 @@ typedef struct lts_render_params {
     /* wavefront only (0 / -1 = default or the autotuned value) */
     int32_t trace_block;        /* block size of the persistent traversal kernels: 64, 128, 256 */
     int32_t persistent_blocks;  /* grid of the persistent traversal kernels                     */
-    int32_t sort_materials;     /* -1 default (on), 0 off, 1 counting-sort shading by material  */
+    int32_t sort_materials;     /* -1 default (on), 0 off, 1 shade in material order            */
     int32_t use_graph;          /* -1 default (on), 0 off: capture each pass in a hipGraph       */
     int32_t autotune;           /* 1: time candidate tunings on this scene before rendering:    */
                                 /*    trace block, persistent grid, material sort, tile rows and */
@@ -114,11 +114,11 @@ int lts_film_resolve(lts_ctx* ctx, float* rgb_out);
 /* Wavefront phases timed when profile_phases is set (indices into lts_stats.phase_ms). */
 #define LTS_PHASE_EXTEND 0      /* all traversal: path rays with the shadow and MIS rays traced */
                                 /* in the same launches (one per bounce)                      */
-#define LTS_PHASE_SORT 1        /* material sort of the shading queue                        */
+#define LTS_PHASE_SORT 1        /* 0: shading orders its own chunks by material (SHADE)       */
 #define LTS_PHASE_SHADE 2
 #define LTS_PHASE_SHADOW 3      /* 0: shadow rays are traced with the path rays (EXTEND)      */
 #define LTS_PHASE_MIS 4         /* 0: MIS-BSDF rays are traced with the path rays (EXTEND)    */
-#define LTS_PHASE_FINALIZE 5
+#define LTS_PHASE_FINALIZE 5    /* the last bounce's (SHADE completes the earlier bounces')    */
 #define LTS_PHASE_CACHE_INFER 6 /* radiance-cache inference (cached integrator)              */
 #define LTS_PHASE_CACHE_TRAIN 7 /* training-batch compaction and Adam steps                   */
 

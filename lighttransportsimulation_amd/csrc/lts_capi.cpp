@@ -672,11 +672,11 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
         if (prof && p->max_bounce > 0) {
             const int64_t perBounce = launches * p->max_bounce;
             st->phase_launches[LTS_PHASE_EXTEND] = perBounce + launches;
-            st->phase_launches[LTS_PHASE_SORT] = t.sortMaterials ? 2 * perBounce : 0;
+            st->phase_launches[LTS_PHASE_SORT] = 0;
             st->phase_launches[LTS_PHASE_SHADE] = perBounce;
             st->phase_launches[LTS_PHASE_SHADOW] = 0;
             st->phase_launches[LTS_PHASE_MIS] = 0;
-            st->phase_launches[LTS_PHASE_FINALIZE] = perBounce;
+            st->phase_launches[LTS_PHASE_FINALIZE] = launches;
             st->phase_launches[LTS_PHASE_CACHE_INFER] = cached ? launches : 0;
             st->phase_launches[LTS_PHASE_CACHE_TRAIN] = cached ? launches * c->nrc.steps : 0;
         }

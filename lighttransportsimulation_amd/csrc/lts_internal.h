@@ -128,9 +128,10 @@ hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t str
 // ---------------------------------------------------------------- wavefront tracer (wavefront.hip)
 constexpr int kWfAlive = 1, kWfSpecular = 2;
 // per bounce b: [0] path queue, [1] shadow rays, [2] MIS rays, [3] ended paths awaiting their
-// light sample; the 8 work counters of the trace
+// light sample; the work counter of its shading at kWfShadeWork; the 8 work counters of the trace
 // launch of bounce b's path rays at kWfWorkBase + kWfWorkStride * j (one 64-byte line each)
 constexpr int kWfCountsPerBounce = 160;
+constexpr int kWfShadeWork = 16;
 constexpr int kWfWorkBase = 32, kWfWorkStride = 16, kWfWorkSegments = 8;
 static_assert(kWfWorkBase + kWfWorkStride * kWfWorkSegments <= kWfCountsPerBounce, "work counters of a bounce");
 constexpr int kWfMaxMatBins = 64;
@@ -179,7 +180,7 @@ struct WfTuning {
     int traceBlock = 256;         // block size of the persistent traversal kernels (64, 128, 256)
     int persistentBlocks = 2048;  // grid of the traversal kernels
     int sweepBlocks = 2048;       // grid of the generate / shade / finalize sweeps
-    int sortMaterials = 1;        // counting-sort the shade queue by material
+    int sortMaterials = 1;        // shade in material order within chunks of the queue
     int useGraph = 1;             // capture the pass in a hipGraph and replay it
     int tileRows = 8;             // band height of the path order (a wave of 64 paths covers tileRows x 64/tileRows pixels)
     int passSpp = 0;              // samples per pass chosen by the autotuner (0: the automatic pass)
@@ -202,11 +203,10 @@ struct WfBuffers {
     WfHit* hits = nullptr;
     WfNee* nee = nullptr;
     int32_t* queue[2] = {nullptr, nullptr};
-    int32_t* sorted = nullptr;
-    int32_t* done = nullptr;      // paths that ended with a light sample still in flight
+    int32_t* done[2] = {nullptr, nullptr};  // paths that ended at a bounce with a light sample still in flight
     int32_t* shadowQ = nullptr;   // paths with a shadow ray (their records sit at the path index)
     int32_t* misQ = nullptr;      // paths with an MIS-BSDF ray (likewise)
-    int32_t* bins = nullptr;      // material bin of each path's hit, written by the extend kernel
+    uint8_t* bins = nullptr;      // material bin of each path's hit, written by the trace kernel
     WfLightRay* shadows = nullptr;  // per path
     WfLightRay* mis = nullptr;      // per path
     int32_t* counts = nullptr;
@@ -221,15 +221,14 @@ struct WfBuffers {
     float* sampleBase = nullptr;  // sample buffer of the pass (path i's radiance at 3 i)
 };
 
-// counts: per bounce kWfCountsPerBounce counters, then per-bounce material histograms, then the
-// pass-wide counters below.
-constexpr int kWfGlobalBase = (kWfCountsPerBounce + kWfMaxMatBins) * (kWfMaxBounce + 1);
-constexpr int kWfGlobalCounts = 8;  // [0] cache queries
+// counts: the pass-wide counters, then per bounce kWfCountsPerBounce counters.
+constexpr int kWfGlobalBase = 0;   // [0] cache queries
+constexpr int kWfBounceBase = 32;
 
 // Optional phase timing: events recorded between the kernels of a pass launched directly (not
 // captured). ev[8 kWfMaxBounce + 3] precedes the pass's first trace; bounce b uses ev[8b + 0..4]:
-// before the sort, after the sort, after shading, after the trace of the next path rays with this
-// bounce's shadow and MIS rays, after finalize; the cached integrator's tail uses
+// two before shading, after shading, after the trace of the next path rays with this bounce's shadow
+// and MIS rays, after the last bounce's finalize; the cached integrator's tail uses
 // ev[8 kWfMaxBounce + 0..2]: before inference, after inference, after the training steps.
 constexpr int kWfPhaseEvents = 8 * kWfMaxBounce + 4;
 struct WfProfile { hipEvent_t ev[kWfPhaseEvents]; };
@@ -240,7 +239,7 @@ constexpr int kTraceCounters = 6;
 hipError_t wf_reserve(WfBuffers& b, size_t cap, int maxScenes);
 hipError_t wf_reserve_cache(WfBuffers& b, size_t cap, int trainCap);
 void wf_release(WfBuffers& b);
-// Enqueues one pass: generate, then per bounce extend / (sort) / shade / shadow / mis / finalize.
+// Enqueues one pass: generate, trace, then per bounce shade and trace, then the last bounce's finalize.
 // With nrc (cached integrator): queries, training records, then cache inference into the sample
 // buffer, the training batch of path-suffix radiance and one Adam step.
 // traceCounts (6 counters, or null): launches the counting instantiation of the traversal kernel,

@@ -3,8 +3,7 @@
 // The reference integrator (intergrators/PathTracingIntegrator.cuh:38-104 with estimateDirect,
 // IntegratorHelper.cuh:51-125) is cut at its three ray casts:
 //   extend   closest hit of every live path ray                     (persistent)
-//   sort     optional counting sort of the hit queue by material
-//   shade    emission, BSDF, light sample + MIS-BSDF sample (NEE set-up), continuation, roulette;
+//   shade    (by default in material order within chunks of the queue) emission, BSDF, light sample + MIS-BSDF sample (NEE set-up), continuation, roulette;
 //            appends one shadow ray and one MIS ray per path at most
 //   shadow   any hit of the shadow rays                             (persistent, in extend's launch)
 //   mis      whether an MIS-BSDF ray reaches its light              (persistent, in extend's launch)
@@ -72,11 +71,10 @@ LTS_D int train_slot(const WfParams& P, const WfSceneSlot& sl, int scene, int pi
 // follows from the path index, and the first shading builds them.
 __global__ __launch_bounds__(256) void k_wf_generate(const SceneView* __restrict__ scenes, const WfParams* __restrict__ prm,
                                                      const WfSceneSlot* __restrict__ slots, WfRay* __restrict__ rays,
-                                                     int32_t* __restrict__ queue, int32_t* __restrict__ counts,
-                                                     WfTrainRec* __restrict__ tRec) {
+                                                     int32_t* __restrict__ counts, WfTrainRec* __restrict__ tRec) {
     const WfParams P = *prm;
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i == 0) counts[0] = (int)P.nPaths;  // bounce-0 queue holds every path of the pass
+    if (i == 0) counts[0] = (int)P.nPaths;  // bounce 0 has every path of the pass, in order (no queue)
     for (long k = i; k < P.nPaths; k += (long)gridDim.x * 256) {
         int sc, pixel, sample;
         path_origin(P, slots, k, sc, pixel, sample);
@@ -92,18 +90,6 @@ __global__ __launch_bounds__(256) void k_wf_generate(const SceneView* __restrict
         r.d[0] = cr.d.x; r.d[1] = cr.d.y; r.d[2] = cr.d.z;
         r.scene = sc; r.pad = 0;
         rays[k] = r;
-        queue[k] = (int)k;
-    }
-}
-
-// Counting sort of a queue by the material bin the extend kernel filed each hit under: one block
-// turns the histogram into bin offsets; each scatter block then takes one contiguous chunk of the
-// queue, counts its entries per bin, reserves its range of every bin with one atomic per bin and
-// writes the chunk's entries into those ranges, ranked within each wave by ballots.
-__global__ void k_wf_mat_scan(int32_t* __restrict__ hist, int nBins) {
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int b = 0; b < nBins; b++) { int c = hist[b]; hist[b] = run; run += c; }
     }
 }
 
@@ -125,34 +111,6 @@ LTS_D int wave_bin_rank(int bin, int32_t* h) {
         todo &= ~peers;
     }
     return slot;
-}
-
-__global__ __launch_bounds__(256) void k_wf_mat_scatter(const int32_t* __restrict__ bins, const int32_t* __restrict__ queue,
-                                                        const int32_t* __restrict__ count, int32_t* __restrict__ offs, int nBins,
-                                                        int32_t* __restrict__ sorted) {
-    __shared__ int32_t h[kWfMaxMatBins], base[kWfMaxMatBins];
-    const int n = *count;
-    const int per = ((n + (int)gridDim.x - 1) / (int)gridDim.x + 255) / 256 * 256;
-    const int begin = min((int)blockIdx.x * per, n), end = min(begin + per, n);
-    if (threadIdx.x < kWfMaxMatBins) h[threadIdx.x] = 0;
-    __syncthreads();
-    for (int k0 = begin; k0 < end; k0 += 256) {
-        const int k = k0 + threadIdx.x;
-        (void)wave_bin_rank(k < end ? bins[queue[k]] : -1, h);
-    }
-    __syncthreads();
-    if (threadIdx.x < nBins) {
-        base[threadIdx.x] = h[threadIdx.x] ? atomicAdd(&offs[threadIdx.x], h[threadIdx.x]) : 0;
-        h[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    for (int k0 = begin; k0 < end; k0 += 256) {
-        const int k = k0 + threadIdx.x;
-        const int pi = k < end ? queue[k] : -1;
-        const int bin = pi >= 0 ? bins[pi] : -1;
-        const int slot = wave_bin_rank(bin, h);
-        if (pi >= 0) sorted[base[bin] + slot] = pi;
-    }
 }
 
 LTS_D float clamp01(float x) { return fminf(fmaxf(x, 0.0f), 1.0f); }
@@ -181,16 +139,51 @@ LTS_D void nrc_raw_record(const SurfacePoint& si, const Bsdf& bsdf, const WfScen
     q[0] = r0; q[1] = r1; q[2] = r2; q[3] = r3;
 }
 
+// The traced light sample of a path that ended with one in flight completes its radiance (a continuing
+// path takes its sample at the start of the next bounce's shading).
+LTS_D void finalize_path(const WfParams& P, const WfSceneSlot* slots, const WfPath* paths, const WfNee* nee, int pi) {
+    const WfPath p = paths[pi];
+    const WfNee ne = nee[pi];
+    Spec L = spec(p.L[0], p.L[1], p.L[2]);
+    Spec Ld = spec(ne.p1[0], ne.p1[1], ne.p1[2]) + spec(ne.p2[0], ne.p2[1], ne.p2[2]);
+    L = L + spec(ne.nb[0], ne.nb[1], ne.nb[2]) * (Ld / ne.lpdf);
+    const WfSceneSlot& sl = slots[path_scene(P, slots, pi)];
+    const int sample = (int)(p.sampleFlags >> kWfFlagBits);
+    float* o = sl.sampleL + 3 * ((size_t)(sample - sl.s0) * sl.width * sl.height + p.pixel);
+    o[0] = L.r; o[1] = L.g; o[2] = L.b;
+}
+
 // One shading kernel per (integrator, first bounce or not), so that each carries only its own code
-// and registers: the radiance cache's records, and the camera-ray differentials of bounce 0. The
-// kernel waits on a chain of dependent gathers; at 3 waves per SIMD (168 VGPRs, a few dozen spilled)
-// it runs about 4 % faster than at the 2 its 209-233 registers would allow.
+// and registers: the radiance cache's records, and the camera-ray differentials of bounce 0. It first
+// completes the paths that ended at the previous bounce (prevDone).
+//
+// Material order. A block takes chunks of up to kSortChunk paths from the bounce's work counter and
+// orders each by the material bin the trace filed (bins; null: queue order) in LDS, so that most waves
+// shade one material. A chunk is 64-path pieces at equal strides over the queue: every chunk holds
+// about the pass's mix of materials and costs about the same (chunks of neighbouring paths are all
+// sky or all marble, and the last ones kept the launch waiting: 23.5 ms instead of 20.8 for the
+// shading of a 64-spp 1920x1080 frame of the 1M-triangle displaced sphere), and the waves of the
+// resident blocks work on neighbouring pieces. That frame with chunks of 256/512/1024/2048/4096
+// paths: 58.0/53.0/51.8/51.7/52.1 ms; a count, scan and scatter of the whole queue before the
+// shading: 54.5 ms. Small launches halve the chunk until every resident block has kChunksPerBlock
+// (a 256x256 4-spp frame: 2.38 ms with 1 chunk a block, 2.29 with 2, 2.26 with 4).
+constexpr int kSortChunk = 1024, kChunksPerBlock = 4;
+constexpr int kShadeGrid = 3 * 256;  // the workgroups resident at once: 3 of 4 waves on each of 256 CUs
+
+// queue position of item x of chunk c
+__device__ __forceinline__ int chunk_item(int x, int c, int chunks) { return ((x >> 6) * chunks + c) * 64 + (x & 63); }
+
+constexpr int kSortItemsPerThread = kSortChunk / kShadeBlock;
+
 template <bool kCached, bool kFirst>
 __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __restrict__ scenes, const WfParams* __restrict__ prm,
                                                           const WfSceneSlot* __restrict__ slots, int bounce,
                                                           WfPath* __restrict__ paths, WfRay* __restrict__ rays,
                                                           const WfHit* __restrict__ hits, WfNee* __restrict__ nee,
                                                           const int32_t* __restrict__ queue, const int32_t* __restrict__ count,
+                                                          const uint8_t* __restrict__ bins,
+                                                          const int32_t* __restrict__ prevDone, const int32_t* __restrict__ prevDoneCount,
+                                                          int32_t* __restrict__ work,
                                                           int32_t* __restrict__ nextQueue, int32_t* __restrict__ nextCount,
                                                           WfLightRay* __restrict__ shadows, int32_t* __restrict__ shadowCount,
                                                           WfLightRay* __restrict__ misRays, int32_t* __restrict__ misCount,
@@ -208,256 +201,302 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
     // until the round's append gives the query its compact slot
     constexpr int kStage = 7;
     __shared__ float4 qStage[kCached ? kShadeBlock * kStage : 1];
+    __shared__ int32_t nextChunk;
+    __shared__ int32_t order[kSortChunk], binCount[kWfMaxMatBins], binBase[kWfMaxMatBins];
     noise_tables(perm, scenes[0].perm, threadIdx.x, kShadeBlock);
+    if (!kFirst) {
+        const int nDone = *prevDoneCount;
+        const WfParams P = *prm;
+        for (int k = blockIdx.x * kShadeBlock + threadIdx.x; k < nDone; k += gridDim.x * kShadeBlock)
+            finalize_path(P, slots, paths, nee, prevDone[k]);
+    }
+    int per = kSortChunk;  // paths of a chunk
+    while (per > kShadeBlock && (long)per * gridDim.x * kChunksPerBlock > n) per >>= 1;
+    const int chunks = (n + per - 1) / per;
     __syncthreads();
-    const int stride = gridDim.x * kShadeBlock;
-    const int rounds = (n + stride - 1) / stride;  // uniform trip count: the appends below are wave-collective
-    // chunk of the block within a round: workgroups are dealt to the 8 XCDs round robin, so the
-    // blocks of one XCD take neighbouring chunks (neighbouring paths hit neighbouring geometry)
-    const int chunk = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
-    for (int round = 0; round < rounds; round++) {
-        const int k = round * stride + chunk * kShadeBlock + threadIdx.x;
-        const bool active = k < n;
-        const int pi = active ? queue[k] : 0;
-        bool wantShadow = false, wantMis = false, wantNext = false, wantQuery = false, wantDone = false;
-        WfLightRay sh;
-        if (active) {
-            const WfParams P = *prm;
-            WfPath p;
-            int scene, pixel, sample, pflags;
-            if (kFirst) {
-                // bounce 0: the path record follows from the path index
-                p.beta[0] = p.beta[1] = p.beta[2] = 1.0f;
-                p.L[0] = p.L[1] = p.L[2] = 0.0f;
-                path_origin(P, slots, pi, scene, pixel, sample);
-                pflags = kWfAlive;
-            } else {
-                p = paths[pi];
-                scene = path_scene(P, slots, pi);
-                pixel = p.pixel;
-                sample = (int)(p.sampleFlags >> kWfFlagBits);
-                pflags = (int)(p.sampleFlags & ((1u << kWfFlagBits) - 1));
+    int turn = 0;
+    while (true) {
+        if (threadIdx.x == 0) nextChunk = atomicAdd(work, 1);
+        __syncthreads();  // also: the previous chunk's order has been read
+        const int c = __builtin_amdgcn_readfirstlane(nextChunk);
+        if (c >= chunks) break;
+        int m = 0;
+        if (bins) {
+            // counting sort of the chunk: ranks within each bin, then the bins' starts
+            int pis[kSortItemsPerThread], slots_[kSortItemsPerThread], bin[kSortItemsPerThread];
+            if (threadIdx.x < kWfMaxMatBins) binCount[threadIdx.x] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kSortItemsPerThread; j++) {
+                const int x = j * kShadeBlock + threadIdx.x;
+                const int k = chunk_item(x, c, chunks);
+                pis[j] = x < per && k < n ? (kFirst ? k : queue[k]) : -1;
+                bin[j] = pis[j] >= 0 ? (int)bins[pis[j]] : -1;
+                slots_[j] = wave_bin_rank(bin[j], binCount);
             }
-            const WfHit hh = hits[pi];
-            const SceneView& sv = scenes[scene];
-            const WfSceneSlot& sl = slots[scene];
-            const int trainSlot = cached ? train_slot(P, sl, scene, pixel, sample) : -1;
-            Ray r;
-            CameraSample cam;
-            if (kFirst) {
-                // the camera ray, drawn again as the generate kernel drew it (a path that escapes has no
-                // need of it)
-                if (hh.leaf >= 0) {
-                    cam = camera_sample(sv, pixel % sv.cam.width, pixel / sv.cam.width, sample, sl.spp, sl.stratified, sl.seed);
-                    r = camera_ray(sv, cam);
+            __syncthreads();
+            if (threadIdx.x < kWfMaxMatBins) {
+                const int c = binCount[threadIdx.x];
+                int x = c;
+#pragma unroll
+                for (int o = 1; o < kWfMaxMatBins; o <<= 1) {
+                    const int y = __shfl_up(x, o);
+                    if ((int)threadIdx.x >= o) x += y;
                 }
-            } else {
-                const WfRay rr = rays[pi];
-                r.o = v3(rr.o[0], rr.o[1], rr.o[2]);
-                r.d = v3(rr.d[0], rr.d[1], rr.d[2]);
+                binBase[threadIdx.x] = x - c;
             }
-            r.tMax = INFINITY;
-            Spec L = spec(p.L[0], p.L[1], p.L[2]), beta = spec(p.beta[0], p.beta[1], p.beta[2]);
-            if (!kFirst) {
-                // the light sample of the previous vertex, traced since: added before anything of
-                // this vertex, as the reference's loop adds it before the next intersection
-                const WfNee pn = nee[pi];
-                if (pn.used) {
-                    Spec Ld = spec(pn.p1[0], pn.p1[1], pn.p1[2]) + spec(pn.p2[0], pn.p2[1], pn.p2[2]);
-                    L = L + spec(pn.nb[0], pn.nb[1], pn.nb[2]) * (Ld / pn.lpdf);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kSortItemsPerThread; j++)
+                if (pis[j] >= 0) order[binBase[bin[j]] + slots_[j]] = pis[j];
+            __syncthreads();
+            m = binBase[kWfMaxMatBins - 1] + binCount[kWfMaxMatBins - 1];
+        }
+        for (int sub = 0; sub < (bins ? m : per); sub += kShadeBlock, turn++) {
+            const int x = sub + threadIdx.x;
+            const int k = chunk_item(x, c, chunks);
+            const bool active = bins ? x < m : k < n;
+            const int pi = !active ? 0 : bins ? order[x] : kFirst ? k : queue[k];
+            bool wantShadow = false, wantMis = false, wantNext = false, wantQuery = false, wantDone = false;
+            WfLightRay sh;
+            if (active) {
+                const WfParams P = *prm;
+                WfPath p;
+                int scene, pixel, sample, pflags;
+                if (kFirst) {
+                    // bounce 0: the path record follows from the path index
+                    p.beta[0] = p.beta[1] = p.beta[2] = 1.0f;
+                    p.L[0] = p.L[1] = p.L[2] = 0.0f;
+                    path_origin(P, slots, pi, scene, pixel, sample);
+                    pflags = kWfAlive;
+                } else {
+                    p = paths[pi];
+                    scene = path_scene(P, slots, pi);
+                    pixel = p.pixel;
+                    sample = (int)(p.sampleFlags >> kWfFlagBits);
+                    pflags = (int)(p.sampleFlags & ((1u << kWfFlagBits) - 1));
                 }
-            }
-            const bool specularBounce = (pflags & kWfSpecular) != 0;
-            WfNee ne;
-            ne.used = 0;
-            ne.p1[0] = ne.p1[1] = ne.p1[2] = 0.0f;
-            ne.p2[0] = ne.p2[1] = ne.p2[2] = 0.0f;
-            bool alive = true;
-            if (kFirst || specularBounce) {
-                if (hh.leaf >= 0) {
-                    const int l = sv.shade[hh.leaf].light;
-                    if (l >= 0) {
-                        SurfacePoint e = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
-                        Spec le = dot(e.n, -r.d) > 0.f ? light_le(sv.lights[l]) : spec(0.0f);
-                        L = L + beta * le;
-                    } else {
-                        L = L + beta * spec(0.0f);
+                const WfHit hh = hits[pi];
+                const SceneView& sv = scenes[scene];
+                const WfSceneSlot& sl = slots[scene];
+                const int trainSlot = cached ? train_slot(P, sl, scene, pixel, sample) : -1;
+                Ray r;
+                CameraSample cam;
+                if (kFirst) {
+                    // the camera ray, drawn again as the generate kernel drew it (a path that escapes has no
+                    // need of it)
+                    if (hh.leaf >= 0) {
+                        cam = camera_sample(sv, pixel % sv.cam.width, pixel / sv.cam.width, sample, sl.spp, sl.stratified, sl.seed);
+                        r = camera_ray(sv, cam);
                     }
                 } else {
-                    for (int l = 0; l < sv.nLights; l++) L = L + beta * (sv.lights[l].kind == 1 ? light_le(sv.lights[l]) : spec(0.0f));
+                    const WfRay rr = rays[pi];
+                    r.o = v3(rr.o[0], rr.o[1], rr.o[2]);
+                    r.d = v3(rr.d[0], rr.d[1], rr.d[2]);
                 }
-            }
-            if (hh.leaf < 0) {
-                alive = false;
-            } else {
-                SurfacePoint si = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
-                if (kFirst) camera_footprint(sv, si, cam, sl.spp, r, hh.invDet);
-                Bsdf bsdf = make_bsdf(sv, si, perm);
-                const int slot = (sample - sl.s0) * sl.width * sl.height + pixel;  // sample index of the path
-                if (cached && (bsdf.kind == 0 || bsdf.kind == 1 || bsdf.kind == 4)) {
-                    if (trainSlot >= 0) {
-                        // training vertex: radiance so far and throughput, for the suffix target
-                        const size_t r = (size_t)trainSlot * kWfMaxBounce + bounce;
-                        nrc_raw_record(si, bsdf, sl, tRaw + 16 * r);
-                        WfTrainRec tr;
-                        tr.Lb[0] = L.r; tr.Lb[1] = L.g; tr.Lb[2] = L.b;
-                        tr.beta[0] = beta.r; tr.beta[1] = beta.g; tr.beta[2] = beta.b;
-                        tr.a[0] = bsdf.R.r; tr.a[1] = bsdf.R.g; tr.a[2] = bsdf.R.b;
-                        tr.slot = slot; tr.valid = 1; tr.pad = 0;
-                        tRec[r] = tr;
-                    } else if (bounce >= queryBounce) {
-                        // the cache stands for all radiance scattered here
-                        nrc_raw_record(si, bsdf, sl, reinterpret_cast<float*>(&qStage[kStage * threadIdx.x]));
-                        NrcQuery q;
-                        q.beta[0] = beta.r; q.beta[1] = beta.g; q.beta[2] = beta.b;
-                        q.a[0] = bsdf.R.r; q.a[1] = bsdf.R.g; q.a[2] = bsdf.R.b;
-                        q.L[0] = q.L[1] = q.L[2] = 0.0f;  // set where the path ends, below
-                        q.slot = slot; q.pad[0] = q.pad[1] = 0;
-                        *reinterpret_cast<NrcQuery*>(&qStage[kStage * threadIdx.x + 4]) = q;
-                        wantQuery = true;
-                        alive = false;
+                r.tMax = INFINITY;
+                Spec L = spec(p.L[0], p.L[1], p.L[2]), beta = spec(p.beta[0], p.beta[1], p.beta[2]);
+                if (!kFirst) {
+                    // the light sample of the previous vertex, traced since: added before anything of
+                    // this vertex, as the reference's loop adds it before the next intersection
+                    const WfNee pn = nee[pi];
+                    if (pn.used) {
+                        Spec Ld = spec(pn.p1[0], pn.p1[1], pn.p1[2]) + spec(pn.p2[0], pn.p2[1], pn.p2[2]);
+                        L = L + spec(pn.nb[0], pn.nb[1], pn.nb[2]) * (Ld / pn.lpdf);
                     }
                 }
-                Sampler smp;
-                smp.seed = sl.seed; smp.pixel = (uint32_t)pixel; smp.sample = (uint32_t)sample;
-                float u0[4], u1[4];
-                smp.block(1 + 2 * bounce, u0);
-                smp.block(2 + 2 * bounce, u1);
-                if (!wantQuery && sv.nLights > 0) {
-                    float lpdf;
-                    const int li = sample_light(sv, u0[0], &lpdf);
-                    const LightDesc& Lt = sv.lights[li];
-                    ne.used = 1;
-                    ne.nb[0] = beta.r; ne.nb[1] = beta.g; ne.nb[2] = beta.b;
-                    ne.lpdf = lpdf;
-                    const int flags = specularBounce ? B_ALL : (B_ALL & ~B_SPEC);
-                    // light sample with MIS (IntegratorHelper.cuh:76-95)
-                    V3 wi;
-                    float lightPdf = 0.0f, scatteringPdf = 0.0f;
-                    LightPoint vis;
-                    Spec Li = sample_li(sv, Lt, si, v2(u0[1], u0[2]), &wi, &lightPdf, &vis);
-                    if (lightPdf > 0 && !isBlack(Li)) {
-                        Spec f = bsdf.f(si.wo, wi, flags) * absDot(wi, si.sn);
-                        scatteringPdf = bsdf.pdf(si.wo, wi, flags);
-                        if (!isBlack(f)) {
-                            float weight = power_heuristic(lightPdf, scatteringPdf);
-                            Spec c = f * Li * weight / lightPdf;
-                            V3 origin = offsetRayOrigin(si.p, si.pError, si.n, vis.p - si.p);
-                            V3 target = offsetRayOrigin(vis.p, vis.pError, vis.n, origin - vis.p);
-                            V3 d = target - origin;
-                            sh.o[0] = origin.x; sh.o[1] = origin.y; sh.o[2] = origin.z;
-                            sh.d[0] = d.x; sh.d[1] = d.y; sh.d[2] = d.z;
-                            sh.scene = scene; sh.tieLeaf = -1; sh.tMax = 1 - SHADOW_EPS;
-                            sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
-                            wantShadow = true;
-                            shadows[pi] = sh;  // per path; the queue below lists the paths
+                const bool specularBounce = (pflags & kWfSpecular) != 0;
+                WfNee ne;
+                ne.used = 0;
+                ne.p1[0] = ne.p1[1] = ne.p1[2] = 0.0f;
+                ne.p2[0] = ne.p2[1] = ne.p2[2] = 0.0f;
+                bool alive = true;
+                if (kFirst || specularBounce) {
+                    if (hh.leaf >= 0) {
+                        const int l = sv.shade[hh.leaf].light;
+                        if (l >= 0) {
+                            SurfacePoint e = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
+                            Spec le = dot(e.n, -r.d) > 0.f ? light_le(sv.lights[l]) : spec(0.0f);
+                            L = L + beta * le;
+                        } else {
+                            L = L + beta * spec(0.0f);
                         }
-                    }
-                    // BSDF sample with MIS (IntegratorHelper.cuh:96-122)
-                    int sampledType = 0;
-                    Spec f2 = bsdf.sampleF(si.wo, &wi, v2(u0[3], u1[0]), &scatteringPdf, flags, &sampledType);
-                    f2 = f2 * absDot(wi, si.sn);
-                    const bool sampledSpecular = (sampledType & B_SPEC) != 0;
-                    const Spec Li2 = light_le(Lt);
-                    if (!isBlack(f2) && scatteringPdf > 0 && !isBlack(Li2)) {
-                        const Ray mr = spawn_ray(si, wi);
-                        float weight;
-                        if (mis_ray(sv, Lt, li, si, mr, sampledSpecular, scatteringPdf, weight, sh.tMax, sh.tieLeaf)) {
-                            const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
-                            sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
-                            sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
-                            sh.scene = scene;
-                            sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
-                            wantMis = true;
-                            misRays[pi] = sh;
-                        }
+                    } else {
+                        for (int l = 0; l < sv.nLights; l++) L = L + beta * (sv.lights[l].kind == 1 ? light_le(sv.lights[l]) : spec(0.0f));
                     }
                 }
-                // continuation (PathTracingIntegrator.cuh:79-103)
-                V3 wo = -r.d, wi;
-                float pdf;
-                int flags = 0;
-                Spec f = wantQuery ? spec(0.0f) : bsdf.sampleF(wo, &wi, v2(u1[1], u1[2]), &pdf, B_ALL, &flags);
-                if (wantQuery || isBlack(f) || pdf == 0) {
+                if (hh.leaf < 0) {
                     alive = false;
                 } else {
-                    pflags = (flags & B_SPEC) ? (pflags | kWfSpecular) : (pflags & ~kWfSpecular);
-                    beta = beta * (f * absDot(wi, si.sn) / pdf);
-                    Ray nr = spawn_ray(si, wi);
-                    WfRay o;
-                    o.o[0] = nr.o.x; o.o[1] = nr.o.y; o.o[2] = nr.o.z;
-                    o.d[0] = wi.x; o.d[1] = wi.y; o.d[2] = wi.z;
-                    o.scene = scene; o.pad = 0;
-                    rays[pi] = o;
-                    if (bounce >= rrStart) {
-                        float q = fmaxf(0.05f, 1 - lum(beta));
-                        if (u1[3] < q) alive = false;
-                        else beta = beta / (1 - q);
+                    SurfacePoint si = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
+                    if (kFirst) camera_footprint(sv, si, cam, sl.spp, r, hh.invDet);
+                    Bsdf bsdf = make_bsdf(sv, si, perm);
+                    const int slot = (sample - sl.s0) * sl.width * sl.height + pixel;  // sample index of the path
+                    if (cached && (bsdf.kind == 0 || bsdf.kind == 1 || bsdf.kind == 4)) {
+                        if (trainSlot >= 0) {
+                            // training vertex: radiance so far and throughput, for the suffix target
+                            const size_t r = (size_t)trainSlot * kWfMaxBounce + bounce;
+                            nrc_raw_record(si, bsdf, sl, tRaw + 16 * r);
+                            WfTrainRec tr;
+                            tr.Lb[0] = L.r; tr.Lb[1] = L.g; tr.Lb[2] = L.b;
+                            tr.beta[0] = beta.r; tr.beta[1] = beta.g; tr.beta[2] = beta.b;
+                            tr.a[0] = bsdf.R.r; tr.a[1] = bsdf.R.g; tr.a[2] = bsdf.R.b;
+                            tr.slot = slot; tr.valid = 1; tr.pad = 0;
+                            tRec[r] = tr;
+                        } else if (bounce >= queryBounce) {
+                            // the cache stands for all radiance scattered here
+                            nrc_raw_record(si, bsdf, sl, reinterpret_cast<float*>(&qStage[kStage * threadIdx.x]));
+                            NrcQuery q;
+                            q.beta[0] = beta.r; q.beta[1] = beta.g; q.beta[2] = beta.b;
+                            q.a[0] = bsdf.R.r; q.a[1] = bsdf.R.g; q.a[2] = bsdf.R.b;
+                            q.L[0] = q.L[1] = q.L[2] = 0.0f;  // set where the path ends, below
+                            q.slot = slot; q.pad[0] = q.pad[1] = 0;
+                            *reinterpret_cast<NrcQuery*>(&qStage[kStage * threadIdx.x + 4]) = q;
+                            wantQuery = true;
+                            alive = false;
+                        }
+                    }
+                    Sampler smp;
+                    smp.seed = sl.seed; smp.pixel = (uint32_t)pixel; smp.sample = (uint32_t)sample;
+                    float u0[4], u1[4];
+                    smp.block(1 + 2 * bounce, u0);
+                    smp.block(2 + 2 * bounce, u1);
+                    if (!wantQuery && sv.nLights > 0) {
+                        float lpdf;
+                        const int li = sample_light(sv, u0[0], &lpdf);
+                        const LightDesc& Lt = sv.lights[li];
+                        ne.used = 1;
+                        ne.nb[0] = beta.r; ne.nb[1] = beta.g; ne.nb[2] = beta.b;
+                        ne.lpdf = lpdf;
+                        const int flags = specularBounce ? B_ALL : (B_ALL & ~B_SPEC);
+                        // light sample with MIS (IntegratorHelper.cuh:76-95)
+                        V3 wi;
+                        float lightPdf = 0.0f, scatteringPdf = 0.0f;
+                        LightPoint vis;
+                        Spec Li = sample_li(sv, Lt, si, v2(u0[1], u0[2]), &wi, &lightPdf, &vis);
+                        if (lightPdf > 0 && !isBlack(Li)) {
+                            Spec f = bsdf.f(si.wo, wi, flags) * absDot(wi, si.sn);
+                            scatteringPdf = bsdf.pdf(si.wo, wi, flags);
+                            if (!isBlack(f)) {
+                                float weight = power_heuristic(lightPdf, scatteringPdf);
+                                Spec c = f * Li * weight / lightPdf;
+                                V3 origin = offsetRayOrigin(si.p, si.pError, si.n, vis.p - si.p);
+                                V3 target = offsetRayOrigin(vis.p, vis.pError, vis.n, origin - vis.p);
+                                V3 d = target - origin;
+                                sh.o[0] = origin.x; sh.o[1] = origin.y; sh.o[2] = origin.z;
+                                sh.d[0] = d.x; sh.d[1] = d.y; sh.d[2] = d.z;
+                                sh.scene = scene; sh.tieLeaf = -1; sh.tMax = 1 - SHADOW_EPS;
+                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
+                                wantShadow = true;
+                                shadows[pi] = sh;  // per path; the queue below lists the paths
+                            }
+                        }
+                        // BSDF sample with MIS (IntegratorHelper.cuh:96-122)
+                        int sampledType = 0;
+                        Spec f2 = bsdf.sampleF(si.wo, &wi, v2(u0[3], u1[0]), &scatteringPdf, flags, &sampledType);
+                        f2 = f2 * absDot(wi, si.sn);
+                        const bool sampledSpecular = (sampledType & B_SPEC) != 0;
+                        const Spec Li2 = light_le(Lt);
+                        if (!isBlack(f2) && scatteringPdf > 0 && !isBlack(Li2)) {
+                            const Ray mr = spawn_ray(si, wi);
+                            float weight;
+                            if (mis_ray(sv, Lt, li, si, mr, sampledSpecular, scatteringPdf, weight, sh.tMax, sh.tieLeaf)) {
+                                const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
+                                sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
+                                sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
+                                sh.scene = scene;
+                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
+                                wantMis = true;
+                                misRays[pi] = sh;
+                            }
+                        }
+                    }
+                    // continuation (PathTracingIntegrator.cuh:79-103)
+                    V3 wo = -r.d, wi;
+                    float pdf;
+                    int flags = 0;
+                    Spec f = wantQuery ? spec(0.0f) : bsdf.sampleF(wo, &wi, v2(u1[1], u1[2]), &pdf, B_ALL, &flags);
+                    if (wantQuery || isBlack(f) || pdf == 0) {
+                        alive = false;
+                    } else {
+                        pflags = (flags & B_SPEC) ? (pflags | kWfSpecular) : (pflags & ~kWfSpecular);
+                        beta = beta * (f * absDot(wi, si.sn) / pdf);
+                        Ray nr = spawn_ray(si, wi);
+                        WfRay o;
+                        o.o[0] = nr.o.x; o.o[1] = nr.o.y; o.o[2] = nr.o.z;
+                        o.d[0] = wi.x; o.d[1] = wi.y; o.d[2] = wi.z;
+                        o.scene = scene; o.pad = 0;
+                        rays[pi] = o;
+                        if (bounce >= rrStart) {
+                            float q = fmaxf(0.05f, 1 - lum(beta));
+                            if (u1[3] < q) alive = false;
+                            else beta = beta / (1 - q);
+                        }
+                    }
+                }
+                p.L[0] = L.r; p.L[1] = L.g; p.L[2] = L.b;
+                p.beta[0] = beta.r; p.beta[1] = beta.g; p.beta[2] = beta.b;
+                if (!alive) pflags &= ~kWfAlive;
+                p.pixel = pixel;
+                p.sampleFlags = ((uint32_t)sample << kWfFlagBits) | (uint32_t)pflags;
+                wantNext = alive && bounce + 1 < maxBounce;
+                // the records are read again only by the next shading or by finalize
+                if (wantNext || ne.used) {
+                    paths[pi] = p;
+                    nee[pi] = ne;
+                }
+                if (!wantNext) {
+                    // the path ends here: its sample is final now, or once its light sample is traced
+                    if (ne.used) {
+                        wantDone = true;
+                    } else if (cached && wantQuery) {
+                        // the sample is written by inference: L plus the cache's estimate
+                        NrcQuery* q = reinterpret_cast<NrcQuery*>(&qStage[kStage * threadIdx.x + 4]);
+                        q->L[0] = L.r; q->L[1] = L.g; q->L[2] = L.b;
+                    } else {
+                        float* o = sl.sampleL + 3 * ((size_t)(sample - sl.s0) * sl.width * sl.height + pixel);
+                        o[0] = L.r; o[1] = L.g; o[2] = L.b;
                     }
                 }
             }
-            p.L[0] = L.r; p.L[1] = L.g; p.L[2] = L.b;
-            p.beta[0] = beta.r; p.beta[1] = beta.g; p.beta[2] = beta.b;
-            if (!alive) pflags &= ~kWfAlive;
-            p.pixel = pixel;
-            p.sampleFlags = ((uint32_t)sample << kWfFlagBits) | (uint32_t)pflags;
-            wantNext = alive && bounce + 1 < maxBounce;
-            // the records are read again only by the next shading or by finalize
-            if (wantNext || ne.used) {
-                paths[pi] = p;
-                nee[pi] = ne;
+            // The round's appends, aggregated per block: each wave files its counts in LDS, one lane per
+            // queue reserves the block's range with a single device atomic (one per wave on a handful of
+            // shared counters serialised), and every lane writes at its offset. The buffers alternate
+            // between rounds so that one barrier pair per round suffices.
+            constexpr int kQueues = 5, kWaves = kShadeBlock / 64;
+            const bool want[kQueues] = {wantShadow, wantMis, wantNext, wantDone, cached && wantQuery};
+            int32_t* const counter[kQueues] = {shadowCount, misCount, nextCount, doneCount, qCount};
+            int32_t* const lds = appendLds[turn & 1];
+            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
+            uint64_t mask[kQueues];
+#pragma unroll
+            for (int q = 0; q < kQueues; q++) {
+                mask[q] = __ballot(want[q]);
+                if (lane == 0) lds[q * kWaves + wave] = (int)__popcll(mask[q]);
             }
-            if (!wantNext) {
-                // the path ends here: its sample is final now, or once its light sample is traced
-                if (ne.used) {
-                    wantDone = true;
-                } else if (cached && wantQuery) {
-                    // the sample is written by inference: L plus the cache's estimate
-                    NrcQuery* q = reinterpret_cast<NrcQuery*>(&qStage[kStage * threadIdx.x + 4]);
-                    q->L[0] = L.r; q->L[1] = L.g; q->L[2] = L.b;
-                } else {
-                    float* o = sl.sampleL + 3 * ((size_t)(sample - sl.s0) * sl.width * sl.height + pixel);
-                    o[0] = L.r; o[1] = L.g; o[2] = L.b;
-                }
+            __syncthreads();
+            if (threadIdx.x < kQueues && (threadIdx.x < 4 || cached)) {
+                const int q = threadIdx.x;
+                int run = 0;
+                for (int w = 0; w < kWaves; w++) { const int c = lds[q * kWaves + w]; lds[q * kWaves + w] = run; run += c; }
+                lds[kQueues * kWaves + q] = run ? atomicAdd(counter[q], run) : 0;
             }
-        }
-        // The round's appends, aggregated per block: each wave files its counts in LDS, one lane per
-        // queue reserves the block's range with a single device atomic (one per wave on a handful of
-        // shared counters serialised), and every lane writes at its offset. The buffers alternate
-        // between rounds so that one barrier pair per round suffices.
-        constexpr int kQueues = 5, kWaves = kShadeBlock / 64;
-        const bool want[kQueues] = {wantShadow, wantMis, wantNext, wantDone, cached && wantQuery};
-        int32_t* const counter[kQueues] = {shadowCount, misCount, nextCount, doneCount, qCount};
-        int32_t* const lds = appendLds[round & 1];
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
-        uint64_t mask[kQueues];
+            __syncthreads();
+            int32_t* const out[kQueues - 1] = {shadowQueue, misQueue, nextQueue, doneQueue};
 #pragma unroll
-        for (int q = 0; q < kQueues; q++) {
-            mask[q] = __ballot(want[q]);
-            if (lane == 0) lds[q * kWaves + wave] = (int)__popcll(mask[q]);
-        }
-        __syncthreads();
-        if (threadIdx.x < kQueues && (threadIdx.x < 4 || cached)) {
-            const int q = threadIdx.x;
-            int run = 0;
-            for (int w = 0; w < kWaves; w++) { const int c = lds[q * kWaves + w]; lds[q * kWaves + w] = run; run += c; }
-            lds[kQueues * kWaves + q] = run ? atomicAdd(counter[q], run) : 0;
-        }
-        __syncthreads();
-        int32_t* const out[kQueues - 1] = {shadowQueue, misQueue, nextQueue, doneQueue};
+            for (int q = 0; q < kQueues - 1; q++)
+                if (want[q]) out[q][lds[kQueues * kWaves + q] + lds[q * kWaves + wave] + (int)__popcll(mask[q] & below)] = pi;
+            if (cached && want[4]) {
+                // queries are stored compactly in append order, so inference reads them in sequence
+                const size_t at = (size_t)(lds[kQueues * kWaves + 4] + lds[4 * kWaves + wave] + (int)__popcll(mask[4] & below));
+                float4* r = reinterpret_cast<float4*>(qRaw + 16 * at);
 #pragma unroll
-        for (int q = 0; q < kQueues - 1; q++)
-            if (want[q]) out[q][lds[kQueues * kWaves + q] + lds[q * kWaves + wave] + (int)__popcll(mask[q] & below)] = pi;
-        if (cached && want[4]) {
-            // queries are stored compactly in append order, so inference reads them in sequence
-            const size_t at = (size_t)(lds[kQueues * kWaves + 4] + lds[4 * kWaves + wave] + (int)__popcll(mask[4] & below));
-            float4* r = reinterpret_cast<float4*>(qRaw + 16 * at);
+                for (int j = 0; j < 4; j++) r[j] = qStage[kStage * threadIdx.x + j];
+                float4* m = reinterpret_cast<float4*>(qMeta + at);
 #pragma unroll
-            for (int j = 0; j < 4; j++) r[j] = qStage[kStage * threadIdx.x + j];
-            float4* m = reinterpret_cast<float4*>(qMeta + at);
-#pragma unroll
-            for (int j = 0; j < 3; j++) m[j] = qStage[kStage * threadIdx.x + 4 + j];
+                for (int j = 0; j < 3; j++) m[j] = qStage[kStage * threadIdx.x + 4 + j];
+            }
         }
     }
 }
@@ -561,20 +600,13 @@ constexpr int kMinWidth = 4;
 template <int BS, bool kCount>
 __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict__ scenes, const WfRay* __restrict__ rays, WfHit* __restrict__ hits,
                                                  const int32_t* __restrict__ ext, const int32_t* __restrict__ extCount,
-                                                 int32_t* __restrict__ bins, int32_t* __restrict__ hist, int nBins,
-                                                 const WfLightRay* __restrict__ shadows, const int32_t* __restrict__ shadowCount,
+                                                 uint8_t* __restrict__ bins, int nBins, const WfLightRay* __restrict__ shadows, const int32_t* __restrict__ shadowCount,
                                                  const WfLightRay* __restrict__ misRays, const int32_t* __restrict__ misCount,
                                                  const int32_t* __restrict__ shadowQueue, const int32_t* __restrict__ misQueue,
                                                  WfNee* __restrict__ nee, int32_t* __restrict__ work,
                                                  unsigned long long* __restrict__ traceCounts) {
     __shared__ int stk[kShortStack * BS];
-    __shared__ int32_t lh[kWfMaxMatBins];
     const TraceStack ts = lds_stack(stk, threadIdx.x, BS);
-    const bool filing = hist != nullptr;
-    if (filing) {
-        for (int b = threadIdx.x; b < kWfMaxMatBins; b += BS) lh[b] = 0;
-        __syncthreads();
-    }
     const int nE = extCount ? *extCount : 0;
     const int nS = shadowCount ? *shadowCount : 0;
     const int nM = misCount ? *misCount : 0;
@@ -607,12 +639,8 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
                     WfHit o;
                     o.leaf = best; o.u = hu; o.v = hv; o.invDet = hInvDet;
                     hits[path] = o;
-                    if (filing) {
-                        // the hit is also filed under its material bin (misses in the last) for the counting sort
-                        const int bin = best < 0 ? nBins - 1 : min(mat, nBins - 2);
-                        bins[path] = bin;
-                        atomicAdd(&lh[bin], 1);
-                    }
+                    // the hit is also filed under its material bin (misses in the last) for shading
+                    if (bins) bins[path] = (uint8_t)(best < 0 ? nBins - 1 : min(mat, nBins - 2));
                 } else if (mat == 0) {  // nothing blocked the light ray
                     const float4 c = reinterpret_cast<const float4*>((kind == 1 ? shadows : misRays) + path)[2];
                     float* p = kind == 1 ? nee[path].p1 : nee[path].p2;
@@ -648,7 +676,7 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
                 const float4* src;
                 if (k < nE) {
                     kind = 0;
-                    path = ext[k];
+                    path = ext ? ext[k] : k;  // bounce 0 has no queue
                     src = reinterpret_cast<const float4*>(rays + path);
                 } else if (k < nE + nS) {
                     kind = 1;
@@ -709,32 +737,15 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
     if constexpr (kCount) {
         for (int q = 0; q < 6; q++) atomicAdd(&traceCounts[q], tally[q]);
     }
-    if (filing) {
-        __syncthreads();
-        for (int b = threadIdx.x; b < nBins; b += BS)
-            if (lh[b]) atomicAdd(&hist[b], lh[b]);
-    }
 }
 
-// Paths that ended at this bounce with a light sample in flight: the traced sample completes their
-// radiance (a continuing path takes its sample at the start of the next bounce's shading).
+// Completes the paths that ended at the last bounce with a light sample in flight.
 __global__ __launch_bounds__(256) void k_wf_finalize(const WfParams* __restrict__ prm, const WfSceneSlot* __restrict__ slots,
                                                      const WfPath* __restrict__ paths, const WfNee* __restrict__ nee,
                                                      const int32_t* __restrict__ done, const int32_t* __restrict__ count) {
     const int n = *count;
     const WfParams P = *prm;
-    for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) {
-        const int pi = done[k];
-        const WfPath p = paths[pi];
-        const WfNee ne = nee[pi];
-        Spec L = spec(p.L[0], p.L[1], p.L[2]);
-        Spec Ld = spec(ne.p1[0], ne.p1[1], ne.p1[2]) + spec(ne.p2[0], ne.p2[1], ne.p2[2]);
-        L = L + spec(ne.nb[0], ne.nb[1], ne.nb[2]) * (Ld / ne.lpdf);
-        const WfSceneSlot& sl = slots[path_scene(P, slots, pi)];
-        const int sample = (int)(p.sampleFlags >> kWfFlagBits);
-        float* o = sl.sampleL + 3 * ((size_t)(sample - sl.s0) * sl.width * sl.height + p.pixel);
-        o[0] = L.r; o[1] = L.g; o[2] = L.b;
-    }
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) finalize_path(P, slots, paths, nee, done[k]);
 }
 
 // Passes with max_bounce == 0 produce black samples.
@@ -762,28 +773,25 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
         if (prof) (void)hipEventRecord(prof->ev[i], s);
     };
     const int gridAll = t.sweepBlocks;
-    const int ncounts = kWfCountsPerBounce * (maxBounce + 1) + kWfMaxMatBins * (maxBounce + 1);
+    const int ncounts = kWfBounceBase + kWfCountsPerBounce * (maxBounce + 1);
     k_wf_fill<<<(ncounts + 255) / 256, 256, 0, s>>>(b.counts, ncounts, 0);
-    k_wf_fill<<<1, 256, 0, s>>>(b.counts + kWfGlobalBase, kWfGlobalCounts, 0);
     if (maxBounce <= 0) {
         k_wf_zero<<<gridAll, 256, 0, s>>>(b.params, b.slots);
         return hipGetLastError();
     }
     const bool cached = nrc != nullptr;
     int32_t* qCount = b.counts + kWfGlobalBase;
-    k_wf_generate<<<gridAll, 256, 0, s>>>(b.scenes, b.params, b.slots, b.rays, b.queue[0], b.counts, b.tRec);
-    auto histOf = [&](int bounce) {
-        return t.sortMaterials ? b.counts + kWfCountsPerBounce * (maxBounce + 1) + kWfMaxMatBins * bounce : nullptr;
-    };
+    int32_t* const bounce0 = b.counts + kWfBounceBase;
+    k_wf_generate<<<gridAll, 256, 0, s>>>(b.scenes, b.params, b.slots, b.rays, bounce0, b.tRec);
+    uint8_t* const bins = t.sortMaterials ? b.bins : nullptr;
     // traces the path rays of `bounce` (queue q, count cnt[0]) and the shadow and MIS rays of the
     // bounce before it (counts prev[1], prev[2]), with the work counters of `bounce`
     auto trace = [&](int bounce, const int32_t* extCount, const int32_t* shadowCount, const int32_t* misCount) {
-        const int32_t* ext = b.queue[bounce & 1];
-        int32_t* work = b.counts + kWfCountsPerBounce * bounce + kWfWorkBase;
-        int32_t* hist = histOf(bounce);
+        const int32_t* ext = bounce > 0 ? b.queue[bounce & 1] : nullptr;
+        int32_t* work = bounce0 + kWfCountsPerBounce * bounce + kWfWorkBase;
         auto launch = [&](auto kernel, int bs) {
-            kernel<<<t.persistentBlocks, bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, b.bins, hist, b.matBins, b.shadows,
-                                                     shadowCount, b.mis, misCount, b.shadowQ, b.misQ, b.nee, work, traceCounts);
+            kernel<<<t.persistentBlocks, bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, bins, b.matBins, b.shadows, shadowCount,
+                                                     b.mis, misCount, b.shadowQ, b.misQ, b.nee, work, traceCounts);
         };
         const bool counting = traceCounts != nullptr;
         switch (t.traceBlock) {
@@ -793,33 +801,26 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
         }
     };
     mark(8 * kWfMaxBounce + 3);
-    trace(0, b.counts, nullptr, nullptr);
+    trace(0, bounce0, nullptr, nullptr);
     for (int bounce = 0; bounce < maxBounce; bounce++) {
         const int q = bounce & 1;
-        int32_t* cnt = b.counts + kWfCountsPerBounce * bounce;
-        int32_t* nxt = b.counts + kWfCountsPerBounce * (bounce + 1);
+        int32_t* cnt = bounce0 + kWfCountsPerBounce * bounce;
+        int32_t* nxt = cnt + kWfCountsPerBounce;
         mark(8 * bounce + 0);
-        const int32_t* shadeQueue = b.queue[q];
-        if (t.sortMaterials) {
-            int32_t* hist = histOf(bounce);
-            k_wf_mat_scan<<<1, 64, 0, s>>>(hist, b.matBins);
-            k_wf_mat_scatter<<<gridAll, 256, 0, s>>>(b.bins, b.queue[q], cnt, hist, b.matBins, b.sorted);
-            shadeQueue = b.sorted;
-        }
         mark(8 * bounce + 1);
         {
             auto shade = cached ? (bounce == 0 ? k_wf_shade<true, true> : k_wf_shade<true, false>)
                                 : (bounce == 0 ? k_wf_shade<false, true> : k_wf_shade<false, false>);
-            shade<<<gridAll, kShadeBlock, 0, s>>>(b.scenes, b.params, b.slots, bounce, b.paths, b.rays, b.hits, b.nee, shadeQueue,
-                                                  cnt, b.queue[q ^ 1], nxt, b.shadows, cnt + 1, b.mis, cnt + 2,
-                                                  cached ? b.qRaw : nullptr, b.qMeta, qCount, b.tRec, b.tRaw,
-                                                  b.done, cnt + 3, b.shadowQ, b.misQ);
+            shade<<<kShadeGrid, kShadeBlock, 0, s>>>(b.scenes, b.params, b.slots, bounce, b.paths, b.rays, b.hits, b.nee, b.queue[q], cnt,
+                                                  bins, b.done[q ^ 1], cnt - kWfCountsPerBounce + 3, cnt + kWfShadeWork, b.queue[q ^ 1], nxt, b.shadows,
+                                                  cnt + 1, b.mis, cnt + 2, cached ? b.qRaw : nullptr, b.qMeta, qCount, b.tRec, b.tRaw,
+                                                  b.done[q], cnt + 3, b.shadowQ, b.misQ);
         }
         mark(8 * bounce + 2);
         // the next bounce's path rays (none after the last bounce) with this bounce's shadow and MIS rays
         trace(bounce + 1, nxt, cnt + 1, cnt + 2);
         mark(8 * bounce + 3);
-        k_wf_finalize<<<gridAll, 256, 0, s>>>(b.params, b.slots, b.paths, b.nee, b.done, cnt + 3);
+        if (bounce + 1 == maxBounce) k_wf_finalize<<<gridAll, 256, 0, s>>>(b.params, b.slots, b.paths, b.nee, b.done[q], cnt + 3);
         mark(8 * bounce + 4);
     }
     if (cached) {
@@ -864,14 +865,14 @@ hipError_t wf_reserve(WfBuffers& b, size_t cap, int maxScenes) {
     WTRY(wf_alloc(&b.nee, cap));
     WTRY(wf_alloc(&b.queue[0], cap));
     WTRY(wf_alloc(&b.queue[1], cap));
-    WTRY(wf_alloc(&b.sorted, cap));
-    WTRY(wf_alloc(&b.done, cap));
+    WTRY(wf_alloc(&b.done[0], cap));
+    WTRY(wf_alloc(&b.done[1], cap));
     WTRY(wf_alloc(&b.shadowQ, cap));
     WTRY(wf_alloc(&b.misQ, cap));
     WTRY(wf_alloc(&b.bins, cap));
     WTRY(wf_alloc(&b.shadows, cap));
     WTRY(wf_alloc(&b.mis, cap));
-    WTRY(wf_alloc(&b.counts, (size_t)kWfGlobalBase + kWfGlobalCounts));
+    WTRY(wf_alloc(&b.counts, (size_t)kWfBounceBase + kWfCountsPerBounce * (kWfMaxBounce + 1)));
 #undef WTRY
     b.cap = cap;
     b.maxScenes = maxScenes;
@@ -904,7 +905,7 @@ void wf_release(WfBuffers& b) {
     void* cs[] = {b.qRaw, b.qMeta, b.tRec, b.tRaw, b.tCount};
     for (void* p : cs)
         if (p) (void)hipFree(p);
-    void* ps[] = {b.scenes, b.params, b.slots, b.paths, b.rays, b.hits, b.nee, b.queue[0], b.queue[1], b.sorted, b.done, b.shadowQ, b.misQ, b.bins, b.shadows, b.mis, b.counts};
+    void* ps[] = {b.scenes, b.params, b.slots, b.paths, b.rays, b.hits, b.nee, b.queue[0], b.queue[1], b.done[0], b.done[1], b.shadowQ, b.misQ, b.bins, b.shadows, b.mis, b.counts};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     b = WfBuffers();

@@ -178,7 +178,7 @@ constexpr int kMaxTileRows = 64;
 
 struct WfTuning {
     int traceBlock = 256;         // block size of the persistent traversal kernels (64, 128, 256)
-    int persistentBlocks = 2048;  // grid of the traversal kernels
+    int persistentBlocks = 2048;  // grid of the traversal kernels, at most the workgroups resident at once
     int sweepBlocks = 2048;       // grid of the generate / shade / finalize sweeps
     int sortMaterials = 1;        // shade in material order within chunks of the queue
     int useGraph = 1;             // capture the pass in a hipGraph and replay it

@@ -12,7 +12,9 @@
 // Each path's arithmetic is the megakernel's, so the image does not depend on queue order.
 // Every count lives in device memory and is reset by kernels, so the bounce loop of a pass is
 // captured once in a hipGraph and replayed.
-#include "lts_internal.h"
+#include <algorithm>
+
+#include "path_order.h"
 #include "pt_device.h"
 
 namespace lts {
@@ -20,38 +22,6 @@ namespace lts {
 namespace {
 
 constexpr int kShadeBlock = 256;
-
-// Pixel of the j-th path of a sample: the image is cut into bands of T rows and each band is walked
-// column by column, so 64 consecutive paths (one wave) cover a T x 64/T tile and their rays stay
-// close (T = 8: an 8x8 tile; T = 1: scanline order). The last band holds the remaining rows.
-LTS_D int band_pixel(int j, int W, int H, int T) {
-    const int band = j / (T * W);
-    const int rows = min(T, H - T * band);
-    const int jj = j - band * T * W;
-    return (T * band + jj % rows) * W + jj / rows;
-}
-
-// Scene of path i of the pass: the last slot whose path range starts at or before i.
-LTS_D int path_scene(const WfParams& P, const WfSceneSlot* slots, long i) {
-    int lo = 0, hi = P.nScenes - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (slots[mid].pathBase <= i) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// Path i of the pass -> (scene, pixel, sample).
-LTS_D void path_origin(const WfParams& P, const WfSceneSlot* slots, long i, int& scene, int& pixel, int& sample) {
-    const int s = path_scene(P, slots, i);
-    const WfSceneSlot& sl = slots[s];
-    const long local = i - sl.pathBase;
-    const long npix = (long)sl.width * sl.height;
-    scene = s;
-    sample = sl.s0 + (int)(local / npix);
-    pixel = band_pixel((int)(local % npix), sl.width, sl.height, P.tileRows);
-}
 
 // Training paths of the radiance cache: in scene 0, every trainStride-th (sample, pixel) pair of
 // the pass in sample-major, row-major order from trainOffset, so that the set and its slot order
@@ -258,7 +228,6 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
             const bool active = bins ? x < m : k < n;
             const int pi = !active ? 0 : bins ? order[x] : kFirst ? k : queue[k];
             bool wantShadow = false, wantMis = false, wantNext = false, wantQuery = false, wantDone = false;
-            WfLightRay sh;
             if (active) {
                 const WfParams P = *prm;
                 WfPath p;
@@ -311,20 +280,7 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                 ne.p1[0] = ne.p1[1] = ne.p1[2] = 0.0f;
                 ne.p2[0] = ne.p2[1] = ne.p2[2] = 0.0f;
                 bool alive = true;
-                if (kFirst || specularBounce) {
-                    if (hh.leaf >= 0) {
-                        const int l = sv.shade[hh.leaf].light;
-                        if (l >= 0) {
-                            SurfacePoint e = make_surface(sv, hh.leaf, r, hh.u, hh.v, hh.invDet);
-                            Spec le = dot(e.n, -r.d) > 0.f ? light_le(sv.lights[l]) : spec(0.0f);
-                            L = L + beta * le;
-                        } else {
-                            L = L + beta * spec(0.0f);
-                        }
-                    } else {
-                        for (int l = 0; l < sv.nLights; l++) L = L + beta * (sv.lights[l].kind == 1 ? light_le(sv.lights[l]) : spec(0.0f));
-                    }
-                }
+                if (kFirst || specularBounce) add_emission(sv, hh.leaf, r, hh.u, hh.v, hh.invDet, beta, L);
                 if (hh.leaf < 0) {
                     alive = false;
                 } else {
@@ -364,52 +320,21 @@ __global__ __launch_bounds__(kShadeBlock, 3) void k_wf_shade(const SceneView* __
                     if (!wantQuery && sv.nLights > 0) {
                         float lpdf;
                         const int li = sample_light(sv, u0[0], &lpdf);
-                        const LightDesc& Lt = sv.lights[li];
                         ne.used = 1;
                         ne.nb[0] = beta.r; ne.nb[1] = beta.g; ne.nb[2] = beta.b;
                         ne.lpdf = lpdf;
-                        const int flags = specularBounce ? B_ALL : (B_ALL & ~B_SPEC);
-                        // light sample with MIS (IntegratorHelper.cuh:76-95)
-                        V3 wi;
-                        float lightPdf = 0.0f, scatteringPdf = 0.0f;
-                        LightPoint vis;
-                        Spec Li = sample_li(sv, Lt, si, v2(u0[1], u0[2]), &wi, &lightPdf, &vis);
-                        if (lightPdf > 0 && !isBlack(Li)) {
-                            Spec f = bsdf.f(si.wo, wi, flags) * absDot(wi, si.sn);
-                            scatteringPdf = bsdf.pdf(si.wo, wi, flags);
-                            if (!isBlack(f)) {
-                                float weight = power_heuristic(lightPdf, scatteringPdf);
-                                Spec c = f * Li * weight / lightPdf;
-                                V3 origin = offsetRayOrigin(si.p, si.pError, si.n, vis.p - si.p);
-                                V3 target = offsetRayOrigin(vis.p, vis.pError, vis.n, origin - vis.p);
-                                V3 d = target - origin;
-                                sh.o[0] = origin.x; sh.o[1] = origin.y; sh.o[2] = origin.z;
-                                sh.d[0] = d.x; sh.d[1] = d.y; sh.d[2] = d.z;
-                                sh.scene = scene; sh.tieLeaf = -1; sh.tMax = 1 - SHADOW_EPS;
-                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
-                                wantShadow = true;
-                                shadows[pi] = sh;  // per path; the queue below lists the paths
-                            }
-                        }
-                        // BSDF sample with MIS (IntegratorHelper.cuh:96-122)
-                        int sampledType = 0;
-                        Spec f2 = bsdf.sampleF(si.wo, &wi, v2(u0[3], u1[0]), &scatteringPdf, flags, &sampledType);
-                        f2 = f2 * absDot(wi, si.sn);
-                        const bool sampledSpecular = (sampledType & B_SPEC) != 0;
-                        const Spec Li2 = light_le(Lt);
-                        if (!isBlack(f2) && scatteringPdf > 0 && !isBlack(Li2)) {
-                            const Ray mr = spawn_ray(si, wi);
-                            float weight;
-                            if (mis_ray(sv, Lt, li, si, mr, sampledSpecular, scatteringPdf, weight, sh.tMax, sh.tieLeaf)) {
-                                const Spec c = f2 * Li2 * spec(1.0f) * weight / scatteringPdf;
-                                sh.o[0] = mr.o.x; sh.o[1] = mr.o.y; sh.o[2] = mr.o.z;
-                                sh.d[0] = wi.x; sh.d[1] = wi.y; sh.d[2] = wi.z;
-                                sh.scene = scene;
-                                sh.c[0] = c.r; sh.c[1] = c.g; sh.c[2] = c.b;
-                                wantMis = true;
-                                misRays[pi] = sh;
-                            }
-                        }
+                        // the records are per path; the queues below list the paths
+                        auto record = [&](V3 o, V3 d, Spec c, float tMax, int tieLeaf) {
+                            WfLightRay q;
+                            q.o[0] = o.x; q.o[1] = o.y; q.o[2] = o.z;
+                            q.d[0] = d.x; q.d[1] = d.y; q.d[2] = d.z;
+                            q.scene = scene; q.tieLeaf = tieLeaf; q.tMax = tMax;
+                            q.c[0] = c.r; q.c[1] = c.g; q.c[2] = c.b;
+                            return q;
+                        };
+                        light_rays(sv, si, bsdf, li, u0, u1, specularBounce,
+                                   [&](V3 o, V3 d, Spec c) { shadows[pi] = record(o, d, c, 1 - SHADOW_EPS, -1); wantShadow = true; },
+                                   [&](V3 o, V3 d, float tMax, int tieLeaf, Spec c) { misRays[pi] = record(o, d, c, tMax, tieLeaf); wantMis = true; });
                     }
                     // continuation (PathTracingIntegrator.cuh:79-103)
                     V3 wo = -r.d, wi;
@@ -586,19 +511,30 @@ __global__ __launch_bounds__(kCollectBlock) void k_wf_nrc_scatter(const WfParams
 // steps with 26 % of its lanes. Instead a lane whose ray has ended takes the next one as soon as half of
 // the wave's lanes are free (refilling at a quarter measured the same, at three quarters 8 % slower), and
 // the lanes that hold a triangle wait until they are half as many as those that hold a node
-// (kGateRatio; 29.5 ms of tracing per 64-spp frame of the 1M-triangle displaced sphere at 1920x1080,
-// 30.5 at a ratio of 1, 29.8 at 3, 31.1 at 6 and 38.0 without waiting; 43 ms before both). The lanes carry
+// (kGateRatio; measured before rays were shared: 29.5 ms of tracing per 64-spp frame of the 1M-triangle
+// displaced sphere at 1920x1080, 30.5 at a ratio of 1, 29.8 at 3, 31.1 at 6 and 38.0 without waiting; 43 ms
+// before both). Once no rays are left, a wave's free lanes help the others (ray_share). The lanes carry
 // rays of any kind: a shadow ray's triangle test (Triangle::simpleIntersect) is the closest-hit test with
 // the triangle's second and third corners exchanged and wider margins.
-// The launch asks for 7 waves per SIMD (at most 72 VGPRs).
+// The launch asks for 6 waves per SIMD (80 VGPRs): 25.1 ms for that frame, 27.3 at 7 waves (72 VGPRs, spilling
+// in the loop), 26.9 at 5.
 // kCount: the counting instantiation, which also adds every lane's render-node fetches and
 // triangle tests per ray kind (path, shadow, MIS) to traceCounts[0..5] (nodes, tests per kind).
-constexpr int kGateRatio = 2;
-// fewest lanes of a wave that carry rays
-constexpr int kMinWidth = 4;
+constexpr int kTraceWaves = 6;  // per SIMD
+constexpr int kMinWidth = 4;    // fewest lanes of a wave that carry rays
+// Workgroups of BS threads that the 1024 SIMDs hold at once: a grid above that leaves late workgroups.
+constexpr int resident_blocks(int bs) { return kTraceWaves * 65536 / bs; }
+
+// Rays that a wave takes at a time: its width, and up to 256 where every wave still has some 8 turns (tracing
+// of that frame: 27.2 ms with up to 256, 28.6 with 64, 28.1 with 1024).
+LTS_D int trace_chunk(int n, int waves, int width) {
+    int c = width;
+    while (c < 256 && (long)c * waves * 8 < n) c <<= 1;
+    return c;
+}
 
 template <int BS, bool kCount>
-__global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict__ scenes, const WfRay* __restrict__ rays, WfHit* __restrict__ hits,
+__global__ __launch_bounds__(BS, kTraceWaves) void k_wf_trace(const SceneView* __restrict__ scenes, const WfRay* __restrict__ rays, WfHit* __restrict__ hits,
                                                  const int32_t* __restrict__ ext, const int32_t* __restrict__ extCount,
                                                  uint8_t* __restrict__ bins, int nBins, const WfLightRay* __restrict__ shadows, const int32_t* __restrict__ shadowCount,
                                                  const WfLightRay* __restrict__ misRays, const int32_t* __restrict__ misCount,
@@ -611,7 +547,6 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
     const int nS = shadowCount ? *shadowCount : 0;
     const int nM = misCount ? *misCount : 0;
     const int n = nE + nS + nM;
-    const int segLen = ((n + kWfWorkSegments - 1) / kWfWorkSegments + 63) / 64 * 64;
     // lanes of a wave that carry rays: 64, or fewer in a small launch so that every wave gets some (a step
     // takes as long as the slowest of its lanes, and a wave with few lanes alternates less between node
     // and triangle steps: 1.61 against 1.74 ms of tracing for one sample of an 853x479 frame)
@@ -619,120 +554,77 @@ __global__ __launch_bounds__(BS, 7) void k_wf_trace(const SceneView* __restrict_
     int width = 64;
     while (width > kMinWidth && (long)width * waves > 2L * n) width >>= 1;
     const int spare = 64 - width, refill = spare + width / 2;
-    int seg = 0;             // segments found empty so far
-    int next = 0, end = 0;   // items of the wave's current chunk that no lane has taken yet
+    WorkDeal<int> q = work_deal(n, trace_chunk(n, waves, width));
     unsigned long long tally[6] = {0, 0, 0, 0, 0, 0};
     int spill[kStack - kShortStack];
-    // the lane's ray: path, kind (-1: none), direction, bound and hit
-    TraceLane l;
-    l.cur = kTraceDone; l.sp = 1; l.o = l.inv = v3(0, 0, 0); l.nx = l.ny = l.nz = false;
-    const TraceRec* recs = nullptr;
-    int path = 0, kind = -1, best = -1, mat = 0;
-    V3 d = v3(0, 0, 0);
-    float tMax = 0, hu = 0, hv = 0, hInvDet = 0;
+    __shared__ uint8_t marks[BS];
+    uint8_t* const mark = marks + (threadIdx.x & ~63);
+    const int lane = threadIdx.x & 63;
+    TraceRay t;
+    ray_none(t, lane);
+    int path = 0, wait = 0;
+    auto finish = [&]() {
+        if (t.kind == kRayClosest) {
+            WfHit o;
+            o.leaf = t.best; o.u = t.u; o.v = t.v; o.invDet = t.invDet;
+            hits[path] = o;
+            if (bins) bins[path] = (uint8_t)(t.best < 0 ? nBins - 1 : (t.mat < nBins - 1 ? t.mat : nBins - 2));
+        } else if (!t.mat) {
+            const bool shadow = t.kind == kRayShadow;
+            const float* c = (shadow ? shadows : misRays)[path].c;
+            float* p = shadow ? nee[path].p1 : nee[path].p2;
+            p[0] = c[0]; p[1] = c[1]; p[2] = c[2];
+        }
+        t.kind = kRayNone;
+    };
     for (;;) {
-        const unsigned long long idle = __ballot(l.cur == kTraceDone);
-        const bool dry = seg >= kWfWorkSegments && next >= end;
-        if (idle == ~0ull || (!dry && __popcll(idle) >= refill)) {
-            if (l.cur == kTraceDone && kind >= 0) {
-                if (kind == 0) {
-                    WfHit o;
-                    o.leaf = best; o.u = hu; o.v = hv; o.invDet = hInvDet;
-                    hits[path] = o;
-                    // the hit is also filed under its material bin (misses in the last) for shading
-                    if (bins) bins[path] = (uint8_t)(best < 0 ? nBins - 1 : min(mat, nBins - 2));
-                } else if (mat == 0) {  // nothing blocked the light ray
-                    const float4 c = reinterpret_cast<const float4*>((kind == 1 ? shadows : misRays) + path)[2];
-                    float* p = kind == 1 ? nee[path].p1 : nee[path].p2;
-                    p[0] = c.x; p[1] = c.y; p[2] = c.z;
-                }
-                kind = -1;
+        const unsigned long long idle = __ballot(t.l.cur == kTraceDone);
+        if (q.open && (idle == ~0ull || __popcll(idle) >= refill)) {
+            if (t.l.cur == kTraceDone && t.kind >= 0) finish();
+            if (q.next >= q.end) {
+                work_next(q, BS / 64, resident_blocks(BS), work);
+                if (!q.open) continue;
             }
-            if (next >= end) {
-                // workgroups are dealt to the 8 XCDs round robin: the waves of XCD blockIdx % 8 start on
-                // their own segment and keep neighbouring rays in one L2, then move on to the others
-                while (seg < kWfWorkSegments) {
-                    const int s = (blockIdx.x + seg) % kWfWorkSegments;
-                    int base = 0;
-                    if ((threadIdx.x & 63) == 0) base = atomicAdd(&work[kWfWorkStride * s], width);
-                    base = __builtin_amdgcn_readfirstlane(base);
-                    if (base < segLen) {
-                        next = s * segLen + base;
-                        end = min(next + width, n);
-                        if (next < end) break;
-                    }
-                    seg++;
-                }
-                if (seg >= kWfWorkSegments) {
-                    next = end = 0;
-                    if (idle == ~0ull) break;
-                    continue;
-                }
-            }
-            const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0));
-            const int k = next + rank;
-            const int give = min((int)__popcll(idle) - spare, end - next);
-            if (l.cur == kTraceDone && rank < give) {
+            const int rank = lanes_below(idle), k = q.next + rank;
+            const int give = min((int)__popcll(idle) - spare, q.end - q.next);
+            if (t.l.cur == kTraceDone && rank < give) {
                 const float4* src;
+                int kind;
                 if (k < nE) {
-                    kind = 0;
+                    kind = kRayClosest;
                     path = ext ? ext[k] : k;  // bounce 0 has no queue
                     src = reinterpret_cast<const float4*>(rays + path);
                 } else if (k < nE + nS) {
-                    kind = 1;
+                    kind = kRayShadow;
                     path = shadowQueue[k - nE];
                     src = reinterpret_cast<const float4*>(shadows + path);
                 } else {
-                    kind = 2;
+                    kind = kRayMis;
                     path = misQueue[k - nE - nS];
                     src = reinterpret_cast<const float4*>(misRays + path);
                 }
                 const float4 a = src[0], b = src[1];
-                best = -1;
-                tMax = INFINITY;
-                if (kind > 0) {
-                    tMax = src[2].w;
-                    best = __float_as_int(b.w);
-                }
                 const SceneView& sv = scenes[__float_as_int(b.z)];
-                recs = sv.recs;
-                d = v3(a.w, b.x, b.y);
-                mat = 0;
-                hu = hv = hInvDet = 0;
-                trace_begin(l, v3(a.x, a.y, a.z), d, sv.root, ts);
+                const bool closest = kind == kRayClosest;
+                ray_begin(t, kind, v3(a.x, a.y, a.z), v3(a.w, b.x, b.y), closest ? INFINITY : src[2].w,
+                          closest ? -1 : __float_as_int(b.w), sv.recs, sv.root, ts);
             }
-            next += give;
+            q.next += give;
             continue;
         }
-        const bool done = l.cur == kTraceDone, leafStep = l.cur < 0 && !done;
-        const unsigned long long waiting = __ballot(leafStep), walking = __ballot(l.cur >= 0);
-        if (walking != 0 && kGateRatio * __popcll(waiting) < __popcll(walking)) {
-            if (l.cur >= 0) {
-                if (kCount) tally[0] += kind == 0, tally[2] += kind == 1, tally[4] += kind == 2;
-                trace_node(l, recs, tMax, ts, spill);
-            }
-        } else if (leafStep) {
-            if (kCount) tally[1] += kind == 0, tally[3] += kind == 1, tally[5] += kind == 2;
-            const TraceTri tr = trace_triangle(l, recs);
-            Ray r;
-            r.o = l.o; r.d = d; r.tMax = tMax;
-            const bool shadow = kind == 1;
-            const V3 p1 = shadow ? tr.p2 : tr.p1, p2 = shadow ? tr.p1 : tr.p2;
-            const float limit = shadow ? kOnePlusEpsF : kOneMinusEpsF;
-            float t, u, v, id;
-            bool over = false;
-            if (tri_mt(tr.p0, p1, p2, r, limit, t, u, v, id) && t > 0 && (t < tMax || (t == tMax && !shadow && tr.leaf < best))) {
-                if (kind == 0) {
-                    tMax = t;
-                    best = tr.leaf; mat = tr.mat; hu = u; hv = v; hInvDet = id;
-                } else if (!shadow || leaf_box_passes(tr.p0, tr.p1, tr.p2, r)) {
-                    mat = 1;  // blocked
-                    over = true;
-                }
-            }
-            if (over) l.cur = kTraceDone;
-            else trace_pop(l, ts, spill);
+        if (!q.open && idle == ~0ull) {
+            ray_settle(t, lane);
+            if (t.kind >= 0) finish();
+            break;
         }
+        if (!kCount && !q.open && __popcll(idle) >= kShareIdle && --wait < 0) {
+            wait = kShareSteps;
+            ray_settle(t, lane);
+            const bool held = ray_held(t, lane, mark), free = t.l.cur == kTraceDone && !held;
+            if (free && t.kind >= 0) finish();
+            ray_share(t, free, lane, ts);
+        }
+        ray_step<kCount>(t, ts, spill, tally);
     }
     if constexpr (kCount) {
         for (int q = 0; q < 6; q++) atomicAdd(&traceCounts[q], tally[q]);
@@ -790,7 +682,7 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
         const int32_t* ext = bounce > 0 ? b.queue[bounce & 1] : nullptr;
         int32_t* work = bounce0 + kWfCountsPerBounce * bounce + kWfWorkBase;
         auto launch = [&](auto kernel, int bs) {
-            kernel<<<t.persistentBlocks, bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, bins, b.matBins, b.shadows, shadowCount,
+            kernel<<<std::min(t.persistentBlocks, resident_blocks(bs)), bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, bins, b.matBins, b.shadows, shadowCount,
                                                      b.mis, misCount, b.shadowQ, b.misQ, b.nee, work, traceCounts);
         };
         const bool counting = traceCounts != nullptr;

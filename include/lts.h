@@ -49,7 +49,10 @@ typedef struct lts_bvh_timing {
     double tree_ms;    /* Karras hierarchy + bottom-up refit + node packing        */
 } lts_bvh_timing;
 
-/* Integrators. */
+/* Integrators. The megakernel and the wavefront are the plain path tracer: their samples are the same
+ * bit for bit, and each runs the form that suits the size of its passes, whole paths in one launch up to
+ * 2^22 samples of a scene and a wavefront of queues above. A wavefront for which a tuning option is set
+ * (trace_block .. count_traversal below) runs as queues at any size. */
 #define LTS_INTEGRATOR_MEGAKERNEL 0
 #define LTS_INTEGRATOR_WAVEFRONT 1
 #define LTS_INTEGRATOR_CACHED 2
@@ -69,7 +72,7 @@ typedef struct lts_render_params {
     int32_t integrator;   /* LTS_INTEGRATOR_*                                      */
     int32_t spp_per_pass; /* samples per pass; 0 = automatic (wavefront and cached: */
                           /* 2^27 paths per pass; megakernel: 2^28 / 12 B)          */
-    /* wavefront only (0 / -1 = default or the autotuned value) */
+    /* wavefront of queues only (0 / -1 = default or the autotuned value) */
     int32_t trace_block;        /* block size of the persistent traversal kernels: 64, 128, 256 */
     int32_t persistent_blocks;  /* grid of the persistent traversal kernels                     */
     int32_t sort_materials;     /* -1 default (on), 0 off, 1 shade in material order            */

@@ -83,6 +83,8 @@ struct lts_ctx {
     float* rgb = nullptr;
     size_t filmCap = 0;
     unsigned long long* counters = nullptr;
+    int32_t* pathWork = nullptr;  // two sets of work counters of the whole-path launches, taken in turn
+    int pathTurn = 0;
     int* perm = nullptr;  // Perlin permutation (512 ints)
     hipEvent_t ev[8] = {};
     // wavefront integrator
@@ -494,6 +496,25 @@ int autotune(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_render_p
     return LTS_OK;
 }
 
+// Whether the caller leaves the wavefront's tuning open and asks for none of its measurements.
+bool wavefront_defaults(const lts_render_params* p) {
+    return p->trace_block == 0 && p->persistent_blocks == 0 && p->sort_materials < 0 && p->use_graph < 0 && p->tile_rows == 0 &&
+           !p->autotune && !p->profile_phases && !p->count_traversal;
+}
+
+// Samples of a wavefront pass. Automatic: 2^27 paths (about 36 GB of path state at 268 B per path). Each pass runs its
+// bounces as separate launches whose late ones hold few paths, so fewer, larger passes keep the
+// GPU busy: 2^24 -> 2^26 paths took the 1080p 64-spp frame from 585 to 756 Msamples/s, and
+// 2^26 -> 2^27 (the whole frame in one pass) from 1392 to 1524. The cached integrator takes the
+// same passes: a 64-spp 1080p frame is one pass that queries the cache and trains it once, and
+// the cache is carried from frame to frame (its warm-up passes are the first frames after
+// lts_nrc_configure). Passes of 2^25 paths, which let one fresh frame warm up and then query,
+// cost the cached frame 112 ms against 81 ms in one pass.
+int wavefront_pass(const lts_render_params* p, size_t pixels) {
+    const size_t passPaths = (size_t)1 << 27;
+    return p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, passPaths / pixels);
+}
+
 // The wavefront integrator over one or more scenes, executed on c's stream and buffers.
 int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_render_params* p, float* const* rgb_out,
                      float* sample_rgb, lts_stats* st) {
@@ -512,22 +533,18 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
     sample_range(p, &b0, &b1);
     if (b0 > 0 && scenes.size() != 1) return fail(c, LTS_E_ARG, "progressive rendering is for one scene");
     if (b0 > 0 && (rc = film_continues(c, p, b0)) != LTS_OK) return rc;
-    // automatic pass: 2^27 paths (about 36 GB of path state at 268 B per path). Each pass runs its
-    // bounces as separate launches whose late ones hold few paths, so fewer, larger passes keep the
-    // GPU busy: 2^24 -> 2^26 paths took the 1080p 64-spp frame from 585 to 756 Msamples/s, and
-    // 2^26 -> 2^27 (the whole frame in one pass) from 1392 to 1524. The cached integrator takes the
-    // same passes: a 64-spp 1080p frame is one pass that queries the cache and trains it once, and
-    // the cache is carried from frame to frame (its warm-up passes are the first frames after
-    // lts_nrc_configure). Passes of 2^25 paths, which let one fresh frame warm up and then query,
-    // cost the cached frame 112 ms against 81 ms in one pass.
-    const size_t passPaths = (size_t)1 << 27;
-    int pass = p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, passPaths / totalPix);
+    int pass = wavefront_pass(p, totalPix);
     if (sample_rgb) pass = b1 - b0;
     pass = std::min(pass, b1 - b0);
     const size_t cap = totalPix * (size_t)pass;
     if (cap > (size_t)INT32_MAX) return fail(c, LTS_E_ARG, "pass holds more than 2^31 paths");
     const bool realloc = cap > c->wf.cap || (int)scenes.size() > c->wf.maxScenes;
-    HIPCHK(c, wf_reserve(c->wf, cap, (int)scenes.size()));
+    const hipError_t reserved = wf_reserve(c->wf, cap, (int)scenes.size());
+    if (reserved == hipErrorOutOfMemory && p->integrator == LTS_INTEGRATOR_MEGAKERNEL) {
+        (void)hipGetLastError();
+        return LTS_E_NOMEM;  // the caller has a form that needs no path state
+    }
+    HIPCHK(c, reserved);
     if (realloc && c->wfExec) {
         (void)hipGraphExecDestroy(c->wfExec);
         c->wfExec = nullptr;
@@ -807,7 +824,10 @@ int lts_create(lts_ctx** out, int dev) {
     for (int i = 0; i < 512; i++) table[i] = kPerm256[i & 255];
     if (hipMalloc((void**)&c->perm, sizeof(table)) != hipSuccess ||
         hipMemcpy(c->perm, table, sizeof(table), hipMemcpyHostToDevice) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
-    if (hipMalloc((void**)&c->counters, kTraceCounters * sizeof(unsigned long long)) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
+    const int32_t clear[2 * kPathWork] = {};
+    if (hipMalloc((void**)&c->counters, kTraceCounters * sizeof(unsigned long long)) != hipSuccess ||
+        hipMalloc((void**)&c->pathWork, 2 * kPathWork * sizeof(int32_t)) != hipSuccess ||
+        hipMemcpy(c->pathWork, clear, sizeof(clear), hipMemcpyHostToDevice) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
     *out = c;
     return LTS_OK;
 }
@@ -818,7 +838,7 @@ void lts_destroy(lts_ctx* c) {
     (void)hipStreamSynchronize(c->stream);
     free_scene(c->scene);
     bvh_release(c->build);
-    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->perm, c->xfBuf};
+    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->pathWork, c->perm, c->xfBuf};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : c->ev)
@@ -1102,19 +1122,38 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
     int rc = check_render_params(c, p);
     if (rc != LTS_OK) return rc;
     HIPCHK(c, hipSetDevice(c->device));
-    if (p->integrator == LTS_INTEGRATOR_WAVEFRONT || p->integrator == LTS_INTEGRATOR_CACHED) {
-        std::vector<lts_ctx*> one{c};
-        return render_wavefront(c, one, p, &rgb_out, sample_rgb, st);
-    }
     const SceneView& sv = c->scene.view;
     const int W = sv.cam.width, H = sv.cam.height;
     const size_t npix = (size_t)W * H;
     int b0, b1;
     sample_range(p, &b0, &b1);
-    if ((rc = film_continues(c, p, b0)) != LTS_OK) return rc;
-    int pass = p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, std::min<size_t>((size_t)(b1 - b0), (size_t)(1u << 28) / (npix * 12)));
-    if (sample_rgb) pass = b1 - b0;  // all samples are returned: one pass
+    // samples of a pass; all of them where they are returned
+    const bool wavefront = p->integrator == LTS_INTEGRATOR_WAVEFRONT;
+    int pass = wavefront ? wavefront_pass(p, npix)
+               : p->spp_per_pass > 0 ? p->spp_per_pass
+                                     : (int)std::max<size_t>(1, std::min<size_t>((size_t)(b1 - b0), (size_t)(1u << 28) / (npix * 12)));
+    if (sample_rgb) pass = b1 - b0;
     pass = std::min(pass, b1 - b0);
+    const std::vector<lts_ctx*> one{c};
+    if (p->integrator == LTS_INTEGRATOR_CACHED) return render_wavefront(c, one, p, &rgb_out, sample_rgb, st);
+    // The plain path tracer has two forms with the same samples: whole paths in one launch, and the wavefront.
+    // The size of the pass decides (kPathPass) for the megakernel, whose traversal counts are of whole paths,
+    // and for a wavefront whose tuning the caller leaves open. A megakernel pass stays whole where the path
+    // state finds no memory.
+    const bool small = npix * (size_t)pass <= kPathPass;
+    if (wavefront && !(small && p->max_bounce > 0 && wavefront_defaults(p)))
+        return render_wavefront(c, one, p, &rgb_out, sample_rgb, st);
+    if (p->integrator == LTS_INTEGRATOR_MEGAKERNEL && !small && p->max_bounce > 0 && p->max_bounce <= kWfMaxBounce &&
+        !p->count_traversal && npix * (size_t)pass <= ((size_t)1 << 27)) {
+        lts_render_params q = *p;
+        q.spp_per_pass = pass;
+        q.trace_block = q.persistent_blocks = q.tile_rows = q.autotune = q.profile_phases = 0;
+        q.sort_materials = q.use_graph = -1;
+        rc = render_wavefront(c, one, &q, &rgb_out, sample_rgb, st);
+        if (rc == LTS_OK && st) st->trace_block = st->persistent_blocks = st->sort_materials = st->use_graph = st->tile_rows = st->spp_per_pass = 0;
+        if (rc != LTS_E_NOMEM) return rc;
+    }
+    if ((rc = film_continues(c, p, b0)) != LTS_OK) return rc;
     if ((rc = ensure_samples(c, npix * (size_t)pass * 3)) != LTS_OK) return rc;
     if ((rc = ensure_film(c, npix)) != LTS_OK) return rc;
     hipStream_t s = c->stream;
@@ -1123,14 +1162,19 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
     rl.spp = p->spp; rl.maxBounce = p->max_bounce; rl.rrStart = p->rr_start; rl.seed = p->seed;
     rl.stratified = p->stratified; rl.sampleL = c->sampleL; rl.film = c->film;
     rl.counters = p->count_traversal ? c->counters : nullptr;
-    if (rl.counters) HIPCHK(c, hipMemsetAsync(c->counters, 0, 2 * sizeof(unsigned long long), s));
+    if (rl.counters) HIPCHK(c, hipMemsetAsync(c->counters, 0, kTraceCounters * sizeof(unsigned long long), s));
     double renderMs = 0, resolveMs = 0;
     int64_t launches = 0;
     for (int s0 = b0; s0 < b1; s0 += pass) {
         rl.s0 = s0;
         rl.s1 = std::min(b1, s0 + pass);
         HIPCHK(c, hipEventRecord(c->ev[5], s));
-        HIPCHK(c, p->integrator == LTS_INTEGRATOR_BDPT ? launch_bdpt(sv, rl, s) : launch_megakernel(sv, rl, s));
+        if (p->integrator == LTS_INTEGRATOR_BDPT) {
+            HIPCHK(c, launch_bdpt(sv, rl, s));
+        } else {
+            HIPCHK(c, launch_paths(sv, rl, c->pathWork + kPathWork * c->pathTurn, c->pathWork + kPathWork * (1 - c->pathTurn), s));
+            c->pathTurn = 1 - c->pathTurn;
+        }
         HIPCHK(c, hipEventRecord(c->ev[6], s));
         HIPCHK(c, launch_film_gather(sv, rl, s));
         HIPCHK(c, hipEventRecord(c->ev[7], s));
@@ -1153,6 +1197,15 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         st->kernel_avg_ms = launches ? renderMs / launches : 0;
         st->samples = (int64_t)npix * (b1 - b0);
         st->msamples_per_s = (renderMs + resolveMs) > 0 ? st->samples / ((renderMs + resolveMs) * 1e3) : 0;
+        if (wavefront) {
+            const WfTuning t;
+            st->trace_block = t.traceBlock;
+            st->persistent_blocks = t.persistentBlocks;
+            st->sort_materials = t.sortMaterials;
+            st->use_graph = t.useGraph;
+            st->tile_rows = t.tileRows;
+            st->spp_per_pass = pass;
+        }
         if (rl.counters) {
             unsigned long long cnt[2];
             HIPCHK(c, hipMemcpy(cnt, c->counters, sizeof cnt, hipMemcpyDeviceToHost));

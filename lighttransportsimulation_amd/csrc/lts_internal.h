@@ -111,8 +111,16 @@ struct RenderLaunch {
     float* film;         // [H][W][4] rgb + weight, accumulated across passes
     unsigned long long* counters;  // optional [2]: node visits, triangle tests
 };
-hipError_t launch_megakernel(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);
-// Bidirectional path tracing (bdpt.hip): the same launch, sample layout and film as the megakernel.
+// Whole paths in one launch (paths.hip). work, other: kPathWork counters each; the launch takes work cleared
+// and clears other, so a context's launches alternate between two sets.
+constexpr int kPathWork = 128;
+hipError_t launch_paths(const SceneView& sv, const RenderLaunch& rl, int32_t* work, int32_t* other, hipStream_t stream);
+// Passes of at most this many samples of one scene run as whole paths, larger ones as wavefront passes
+// (device ms, whole paths / wavefront, of a 1280x720 frame of a 360k-triangle displaced sphere: 0.92M samples
+// 1.27/1.52, 3.7M 2.88/2.77, 7.4M 5.06/4.06; of a 256x256 Cornell box: 1.0M 1.52/2.08, 4.2M 4.74/5.03; of a
+// 1920x1080 frame of the 1M-triangle sphere: 2.1M 1.89/2.53, 4.1M 3.16/3.45, 8.3M 5.76/5.12).
+constexpr size_t kPathPass = (size_t)1 << 22;
+// Bidirectional path tracing (bdpt.hip), with the same sample layout and film.
 constexpr int kBdptMaxBounce = 8;
 hipError_t launch_bdpt(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);
 hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);

@@ -460,6 +460,32 @@ LTS_D void ray_share(TraceRay& t, bool free, int lane, TraceStack ts) {
     }
 }
 
+// Traces the wave's rays to their ends, sharing them among the lanes without one (kind kRayNone), which are
+// without one again afterwards. Run by all lanes. A function of its own, with the stack's LDS address as a
+// number (a generic pointer would make every access to it a flat one): inlined, its registers took the trace
+// loop's.
+__attribute__((noinline)) static __device__ void ray_finish_shared(TraceRay* ray, unsigned ldsAddress, int stride, int* spill) {
+    const int lane = threadIdx.x & 63;
+    const TraceStack ts{(int*)(__attribute__((address_space(3))) int*)ldsAddress, stride};
+    TraceRay t = *ray;
+    int wait = 0;
+    while (__ballot(t.l.cur != kTraceDone)) {
+        if (--wait < 0) {
+            wait = kShareSteps;
+            ray_settle(t, lane);
+            ray_share(t, t.kind == kRayNone, lane, ts);
+        }
+        ray_step<false>(t, ts, spill, nullptr);
+    }
+    ray_settle(t, lane);
+    *ray = t;
+}
+LTS_D void ray_finish_shared(TraceRay& t, TraceStack ts, int* spill) {
+    TraceRay c = t;
+    ray_finish_shared(&c, (unsigned)(uintptr_t)(__attribute__((address_space(3))) int*)ts.lds, ts.stride, spill);
+    t = c;
+}
+
 // What a traversal does at a triangle.
 enum TraceKind {
     kTraceClosest,  // Triangle::intersect: keep the closest hit
@@ -1216,43 +1242,6 @@ LTS_D void light_rays(const SceneView& sv, const SurfacePoint& si, const Bsdf& b
         if (mis_ray(sv, Lt, li, si, mr, sampledSpecular, scatteringPdf, weight, tMax, tieLeaf))
             mis(mr.o, wi, tMax, tieLeaf, f2 * Li2 * spec(1.0f) * weight / scatteringPdf);
     }
-}
-
-// estimateDirect (intergrators/IntegratorHelper.cuh:51-125)
-LTS_D Spec estimate_direct(const SceneView& sv, const SurfacePoint& si, const Bsdf& bsdf, V2 uScatter, int li, V2 uLight, bool specular,
-                           TraceStack ts) {
-    const LightDesc& L = sv.lights[li];
-    Spec Ld = spec(0.0f);
-    int flags = specular ? B_ALL : (B_ALL & ~B_SPEC);
-    V3 wi;
-    float lightPdf = 0.0f, scatteringPdf = 0.0f;
-    LightPoint vis;
-    Spec Li = sample_li(sv, L, si, uLight, &wi, &lightPdf, &vis);
-    if (lightPdf > 0 && !isBlack(Li)) {
-        Spec f = bsdf.f(si.wo, wi, flags) * absDot(wi, si.sn);
-        scatteringPdf = bsdf.pdf(si.wo, wi, flags);
-        if (!isBlack(f)) {
-            if (!unoccluded(sv, si, vis, ts)) Li = spec(0.0f);
-            if (!isBlack(Li)) {
-                float weight = power_heuristic(lightPdf, scatteringPdf);
-                Ld = Ld + f * Li * weight / lightPdf;
-            }
-        }
-    }
-    int sampledType = 0;
-    Spec f = bsdf.sampleF(si.wo, &wi, uScatter, &scatteringPdf, flags, &sampledType);
-    f = f * absDot(wi, si.sn);
-    const bool sampledSpecular = (sampledType & B_SPEC) != 0;
-    const Spec Li2 = light_le(L);
-    if (!isBlack(f) && scatteringPdf > 0 && !isBlack(Li2)) {
-        Ray mr = spawn_ray(si, wi);
-        float weight;
-        int tieLeaf;
-        if (mis_ray(sv, L, li, si, mr, sampledSpecular, scatteringPdf, weight, mr.tMax, tieLeaf) &&
-            !trace_any<true>(sv, mr, ts, nullptr, tieLeaf))
-            Ld = Ld + f * Li2 * spec(1.0f) * weight / scatteringPdf;
-    }
-    return Ld;
 }
 
 // Film sample position of (pixel, sample): dims 0-1, stratified per Sampler::stratifiedSample

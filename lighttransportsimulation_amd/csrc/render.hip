@@ -1,75 +1,11 @@
-// Plain path tracer for gfx950: one thread per (pixel, sample), the reference integrator
-// (intergrators/PathTracingIntegrator.cuh:26-109) per thread, followed by a deterministic film
-// gather (rendering/Camera.cu:192-218 without atomics, then getRender, Camera.cu:256-289).
-//
-// Launch shape: blocks of 256 threads cover a 16x16 pixel tile for one sample index, so each
-// 64-wide wavefront traces 4 x 16 neighbouring pixels; grid.y walks the samples of the pass.
+// Film and query kernels (gfx950): the deterministic film gather (rendering/Camera.cu:192-218 without
+// atomics, then getRender, Camera.cu:256-289), caller-given rays, and small fills and copies.
 #include "pt_device.h"
 #include "lts_internal.h"
 
 namespace lts {
 
 namespace {
-
-constexpr int kTileSide = 16;
-
-// One camera sample of PathTracingIntegrator::evaluate.
-LTS_D Spec radiance(const SceneView& sv, int px, int py, int sample, const RenderLaunch& rl, unsigned long long* cnt,
-                     TraceStack ts, const NoiseTables& perm) {
-    Sampler smp;
-    smp.seed = rl.seed;
-    smp.pixel = (uint32_t)(py * sv.cam.width + px);
-    smp.sample = (uint32_t)sample;
-    const CameraSample cs = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
-    Ray r = camera_ray(sv, cs);
-    Spec L = spec(0.0f), beta = spec(1.0f);
-    bool specularBounce = false;
-    for (int bounce = 0; bounce < rl.maxBounce; bounce++) {
-        Hit h = trace_closest(sv, r, ts, cnt, cnt ? cnt + 1 : nullptr);
-        if (bounce == 0 || specularBounce) {
-            if (h.leaf >= 0) {
-                int l = sv.shade[h.leaf].light;
-                // the geometric normal decides emission; it needs the full interaction
-                if (l >= 0) {
-                    SurfacePoint e = make_surface(sv, h.leaf, r, h.u, h.v, h.invDet);
-                    Spec le = dot(e.n, -r.d) > 0.f ? light_le(sv.lights[l]) : spec(0.0f);
-                    L = L + beta * le;
-                } else {
-                    L = L + beta * spec(0.0f);
-                }
-            } else {
-                for (int l = 0; l < sv.nLights; l++) L = L + beta * (sv.lights[l].kind == 1 ? light_le(sv.lights[l]) : spec(0.0f));
-            }
-        }
-        if (h.leaf < 0) break;
-        SurfacePoint si = make_surface(sv, h.leaf, r, h.u, h.v, h.invDet);
-        if (bounce == 0) camera_footprint(sv, si, cs, rl.spp, r, h.invDet);
-        Bsdf bsdf = make_bsdf(sv, si, perm);
-        float u0[4], u1[4];
-        smp.block(1 + 2 * bounce, u0);
-        smp.block(2 + 2 * bounce, u1);
-        if (sv.nLights > 0) {
-            float lpdf;
-            int ln = sample_light(sv, u0[0], &lpdf);
-            Spec ld = estimate_direct(sv, si, bsdf, v2(u0[3], u1[0]), ln, v2(u0[1], u0[2]), specularBounce, ts);
-            L = L + beta * (ld / lpdf);
-        }
-        V3 wo = -r.d, wi;
-        float pdf;
-        int flags = 0;
-        Spec f = bsdf.sampleF(wo, &wi, v2(u1[1], u1[2]), &pdf, B_ALL, &flags);
-        if (isBlack(f) || pdf == 0) break;
-        specularBounce = (flags & B_SPEC) != 0;
-        beta = beta * (f * absDot(wi, si.sn) / pdf);
-        r = spawn_ray(si, wi);
-        if (bounce >= rl.rrStart) {
-            float q = fmaxf(0.05f, 1 - lum(beta));
-            if (u1[3] < q) break;
-            beta = beta / (1 - q);
-        }
-    }
-    return L;
-}
 
 __global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tris, const ShadeTri* __restrict__ shade, int n,
                                                        TraceRec* __restrict__ recs, int nRecs) {
@@ -79,35 +15,6 @@ __global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tri
         const uint32_t leaf = recs[k].w[11];
         if (leaf < (uint32_t)n) recs[k].w[10] = (uint32_t)shade[leaf].mat;
     }
-}
-
-// Latency-bound: five waves per SIMD (the compiler spills the rest of the path state to scratch)
-// measured 696 Msamples/s on the 1080p workload against 679 at four, 647 at three and 470 at the two
-// waves its natural register count allows.
-__global__ __launch_bounds__(256, 5) void k_megakernel(SceneView sv, RenderLaunch rl) {
-    __shared__ int stk[kShortStack * 256];
-    __shared__ NoiseTables perm;
-    noise_tables(perm, sv.perm, threadIdx.x, 256);
-    __syncthreads();
-    const int W = sv.cam.width, H = sv.cam.height;
-    const int tilesX = (W + kTileSide - 1) / kTileSide;
-    // Workgroups are dealt to the 8 XCDs round robin in dispatch order. Tiles stay dealt round robin
-    // (every XCD gets every eighth tile, which balances sky against geometry), but an XCD runs all
-    // samples of a tile back to back, so the blocks it holds at a time cover a few tiles.
-    const int dispatch = blockIdx.y * gridDim.x + blockIdx.x;
-    int tile = blockIdx.x, sy = blockIdx.y;
-    if (gridDim.x % 8 == 0) {
-        const int i = dispatch / 8;  // the XCD's i-th block
-        tile = dispatch % 8 + 8 * (i / gridDim.y);
-        sy = i % gridDim.y;
-    }
-    const int px = (tile % tilesX) * kTileSide + (threadIdx.x & (kTileSide - 1));
-    const int py = (tile / tilesX) * kTileSide + (threadIdx.x / kTileSide);
-    const int sample = rl.s0 + sy;
-    if (px >= W || py >= H || sample >= rl.s1) return;
-    Spec L = radiance(sv, px, py, sample, rl, rl.counters, lds_stack(stk, threadIdx.x, 256), perm);
-    float* o = rl.sampleL + 3 * ((size_t)sy * W * H + (size_t)py * W + px);
-    o[0] = L.r; o[1] = L.g; o[2] = L.b;
 }
 
 // Pixel (x, y) gathers, for each sample in order and each owner pixel (ox, oy) with ox in
@@ -183,13 +90,6 @@ __global__ void k_get_render(const float4* film, float* rgb, int W, int H) {
 }
 
 }  // namespace
-
-hipError_t launch_megakernel(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream) {
-    const int W = sv.cam.width, H = sv.cam.height;
-    dim3 grid(((W + kTileSide - 1) / kTileSide) * ((H + kTileSide - 1) / kTileSide), rl.s1 - rl.s0);
-    k_megakernel<<<grid, 256, 0, stream>>>(sv, rl);
-    return hipGetLastError();
-}
 
 hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream) {
     const int W = sv.cam.width, H = sv.cam.height;

@@ -207,6 +207,8 @@ int lts_render_tree_info(lts_ctx* ctx, int32_t* kind, int32_t* depth, int32_t* n
  * triangle's primitive number (the order of the scene's meshes, as lts_scene_info counts them) or
  * -1, t[i] the distance in units of the direction's length (infinity for a miss). */
 int lts_trace_rays(lts_ctx* ctx, const float* rays, int32_t n, int32_t* prim, float* t);
+/* The same of rays whose origins and directions (3 floats each) lie in arrays of their own. */
+int lts_trace_rays_split(lts_ctx* ctx, const float* origins, const float* directions, int32_t n, int32_t* prim, float* t);
 
 /* Replaces CreateBVHTree (acceleration/BVH.cuh:411-452) for a triangle soup of n triangles
  * (9 floats each, host memory). mode 0 reproduces the reference's leaf assignment (leaf k holds

@@ -85,6 +85,10 @@ struct lts_ctx {
     unsigned long long* counters = nullptr;
     int32_t* pathWork = nullptr;  // two sets of work counters of the whole-path launches, taken in turn
     int pathTurn = 0;
+    HostStage stage;
+    // lts_trace_rays: rays, then hits, kept up to kRayBufKeep rays
+    float* rayBuf = nullptr;
+    size_t rayCap = 0;
     int* perm = nullptr;  // Perlin permutation (512 ints)
     hipEvent_t ev[8] = {};
     // wavefront integrator
@@ -515,6 +519,8 @@ int wavefront_pass(const lts_render_params* p, size_t pixels) {
     return p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, passPaths / pixels);
 }
 
+size_t image_bytes(const SceneView& sv) { return (size_t)sv.cam.width * sv.cam.height * 3 * sizeof(float); }
+
 // The wavefront integrator over one or more scenes, executed on c's stream and buffers.
 int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_render_params* p, float* const* rgb_out,
                      float* sample_rgb, lts_stats* st) {
@@ -638,6 +644,14 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             HIPCHK(c, launch_film_gather(views[i], rl, s));
         }
         HIPCHK(c, hipEventRecord(c->ev[7], s));
+        if (s1 == b1) {
+            // the images' copies wait on the device, behind the last pass
+            for (size_t i = 0; i < scenes.size(); i++) HIPCHK(c, launch_get_render(views[i], scenes[i]->film, scenes[i]->rgb, s));
+            for (size_t i = 0; rgb_out && i < scenes.size(); i++)
+                if (rgb_out[i]) stage_touch(rgb_out[i], image_bytes(views[i]));
+            for (size_t i = 0; rgb_out && i < scenes.size(); i++)
+                if (rgb_out[i]) HIPCHK(c, stage_to_host(c->stage, rgb_out[i], scenes[i]->rgb, image_bytes(views[i]), s));
+        }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
         renderMs += ms_between(c->ev[5], c->ev[6]);
         resolveMs += ms_between(c->ev[6], c->ev[7]);
@@ -659,16 +673,9 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             }
         }
         if (sample_rgb)
-            HIPCHK(c, hipMemcpy(sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), hipMemcpyDeviceToHost));
+            HIPCHK(c, stage_to_host(c->stage, sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), s));
     }
-    for (size_t i = 0; i < scenes.size(); i++) {
-        lts_ctx* x = scenes[i];
-        HIPCHK(c, launch_get_render(views[i], x->film, x->rgb, s));
-        film_advance(x, p, b1);
-        if (rgb_out && rgb_out[i])
-            HIPCHK(c, hipMemcpyAsync(rgb_out[i], x->rgb, (size_t)views[i].cam.width * views[i].cam.height * 3 * sizeof(float),
-                                     hipMemcpyDeviceToHost, s));
-    }
+    for (lts_ctx* x : scenes) film_advance(x, p, b1);
     HIPCHK(c, hipStreamSynchronize(s));
     if (st) {
         std::memset(st, 0, sizeof(*st));
@@ -827,7 +834,7 @@ int lts_create(lts_ctx** out, int dev) {
     const int32_t clear[2 * kPathWork] = {};
     if (hipMalloc((void**)&c->counters, kTraceCounters * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc((void**)&c->pathWork, 2 * kPathWork * sizeof(int32_t)) != hipSuccess ||
-        hipMemcpy(c->pathWork, clear, sizeof(clear), hipMemcpyHostToDevice) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
+        hipMemcpy(c->pathWork, clear, sizeof(clear), hipMemcpyHostToDevice) != hipSuccess || stage_create(c->stage) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
     *out = c;
     return LTS_OK;
 }
@@ -838,7 +845,7 @@ void lts_destroy(lts_ctx* c) {
     (void)hipStreamSynchronize(c->stream);
     free_scene(c->scene);
     bvh_release(c->build);
-    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->pathWork, c->perm, c->xfBuf};
+    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->pathWork, c->perm, c->xfBuf, c->rayBuf};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : c->ev)
@@ -849,6 +856,7 @@ void lts_destroy(lts_ctx* c) {
             if (e) (void)hipEventDestroy(e);
         delete c->prof;
     }
+    stage_destroy(c->stage);
     wf_release(c->wf);
     nrc_release(c->nrc);
     if (c->nrcIo) (void)hipFree(c->nrcIo);
@@ -1015,31 +1023,51 @@ int lts_set_texture_filter(lts_ctx* c, int32_t mode) {
     return LTS_OK;
 }
 
-static int trace_rays_impl(lts_ctx* c, const float* rays, int32_t n, int32_t* prim, float* t) {
+constexpr size_t kRayBufKeep = (size_t)1 << 21;  // 64 MiB
+
+// Rays interleaved (dirs null: rays holds origin and direction of each), or origins and directions apart.
+static int trace_rays_impl(lts_ctx* c, const float* rays, const float* dirs, int32_t n, int32_t* prim, float* t) {
     if (!c || !rays || !prim || !t || n < 0 || n > (1 << 26)) return fail(c, LTS_E_ARG, "bad trace_rays arguments");
     if (!c->scene.loaded) return fail(c, LTS_E_STATE, "no scene loaded");
     if (n == 0) return LTS_OK;
     HIPCHK(c, hipSetDevice(c->device));
-    float* dr = nullptr;
-    float* dt = nullptr;
-    int32_t* dp = nullptr;
-    hipError_t e = hipMalloc((void**)&dr, 6 * (size_t)n * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&dt, (size_t)n * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&dp, (size_t)n * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMemcpyAsync(dr, rays, 6 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = launch_trace_rays(c->scene.view, dr, n, dp, dt, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(prim, dp, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(t, dt, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
+    if ((size_t)n > c->rayCap) {
+        if (c->rayBuf) (void)hipFree(c->rayBuf);
+        c->rayBuf = nullptr;
+        c->rayCap = 0;
+        HIPCHK(c, hipMalloc((void**)&c->rayBuf, 8 * (size_t)n * sizeof(float)));
+        c->rayCap = (size_t)n;
+    }
+    float* const dr = c->rayBuf;
+    float* const dt = dr + 6 * (size_t)n;
+    int32_t* const dp = reinterpret_cast<int32_t*>(dt + n);
+    const size_t half = 3 * (size_t)n;
+    hipError_t e = stage_to_device(c->stage, dr, rays, (dirs ? half : 2 * half) * sizeof(float), c->stream);
+    if (e == hipSuccess && dirs) e = stage_to_device(c->stage, dr + half, dirs, half * sizeof(float), c->stream);
+    if (e == hipSuccess) e = launch_trace_rays(c->scene.view, dr, dirs ? dr + half : dr + 3, dirs ? 3 : 6, n, dp, dt, c->stream);
+    if (e == hipSuccess) {
+        stage_touch(prim, (size_t)n * sizeof(int32_t));
+        stage_touch(t, (size_t)n * sizeof(float));
+        e = stage_to_host(c->stage, prim, dp, (size_t)n * sizeof(int32_t), c->stream);
+    }
+    if (e == hipSuccess) e = stage_to_host(c->stage, t, dt, (size_t)n * sizeof(float), c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (dr) (void)hipFree(dr);
-    if (dt) (void)hipFree(dt);
-    if (dp) (void)hipFree(dp);
+    if (c->rayCap > kRayBufKeep) {
+        (void)hipFree(c->rayBuf);
+        c->rayBuf = nullptr;
+        c->rayCap = 0;
+    }
     HIPCHK(c, e);
     return LTS_OK;
 }
 
 int lts_trace_rays(lts_ctx* c, const float* rays, int32_t n, int32_t* prim, float* t) {
-    return guarded(c, [&] { return trace_rays_impl(c, rays, n, prim, t); });
+    return guarded(c, [&] { return trace_rays_impl(c, rays, nullptr, n, prim, t); });
+}
+
+int lts_trace_rays_split(lts_ctx* c, const float* origins, const float* directions, int32_t n, int32_t* prim, float* t) {
+    if (!directions) return fail(c, LTS_E_ARG, "bad trace_rays arguments");
+    return guarded(c, [&] { return trace_rays_impl(c, origins, directions, n, prim, t); });
 }
 
 int lts_render_tree_info(lts_ctx* c, int32_t* kind, int32_t* depth, int32_t* nodes4) {
@@ -1178,15 +1206,20 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         HIPCHK(c, hipEventRecord(c->ev[6], s));
         HIPCHK(c, launch_film_gather(sv, rl, s));
         HIPCHK(c, hipEventRecord(c->ev[7], s));
+        if (rl.s1 == b1) {
+            HIPCHK(c, launch_get_render(sv, c->film, c->rgb, s));
+            if (rgb_out) {
+                stage_touch(rgb_out, image_bytes(sv));
+                HIPCHK(c, stage_to_host(c->stage, rgb_out, c->rgb, image_bytes(sv), s));
+            }
+        }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
         renderMs += ms_between(c->ev[5], c->ev[6]);
         resolveMs += ms_between(c->ev[6], c->ev[7]);
         launches++;
         if (sample_rgb)
-            HIPCHK(c, hipMemcpy(sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), hipMemcpyDeviceToHost));
+            HIPCHK(c, stage_to_host(c->stage, sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), s));
     }
-    HIPCHK(c, launch_get_render(sv, c->film, c->rgb, s));
-    if (rgb_out) HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, npix * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
     film_advance(c, p, b1);
     if (st) {
@@ -1423,8 +1456,7 @@ static int film_resolve_impl(lts_ctx* c, float* rgb_out) {
     const SceneView& sv = c->scene.view;
     const size_t npix = (size_t)sv.cam.width * sv.cam.height;
     HIPCHK(c, launch_get_render(sv, c->film, c->rgb, c->stream));
-    HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, npix * 3 * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, stage_to_host(c->stage, rgb_out, c->rgb, npix * 3 * sizeof(float), c->stream));
     return LTS_OK;
 }
 

@@ -99,6 +99,23 @@ hipError_t bvh_enqueue(BvhBuffers& b, const float* soup, int n, int mode, bool p
 // Mesh world transform (mesh.hip): points and normals (3 floats each, device memory) in place.
 hipError_t mesh_transform(const MeshXf& xf, float* P, int nP, float* N, int nN, hipStream_t stream);
 
+// Copies between device memory and a caller's pageable memory (host_stage.cpp): a context's pinned ring of
+// kStageSlots MiB.
+constexpr int kStageSlots = 4;
+struct HostStage {
+    char* mem = nullptr;
+    hipEvent_t ev[kStageSlots] = {};  // the last transfer through each slot
+};
+hipError_t stage_create(HostStage& st);
+void stage_destroy(HostStage& st);
+// Takes the first-touch faults of a destination that the stream's queued work will be copied to, while the
+// device is busy; contents stay as they are.
+void stage_touch(void* dst, size_t bytes);
+// Copies after the stream's earlier work; returns when dst holds the bytes.
+hipError_t stage_to_host(HostStage& st, void* dst, const void* src, size_t bytes, hipStream_t s);
+// Queues the copy on the stream; returns when src has been read.
+hipError_t stage_to_device(HostStage& st, void* dst, const void* src, size_t bytes, hipStream_t s);
+
 // Render launches (render.hip).
 struct RenderLaunch {
     int spp;
@@ -125,7 +142,9 @@ constexpr int kBdptMaxBounce = 8;
 hipError_t launch_bdpt(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);
 hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);
 hipError_t launch_film_clear(float* film, int npix, hipStream_t stream);
-hipError_t launch_trace_rays(const SceneView& sv, const float* rays, int n, int32_t* prim, float* t, hipStream_t stream);
+// ray i: origin at origins[stride i ..], direction at dirs[stride i ..]
+hipError_t launch_trace_rays(const SceneView& sv, const float* origins, const float* dirs, int stride, int n, int32_t* prim,
+                             float* t, hipStream_t stream);
 // The material of each of the n leaves of a loaded scene (shade is in leaf order) into its triangle and
 // its render record (nRecs records).
 hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t stream);

@@ -106,15 +106,17 @@ hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, Tra
 }
 
 // Closest hits of caller-given rays: the renderer's own traversal (trace_closest), one thread per
-// ray. rays[6 i ..] = origin, direction; a miss gives prim -1.
-__global__ __launch_bounds__(256) void k_trace_rays(SceneView sv, const float* __restrict__ rays, int n,
-                                                    int32_t* __restrict__ prim, float* __restrict__ tOut) {
+// ray; a miss gives prim -1.
+__global__ __launch_bounds__(256) void k_trace_rays(SceneView sv, const float* __restrict__ origins, const float* __restrict__ dirs,
+                                                    int stride, int n, int32_t* __restrict__ prim, float* __restrict__ tOut) {
     __shared__ int stk[kShortStack * 256];
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     Ray r;
-    r.o = v3(rays[6 * (size_t)i], rays[6 * (size_t)i + 1], rays[6 * (size_t)i + 2]);
-    r.d = v3(rays[6 * (size_t)i + 3], rays[6 * (size_t)i + 4], rays[6 * (size_t)i + 5]);
+    const float* o = origins + (size_t)stride * i;
+    const float* d = dirs + (size_t)stride * i;
+    r.o = v3(o[0], o[1], o[2]);
+    r.d = v3(d[0], d[1], d[2]);
     r.tMax = INFINITY;
     const Hit h = trace_closest(sv, r, lds_stack(stk, threadIdx.x, 256), nullptr, nullptr);
     int p = -1;
@@ -126,9 +128,10 @@ __global__ __launch_bounds__(256) void k_trace_rays(SceneView sv, const float* _
     tOut[i] = h.leaf >= 0 ? h.t : INFINITY;
 }
 
-hipError_t launch_trace_rays(const SceneView& sv, const float* rays, int n, int32_t* prim, float* t, hipStream_t stream) {
+hipError_t launch_trace_rays(const SceneView& sv, const float* origins, const float* dirs, int stride, int n, int32_t* prim,
+                             float* t, hipStream_t stream) {
     if (n < 1) return hipSuccess;
-    k_trace_rays<<<(n + 255) / 256, 256, 0, stream>>>(sv, rays, n, prim, t);
+    k_trace_rays<<<(n + 255) / 256, 256, 0, stream>>>(sv, origins, dirs, stride, n, prim, t);
     return hipGetLastError();
 }
 

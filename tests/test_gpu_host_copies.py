@@ -1,0 +1,50 @@
+"""Copies through the pinned ring, at the edges of its chunks.
+
+Ray queries send 12 bytes of origin and of direction for each ray and bring back 4 bytes of primitive
+and of distance: sizes of one ray, around 256 KiB (the smallest chunk), 2 MiB (from which chunks are
+1 MiB) and several turns of the ring, above the size whose device buffer is kept. Every ray's answer
+must be the one it has in a query of its own neighbourhood, whether its arrays lie together or apart.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from lighttransportsimulation_amd import scenegen
+
+
+@pytest.mark.gpu
+def test_rays_survive_the_ring(gpu_ctx, tmp_path):
+    cfg = scenegen.gen_cornell_sphere(str(tmp_path), width=16, height=16, spp=1, subdiv=2)
+    gpu_ctx.load_scene(str(tmp_path), cfg["scene"], cfg["subject"], 16, 16)
+    rng = np.random.Generator(np.random.PCG64(3))
+    for n in (1, 21844, 21846, 65536, 65537, 174763, 174764, 349526, 1048577, (1 << 21) + 1, 21846):
+        print(f"[ring {n} rays]", flush=True)
+        o = rng.uniform(-0.9, 0.9, (n, 3)).astype(np.float32)
+        d = rng.normal(size=(n, 3)).astype(np.float32)
+        prim, t = gpu_ctx.trace_rays(o, d)
+        both = np.ascontiguousarray(np.concatenate([o, d], axis=1))
+        prim2, t2 = np.full(n, -7, np.int32), np.full(n, np.nan, np.float32)
+        ptr = lambda a: a.ctypes.data_as(C.c_void_p)
+        assert gpu_ctx.lib.lts_trace_rays(gpu_ctx.h, ptr(both), n, ptr(prim2), ptr(t2)) == 0
+        assert np.array_equal(prim, prim2) and np.array_equal(t.view(np.uint32), t2.view(np.uint32))
+        for at in {0, n // 3, max(0, n - 500)}:  # a few hundred of them by themselves: one chunk
+            p, s = gpu_ctx.trace_rays(o[at:at + 500], d[at:at + 500])
+            assert np.array_equal(p, prim[at:at + 500]) and np.array_equal(s.view(np.uint32), t[at:at + 500].view(np.uint32))
+    with pytest.raises(ValueError):
+        gpu_ctx.trace_rays(np.zeros((3, 3)), np.zeros((2, 3)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,height", [(2, 2), (147, 148), (149, 149), (419, 417), (640, 575)])
+def test_images_and_samples_survive_the_ring(gpu_ctx, tmp_path, width, height):
+    """An unfiltered check of the bytes: the image of a black scene of max_bounce 0, and the samples of a
+    render against those of its halves."""
+    cfg = scenegen.gen_cornell_sphere(str(tmp_path), width=width, height=height, spp=2, subdiv=1)
+    gpu_ctx.load_scene(str(tmp_path), cfg["scene"], cfg["subject"], width, height)
+    rgb, smp, _ = gpu_ctx.render(2, 3, 2, 9, want_samples=True)
+    parts = [gpu_ctx.render(2, 3, 2, 9, want_samples=True, sample_begin=k, sample_end=k + 1) for k in (0, 1)]
+    assert np.array_equal(np.concatenate([p[1] for p in parts]).view(np.uint32), smp.view(np.uint32))
+    assert np.array_equal(parts[1][0].view(np.uint32), rgb.view(np.uint32)) and np.array_equal(gpu_ctx.film_resolve(), rgb)
+    assert (rgb.reshape(-1) != 0).mean() > 0.2
+    assert not gpu_ctx.render(2, 0, 2, 9)[0].any()

@@ -1376,13 +1376,12 @@ static int nrc_train_step_impl(lts_ctx* c, const float* raw, const float* target
         HIPCHK(c, hipMemcpyAsync(c->nrc.trainRaw, raw, (size_t)n * kNrcRaw * sizeof(float), hipMemcpyHostToDevice, s));
         HIPCHK(c, hipMemcpyAsync(c->nrc.trainTarget, target, (size_t)n * 3 * sizeof(float), hipMemcpyHostToDevice, s));
     }
-    HIPCHK(c, hipMemcpyAsync(&c->nrc.state->nTotal, &n, sizeof(int32_t), hipMemcpyHostToDevice, s));
-    HIPCHK(c, nrc_train(c->nrc, s, 1));
-    NrcState st;
-    HIPCHK(c, hipMemcpyAsync(&st, c->nrc.state, sizeof(st), hipMemcpyDeviceToHost, s));
+    HIPCHK(c, nrc_train(c->nrc, s, 1, n));
+    float last = 0.0f;
+    HIPCHK(c, hipMemcpyAsync(&last, &c->nrc.state->loss, sizeof(last), hipMemcpyDeviceToHost, s));
     if (grad) HIPCHK(c, hipMemcpyAsync(grad, c->nrc.grad, kNrcParams * sizeof(float), hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
-    if (loss) *loss = n > 0 ? st.loss : 0.0f;
+    if (loss) *loss = n > 0 ? last : 0.0f;
     return LTS_OK;
 }
 

@@ -336,6 +336,7 @@ hipError_t nrc_infer_queries(const NrcBuffers& b, const float* raw, const NrcQue
                              float* sampleL, hipStream_t stream);
 // `steps` Adam steps over the state->nTotal samples in trainRaw / trainTarget: step k trains on batch
 // (k mod ceil(nTotal / batchCap)), so steps beyond the collected batches make further passes.
-hipError_t nrc_train(const NrcBuffers& b, hipStream_t stream, int steps);
+// samples: state->nTotal, or how many there are.
+hipError_t nrc_train(const NrcBuffers& b, hipStream_t stream, int steps, int samples = -1);
 
 }  // namespace lts

@@ -85,7 +85,6 @@ struct lts_ctx {
     unsigned long long* counters = nullptr;
     int32_t* pathWork = nullptr;  // two sets of work counters of the whole-path launches, taken in turn
     int pathTurn = 0;
-    HostStage stage;
     // lts_trace_rays: rays, then hits, kept up to kRayBufKeep rays
     float* rayBuf = nullptr;
     size_t rayCap = 0;
@@ -519,6 +518,14 @@ int wavefront_pass(const lts_render_params* p, size_t pixels) {
     return p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, passPaths / pixels);
 }
 
+// Takes the first-touch faults of a destination that queued work will be copied to, while the device is busy;
+// its contents stay as they are.
+void touch_pages(void* dst, size_t bytes) {
+    volatile char* p = static_cast<volatile char*>(dst);
+    for (size_t i = 0; i < bytes; i += 4096) p[i] = p[i];
+    if (bytes) p[bytes - 1] = p[bytes - 1];
+}
+
 size_t image_bytes(const SceneView& sv) { return (size_t)sv.cam.width * sv.cam.height * 3 * sizeof(float); }
 
 // The wavefront integrator over one or more scenes, executed on c's stream and buffers.
@@ -648,9 +655,9 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             // the images' copies wait on the device, behind the last pass
             for (size_t i = 0; i < scenes.size(); i++) HIPCHK(c, launch_get_render(views[i], scenes[i]->film, scenes[i]->rgb, s));
             for (size_t i = 0; rgb_out && i < scenes.size(); i++)
-                if (rgb_out[i]) stage_touch(rgb_out[i], image_bytes(views[i]));
+                if (rgb_out[i]) touch_pages(rgb_out[i], image_bytes(views[i]));
             for (size_t i = 0; rgb_out && i < scenes.size(); i++)
-                if (rgb_out[i]) HIPCHK(c, stage_to_host(c->stage, rgb_out[i], scenes[i]->rgb, image_bytes(views[i]), s));
+                if (rgb_out[i]) HIPCHK(c, hipMemcpyAsync(rgb_out[i], scenes[i]->rgb, image_bytes(views[i]), hipMemcpyDeviceToHost, s));
         }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
         renderMs += ms_between(c->ev[5], c->ev[6]);
@@ -673,7 +680,7 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             }
         }
         if (sample_rgb)
-            HIPCHK(c, stage_to_host(c->stage, sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), s));
+            HIPCHK(c, hipMemcpyAsync(sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
     }
     for (lts_ctx* x : scenes) film_advance(x, p, b1);
     HIPCHK(c, hipStreamSynchronize(s));
@@ -834,7 +841,7 @@ int lts_create(lts_ctx** out, int dev) {
     const int32_t clear[2 * kPathWork] = {};
     if (hipMalloc((void**)&c->counters, kTraceCounters * sizeof(unsigned long long)) != hipSuccess ||
         hipMalloc((void**)&c->pathWork, 2 * kPathWork * sizeof(int32_t)) != hipSuccess ||
-        hipMemcpy(c->pathWork, clear, sizeof(clear), hipMemcpyHostToDevice) != hipSuccess || stage_create(c->stage) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
+        hipMemcpy(c->pathWork, clear, sizeof(clear), hipMemcpyHostToDevice) != hipSuccess) { lts_destroy(c); return LTS_E_HIP; }
     *out = c;
     return LTS_OK;
 }
@@ -856,7 +863,6 @@ void lts_destroy(lts_ctx* c) {
             if (e) (void)hipEventDestroy(e);
         delete c->prof;
     }
-    stage_destroy(c->stage);
     wf_release(c->wf);
     nrc_release(c->nrc);
     if (c->nrcIo) (void)hipFree(c->nrcIo);
@@ -1042,15 +1048,15 @@ static int trace_rays_impl(lts_ctx* c, const float* rays, const float* dirs, int
     float* const dt = dr + 6 * (size_t)n;
     int32_t* const dp = reinterpret_cast<int32_t*>(dt + n);
     const size_t half = 3 * (size_t)n;
-    hipError_t e = stage_to_device(c->stage, dr, rays, (dirs ? half : 2 * half) * sizeof(float), c->stream);
-    if (e == hipSuccess && dirs) e = stage_to_device(c->stage, dr + half, dirs, half * sizeof(float), c->stream);
+    hipError_t e = hipMemcpyAsync(dr, rays, (dirs ? half : 2 * half) * sizeof(float), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess && dirs) e = hipMemcpyAsync(dr + half, dirs, half * sizeof(float), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = launch_trace_rays(c->scene.view, dr, dirs ? dr + half : dr + 3, dirs ? 3 : 6, n, dp, dt, c->stream);
     if (e == hipSuccess) {
-        stage_touch(prim, (size_t)n * sizeof(int32_t));
-        stage_touch(t, (size_t)n * sizeof(float));
-        e = stage_to_host(c->stage, prim, dp, (size_t)n * sizeof(int32_t), c->stream);
+        touch_pages(prim, (size_t)n * sizeof(int32_t));
+        touch_pages(t, (size_t)n * sizeof(float));
+        e = hipMemcpyAsync(prim, dp, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
     }
-    if (e == hipSuccess) e = stage_to_host(c->stage, t, dt, (size_t)n * sizeof(float), c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(t, dt, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (c->rayCap > kRayBufKeep) {
         (void)hipFree(c->rayBuf);
@@ -1209,8 +1215,8 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         if (rl.s1 == b1) {
             HIPCHK(c, launch_get_render(sv, c->film, c->rgb, s));
             if (rgb_out) {
-                stage_touch(rgb_out, image_bytes(sv));
-                HIPCHK(c, stage_to_host(c->stage, rgb_out, c->rgb, image_bytes(sv), s));
+                touch_pages(rgb_out, image_bytes(sv));
+                HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, image_bytes(sv), hipMemcpyDeviceToHost, s));
             }
         }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
@@ -1218,7 +1224,7 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         resolveMs += ms_between(c->ev[6], c->ev[7]);
         launches++;
         if (sample_rgb)
-            HIPCHK(c, stage_to_host(c->stage, sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), s));
+            HIPCHK(c, hipMemcpyAsync(sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
     }
     HIPCHK(c, hipStreamSynchronize(s));
     film_advance(c, p, b1);
@@ -1455,7 +1461,8 @@ static int film_resolve_impl(lts_ctx* c, float* rgb_out) {
     const SceneView& sv = c->scene.view;
     const size_t npix = (size_t)sv.cam.width * sv.cam.height;
     HIPCHK(c, launch_get_render(sv, c->film, c->rgb, c->stream));
-    HIPCHK(c, stage_to_host(c->stage, rgb_out, c->rgb, npix * 3 * sizeof(float), c->stream));
+    HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, npix * 3 * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     return LTS_OK;
 }
 

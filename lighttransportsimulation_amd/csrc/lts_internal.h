@@ -99,23 +99,6 @@ hipError_t bvh_enqueue(BvhBuffers& b, const float* soup, int n, int mode, bool p
 // Mesh world transform (mesh.hip): points and normals (3 floats each, device memory) in place.
 hipError_t mesh_transform(const MeshXf& xf, float* P, int nP, float* N, int nN, hipStream_t stream);
 
-// Copies between device memory and a caller's pageable memory (host_stage.cpp): a context's pinned ring of
-// kStageSlots MiB.
-constexpr int kStageSlots = 4;
-struct HostStage {
-    char* mem = nullptr;
-    hipEvent_t ev[kStageSlots] = {};  // the last transfer through each slot
-};
-hipError_t stage_create(HostStage& st);
-void stage_destroy(HostStage& st);
-// Takes the first-touch faults of a destination that the stream's queued work will be copied to, while the
-// device is busy; contents stay as they are.
-void stage_touch(void* dst, size_t bytes);
-// Copies after the stream's earlier work; returns when dst holds the bytes.
-hipError_t stage_to_host(HostStage& st, void* dst, const void* src, size_t bytes, hipStream_t s);
-// Queues the copy on the stream; returns when src has been read.
-hipError_t stage_to_device(HostStage& st, void* dst, const void* src, size_t bytes, hipStream_t s);
-
 // Render launches (render.hip).
 struct RenderLaunch {
     int spp;

@@ -1587,18 +1587,14 @@ int lts_bvh_build_static(const float* d_tri_xyz, int32_t n, int32_t mode, uint32
     void* scratch = nullptr;
     if (bvh_static_scratch(dev, &scratch) != hipSuccess) return LTS_E_HIP;
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
-    int32_t* dStatus = nullptr;
     uint32_t* dKeys = nullptr;
     if (bvh_enqueue_static(scratch, d_tri_xyz, n, mode, d_codes_sorted, d_perm, d_left, d_right, d_parent, d_bounds, s,
-                           &dStatus, &dKeys) != hipSuccess)
+                           &dKeys) != hipSuccess)
         return LTS_E_HIP;
-    int32_t status = 0;
-    uint32_t keys[6];
-    if (hipMemcpyAsync(&status, dStatus, sizeof(status), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        (scene_bounds && hipMemcpyAsync(keys, dKeys, sizeof(keys), hipMemcpyDeviceToHost, s) != hipSuccess) ||
-        hipStreamSynchronize(s) != hipSuccess)
+    uint32_t keys[7];  // the scene-bound keys and the status
+    if (hipMemcpyAsync(keys, dKeys, sizeof(keys), hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
         return LTS_E_HIP;
-    if (status != 0) return LTS_E_STATE;
+    if (keys[6] != 0) return LTS_E_STATE;
     if (scene_bounds)
         for (int a = 0; a < 6; a++) {
             const uint32_t u = (keys[a] & 0x80000000u) ? (keys[a] & 0x7fffffffu) : ~keys[a];

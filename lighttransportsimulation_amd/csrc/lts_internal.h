@@ -84,11 +84,11 @@ constexpr int kStaticMaxDevices = 64;
 hipError_t bvh_static_scratch(int device, void** ptr);
 // Enqueues a build of n <= kStaticMaxPrims primitives whose results go to the caller's device arrays
 // (sorted codes, permutation, children, parents, unified node bounds) and whose temporaries live
-// in the static buffer; *status and *sceneKeys point at the build's status word and scene-bound
-// keys inside that buffer.
+// in the static buffer; *keysAndStatus points at the build's six scene-bound keys and, behind them,
+// its status word inside that buffer.
 hipError_t bvh_enqueue_static(void* scratch, const float* soup, int n, int mode, uint32_t* codesSorted, int32_t* perm,
                               int32_t* left, int32_t* right, int32_t* parent, float* bounds, hipStream_t s,
-                              int32_t** status, uint32_t** sceneKeys);
+                              uint32_t** keysAndStatus);
 
 // Enqueues the whole build on `stream`. `soup` is a device pointer to n*9 floats.
 // mode 0: leaf k holds primitive k (reference); mode 1: leaf k holds perm[k].

@@ -85,9 +85,6 @@ struct lts_ctx {
     unsigned long long* counters = nullptr;
     int32_t* pathWork = nullptr;  // two sets of work counters of the whole-path launches, taken in turn
     int pathTurn = 0;
-    // lts_trace_rays: rays, then hits, kept up to kRayBufKeep rays
-    float* rayBuf = nullptr;
-    size_t rayCap = 0;
     int* perm = nullptr;  // Perlin permutation (512 ints)
     hipEvent_t ev[8] = {};
     // wavefront integrator
@@ -518,14 +515,6 @@ int wavefront_pass(const lts_render_params* p, size_t pixels) {
     return p->spp_per_pass > 0 ? p->spp_per_pass : (int)std::max<size_t>(1, passPaths / pixels);
 }
 
-// Takes the first-touch faults of a destination that queued work will be copied to, while the device is busy;
-// its contents stay as they are.
-void touch_pages(void* dst, size_t bytes) {
-    volatile char* p = static_cast<volatile char*>(dst);
-    for (size_t i = 0; i < bytes; i += 4096) p[i] = p[i];
-    if (bytes) p[bytes - 1] = p[bytes - 1];
-}
-
 size_t image_bytes(const SceneView& sv) { return (size_t)sv.cam.width * sv.cam.height * 3 * sizeof(float); }
 
 // The wavefront integrator over one or more scenes, executed on c's stream and buffers.
@@ -651,14 +640,6 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             HIPCHK(c, launch_film_gather(views[i], rl, s));
         }
         HIPCHK(c, hipEventRecord(c->ev[7], s));
-        if (s1 == b1) {
-            // the images' copies wait on the device, behind the last pass
-            for (size_t i = 0; i < scenes.size(); i++) HIPCHK(c, launch_get_render(views[i], scenes[i]->film, scenes[i]->rgb, s));
-            for (size_t i = 0; rgb_out && i < scenes.size(); i++)
-                if (rgb_out[i]) touch_pages(rgb_out[i], image_bytes(views[i]));
-            for (size_t i = 0; rgb_out && i < scenes.size(); i++)
-                if (rgb_out[i]) HIPCHK(c, hipMemcpyAsync(rgb_out[i], scenes[i]->rgb, image_bytes(views[i]), hipMemcpyDeviceToHost, s));
-        }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
         renderMs += ms_between(c->ev[5], c->ev[6]);
         resolveMs += ms_between(c->ev[6], c->ev[7]);
@@ -680,9 +661,14 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
             }
         }
         if (sample_rgb)
-            HIPCHK(c, hipMemcpyAsync(sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
+            HIPCHK(c, hipMemcpy(sample_rgb, c->sampleL, (size_t)paths * 3 * sizeof(float), hipMemcpyDeviceToHost));
     }
-    for (lts_ctx* x : scenes) film_advance(x, p, b1);
+    for (size_t i = 0; i < scenes.size(); i++) {
+        lts_ctx* x = scenes[i];
+        HIPCHK(c, launch_get_render(views[i], x->film, x->rgb, s));
+        film_advance(x, p, b1);
+        if (rgb_out && rgb_out[i]) HIPCHK(c, hipMemcpyAsync(rgb_out[i], x->rgb, image_bytes(views[i]), hipMemcpyDeviceToHost, s));
+    }
     HIPCHK(c, hipStreamSynchronize(s));
     if (st) {
         std::memset(st, 0, sizeof(*st));
@@ -852,7 +838,7 @@ void lts_destroy(lts_ctx* c) {
     (void)hipStreamSynchronize(c->stream);
     free_scene(c->scene);
     bvh_release(c->build);
-    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->pathWork, c->perm, c->xfBuf, c->rayBuf};
+    void* ps[] = {c->buildSoup, c->sampleL, c->film, c->rgb, c->counters, c->pathWork, c->perm, c->xfBuf};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : c->ev)
@@ -1029,40 +1015,28 @@ int lts_set_texture_filter(lts_ctx* c, int32_t mode) {
     return LTS_OK;
 }
 
-constexpr size_t kRayBufKeep = (size_t)1 << 21;  // 64 MiB
-
 // Rays interleaved (dirs null: rays holds origin and direction of each), or origins and directions apart.
 static int trace_rays_impl(lts_ctx* c, const float* rays, const float* dirs, int32_t n, int32_t* prim, float* t) {
     if (!c || !rays || !prim || !t || n < 0 || n > (1 << 26)) return fail(c, LTS_E_ARG, "bad trace_rays arguments");
     if (!c->scene.loaded) return fail(c, LTS_E_STATE, "no scene loaded");
     if (n == 0) return LTS_OK;
     HIPCHK(c, hipSetDevice(c->device));
-    if ((size_t)n > c->rayCap) {
-        if (c->rayBuf) (void)hipFree(c->rayBuf);
-        c->rayBuf = nullptr;
-        c->rayCap = 0;
-        HIPCHK(c, hipMalloc((void**)&c->rayBuf, 8 * (size_t)n * sizeof(float)));
-        c->rayCap = (size_t)n;
-    }
-    float* const dr = c->rayBuf;
-    float* const dt = dr + 6 * (size_t)n;
-    int32_t* const dp = reinterpret_cast<int32_t*>(dt + n);
     const size_t half = 3 * (size_t)n;
-    hipError_t e = hipMemcpyAsync(dr, rays, (dirs ? half : 2 * half) * sizeof(float), hipMemcpyHostToDevice, c->stream);
+    float* dr = nullptr;
+    float* dt = nullptr;
+    int32_t* dp = nullptr;
+    hipError_t e = hipMalloc((void**)&dr, 2 * half * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&dt, (size_t)n * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&dp, (size_t)n * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMemcpyAsync(dr, rays, (dirs ? half : 2 * half) * sizeof(float), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess && dirs) e = hipMemcpyAsync(dr + half, dirs, half * sizeof(float), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = launch_trace_rays(c->scene.view, dr, dirs ? dr + half : dr + 3, dirs ? 3 : 6, n, dp, dt, c->stream);
-    if (e == hipSuccess) {
-        touch_pages(prim, (size_t)n * sizeof(int32_t));
-        touch_pages(t, (size_t)n * sizeof(float));
-        e = hipMemcpyAsync(prim, dp, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
-    }
+    if (e == hipSuccess) e = hipMemcpyAsync(prim, dp, (size_t)n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(t, dt, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (c->rayCap > kRayBufKeep) {
-        (void)hipFree(c->rayBuf);
-        c->rayBuf = nullptr;
-        c->rayCap = 0;
-    }
+    if (dr) (void)hipFree(dr);
+    if (dt) (void)hipFree(dt);
+    if (dp) (void)hipFree(dp);
     HIPCHK(c, e);
     return LTS_OK;
 }
@@ -1212,20 +1186,15 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         HIPCHK(c, hipEventRecord(c->ev[6], s));
         HIPCHK(c, launch_film_gather(sv, rl, s));
         HIPCHK(c, hipEventRecord(c->ev[7], s));
-        if (rl.s1 == b1) {
-            HIPCHK(c, launch_get_render(sv, c->film, c->rgb, s));
-            if (rgb_out) {
-                touch_pages(rgb_out, image_bytes(sv));
-                HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, image_bytes(sv), hipMemcpyDeviceToHost, s));
-            }
-        }
         HIPCHK(c, hipEventSynchronize(c->ev[7]));
         renderMs += ms_between(c->ev[5], c->ev[6]);
         resolveMs += ms_between(c->ev[6], c->ev[7]);
         launches++;
         if (sample_rgb)
-            HIPCHK(c, hipMemcpyAsync(sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
+            HIPCHK(c, hipMemcpy(sample_rgb, c->sampleL, npix * (size_t)(rl.s1 - rl.s0) * 3 * sizeof(float), hipMemcpyDeviceToHost));
     }
+    HIPCHK(c, launch_get_render(sv, c->film, c->rgb, s));
+    if (rgb_out) HIPCHK(c, hipMemcpyAsync(rgb_out, c->rgb, image_bytes(sv), hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
     film_advance(c, p, b1);
     if (st) {

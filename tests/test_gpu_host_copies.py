@@ -1,9 +1,8 @@
 """Results and ray queries between host and device.
 
 Ray queries send 12 bytes of origin and of direction for each ray and bring back 4 bytes of primitive
-and of distance: sizes of one ray, of some KiB to tens of MiB, and above the size whose device buffer
-is kept. Every ray's answer must be the one it has in a query of its own neighbourhood, whether its
-arrays lie together or apart.
+and of distance: sizes of one ray and of some KiB to tens of MiB. Every ray's answer must be the one
+it has in a query of its own neighbourhood, whether its arrays lie together or apart.
 """
 import ctypes as C
 

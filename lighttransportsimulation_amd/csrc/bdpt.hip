@@ -137,19 +137,6 @@ LTS_D float vertex_pdf(const BVertex& v, const BVertex* prev, const BVertex& nex
     return to_area(pdf, v, next);
 }
 
-LTS_D SurfacePoint as_point(const BVertex& v) {
-    SurfacePoint s;
-    s.p = v.p; s.pError = v.pError; s.n = v.n;
-    return s;
-}
-
-// Mutual visibility of two surface vertices (VisibilityTester between their interactions).
-LTS_D bool visible(const SceneView& sv, const BVertex& a, const BVertex& b, TraceStack ts) {
-    LightPoint lp;
-    lp.p = b.p; lp.n = b.n; lp.pError = b.pError;
-    return unoccluded(sv, as_point(a), lp, ts);
-}
-
 // A surface vertex from a closest hit.
 LTS_D void surface_vertex(const SceneView& sv, BVertex& v, const SurfacePoint& si, const NoiseTables& perm) {
     v.kind = kVSurface;
@@ -162,11 +149,19 @@ LTS_D void surface_vertex(const SceneView& sv, BVertex& v, const SurfacePoint& s
 // Random walk from `ray` (PBRT-v3 RandomWalk): appends vertices path[k0..] until maxVerts, a miss
 // or an absorbed sample. pdfDir is the solid-angle density the ray's direction was sampled with.
 // Camera walks record an escape as a vertex of the infinite light.
-LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool importance, BVertex* path, int k0,
-               int maxVerts, const Sampler& smp, uint32_t block, TraceStack ts, const NoiseTables& perm, const CameraSample* cs, int spp) {
+// The lanes of a wave walk in step, so that their rays are traced together and their vertices, in private
+// memory, are read at the same index; `going`: the lane has a ray (others return k0).
+LTS_D int walk(const SceneView& sv, bool going, Ray ray, Spec beta, float pdfDir, bool importance, BVertex* path, int k0,
+               int maxVerts, const Sampler& smp, uint32_t block, int* lds, const NoiseTables& perm, const CameraSample* cs, int spp) {
     int k = k0;
-    while (k < maxVerts) {
-        Hit h = trace_closest(sv, ray, ts, nullptr, nullptr);
+    going = going && k < maxVerts;
+    while (__ballot(going)) {
+        RayQuery q;
+        q.kind = going ? kRayClosest : kRayNone;
+        q.o = ray.o; q.d = ray.d; q.tMax = INFINITY;
+        const RayAnswer h = trace_wave(sv, q, lds);
+        if (!going) continue;
+        going = false;
         BVertex& v = path[k];
         BVertex& prev = path[k - 1];
         if (h.leaf < 0) {
@@ -181,7 +176,7 @@ LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool impor
                 v.bsdf.kind = -1;
                 k++;
             }
-            break;
+            continue;
         }
         SurfacePoint si = make_surface(sv, h.leaf, ray, h.u, h.v, h.invDet);
         if (cs && k == 1) camera_footprint(sv, si, *cs, spp, ray, h.invDet);
@@ -189,14 +184,14 @@ LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool impor
         v.beta = beta;
         v.pdfFwd = to_area(pdfDir, prev, v);
         v.pdfRev = 0.0f;
-        if (++k >= maxVerts) break;
+        if (++k >= maxVerts) continue;
         float u[4];
         smp.block(block + (uint32_t)k, u);
         V3 wi;
         float pdf = 0.0f;
         int type = 0;
         Spec f = v.bsdf.sampleF(v.wo, &wi, v2(u[0], u[1]), &pdf, B_ALL, &type);
-        if (pdf == 0 || isBlack(f)) break;
+        if (pdf == 0 || isBlack(f)) continue;
         if (importance && v.bsdf.kind == 3 && (type & B_TRANS)) {
             // sampleF scales refracted radiance by (etaI / etaT)^2; importance is not scaled
             const bool entering = cosT(v.bsdf.toLocal(v.wo)) > 0;
@@ -212,6 +207,7 @@ LTS_D int walk(const SceneView& sv, Ray ray, Spec beta, float pdfDir, bool impor
         prev.pdfRev = to_area(pdfRev, v, prev);
         pdfDir = pdf;
         ray = spawn_ray(si, wi);
+        going = true;
     }
     return k;
 }
@@ -226,8 +222,8 @@ LTS_D SurfacePoint light_point(const SceneView& sv, const LightDesc& L, V2 u) {
     return make_surface(sv, L.leaf, dummy, b1, 1 - b0 - b1, 1.0f);
 }
 
-LTS_D int light_subpath(const SceneView& sv, BVertex* path, const Sampler& smp, int maxVerts, TraceStack ts,
-                        const NoiseTables& perm) {
+// Starts a light subpath: its first vertex, and the ray of its walk. Returns the vertices, 0 or 1.
+LTS_D int light_start(const SceneView& sv, BVertex* path, const Sampler& smp, int maxVerts, Ray& r, Spec& beta, float& pdfDir) {
     if (sv.nLights == 0 || maxVerts < 1) return 0;
     float u0[4], u1[4];
     smp.block(kBlockLightStart, u0);
@@ -243,7 +239,7 @@ LTS_D int light_subpath(const SceneView& sv, BVertex* path, const Sampler& smp, 
     coordinateSystem(lp.n, &a, &b);
     const V3 wl = cosine_hemisphere(v2(u0[3], u1[0]));
     const V3 w = a * wl.x + b * wl.y + lp.n * wl.z;
-    const float pdfDir = wl.z * INV_PI_F;
+    pdfDir = wl.z * INV_PI_F;
     if (pdfDir == 0) return 0;
     BVertex& v = path[0];
     v.kind = kVLight;
@@ -255,12 +251,11 @@ LTS_D int light_subpath(const SceneView& sv, BVertex* path, const Sampler& smp, 
     v.pdfFwd = pick / L.area;
     v.pdfRev = 0.0f;
     // Le |cos| / (pick pdfPos pdfDir), with pdfPos = 1 / area and pdfDir = cos / pi
-    const Spec beta = light_le(L) * (PI_F * L.area / pick);
-    Ray r;
+    beta = light_le(L) * (PI_F * L.area / pick);
     r.o = offsetRayOrigin(lp.p, lp.pError, lp.n, w);
     r.d = w;
     r.tMax = INFINITY;
-    return walk(sv, r, beta, pdfDir, true, path, 1, maxVerts, smp, kBlockLightWalk, ts, perm, nullptr, 0);
+    return 1;
 }
 
 LTS_D float remap0(float f) { return f != 0 ? f : 1.0f; }
@@ -301,13 +296,19 @@ LTS_D float mis_weight(const SceneView& sv, const BVertex* lp, const BVertex* cp
     return 1.0f / (1.0f + sum);
 }
 
-// Contribution of strategy (s, t), MIS-weighted (PBRT-v3 ConnectBDPT without t = 1).
-LTS_D Spec connect(const SceneView& sv, const BVertex* lp, const BVertex* cp, int s, int t, const Sampler& smp,
-                   TraceStack ts) {
+// Contribution of strategy (s, t) before its MIS weight (PBRT-v3 ConnectBDPT without t = 1). When it takes the
+// mutual visibility of two surface vertices (VisibilityTester between their interactions), `open` is false and
+// (o, d) the shadow ray of it, to 1 - SHADOW_EPS. sampled: the light vertex of an s = 1 connection.
+LTS_D Spec connect(const SceneView& sv, const BVertex* lp, const BVertex* cp, BVertex& sampled, int s, int t, const Sampler& smp,
+                   bool& open, V3& o, V3& d) {
+    open = true;
+    auto shadow = [&](const BVertex& a, const BVertex& b) {
+        o = offsetRayOrigin(a.p, a.pError, a.n, b.p - a.p);
+        d = offsetRayOrigin(b.p, b.pError, b.n, o - b.p) - o;
+        open = false;
+    };
     const BVertex& pt = cp[t - 1];
     Spec L = spec(0.0f);
-    BVertex sampled;
-    sampled.kind = -1;
     if (s == 0) {
         if (pt.kind == kVEscape) {
             for (int l = 0; l < sv.nLights; l++)
@@ -337,40 +338,40 @@ LTS_D Spec connect(const SceneView& sv, const BVertex* lp, const BVertex* cp, in
         sampled.bsdf.kind = -1;
         sampled.pdfFwd = pick / Ld.area;
         sampled.pdfRev = 0.0f;
-        V3 d = sampled.p - pt.p;
-        const float d2 = lengthSq(d);
+        V3 w = sampled.p - pt.p;
+        const float d2 = lengthSq(w);
         if (d2 == 0) return spec(0.0f);
-        d = d * (1 / sqrtf(d2));
-        const Spec Le = emitted(sv, sampled, -d);
+        w = w * (1 / sqrtf(d2));
+        const Spec Le = emitted(sv, sampled, -w);
         if (isBlack(Le)) return spec(0.0f);
-        const float G = absDot(pt.sn, d) * absDot(sampled.n, d) / d2;
+        const float G = absDot(pt.sn, w) * absDot(sampled.n, w) / d2;
         L = pt.beta * vertex_f(pt, sampled, false) * Le * (G / sampled.pdfFwd);
-        if (!isBlack(L) && !visible(sv, pt, sampled, ts)) L = spec(0.0f);
+        if (!isBlack(L)) shadow(pt, sampled);
     } else {
         const BVertex& qs = lp[s - 1];
         if (!connectible(qs)) return spec(0.0f);
-        V3 d = qs.p - pt.p;
-        const float d2 = lengthSq(d);
+        V3 w = qs.p - pt.p;
+        const float d2 = lengthSq(w);
         if (d2 == 0) return spec(0.0f);
-        d = d * (1 / sqrtf(d2));
+        w = w * (1 / sqrtf(d2));
         L = qs.beta * vertex_f(qs, pt, true) * vertex_f(pt, qs, false) * pt.beta;
         if (isBlack(L)) return L;
-        const float G = absDot(pt.sn, d) * absDot(qs.sn, d) / d2;
+        const float G = absDot(pt.sn, w) * absDot(qs.sn, w) / d2;
         L = L * G;
-        if (!visible(sv, pt, qs, ts)) L = spec(0.0f);
+        shadow(pt, qs);
     }
-    if (isBlack(L)) return L;
-    return L * mis_weight(sv, lp, cp, sampled, s, t);
+    return L;
 }
 
-LTS_D Spec bdpt_radiance(const SceneView& sv, int px, int py, int sample, const RenderLaunch& rl, TraceStack ts,
+// Run by all lanes of a wave; inside: the lane has a sample.
+LTS_D Spec bdpt_radiance(const SceneView& sv, bool inside, int px, int py, int sample, const RenderLaunch& rl, int* lds,
                          const NoiseTables& perm) {
     Sampler smp;
     smp.seed = rl.seed;
     smp.pixel = (uint32_t)(py * sv.cam.width + px);
     smp.sample = (uint32_t)sample;
     const int maxBounce = rl.maxBounce;
-    BVertex cp[kCamVerts], lp[kLightVerts];
+    BVertex cp[kCamVerts], lp[kLightVerts], sampled;
     const CameraSample cs = camera_sample(sv, px, py, sample, rl.spp, rl.stratified, rl.seed);
     const Ray camRay = camera_ray(sv, cs);
     BVertex& c0 = cp[0];
@@ -383,21 +384,43 @@ LTS_D Spec bdpt_radiance(const SceneView& sv, int px, int py, int sample, const 
     c0.delta = false;
     c0.bsdf.kind = -1;
     // pdfDir of the camera ray only feeds the t = 1 strategies, which are not used
-    const int nCam = walk(sv, camRay, spec(1.0f), 0.0f, false, cp, 1, maxBounce + 2, smp, kBlockCamWalk, ts, perm, &cs, rl.spp);
-    const int nLight = light_subpath(sv, lp, smp, maxBounce + 1, ts, perm);
+    const int nCam = walk(sv, inside, camRay, spec(1.0f), 0.0f, false, cp, 1, maxBounce + 2, smp, kBlockCamWalk, lds, perm, &cs, rl.spp);
+    Ray lightRay;
+    Spec beta;
+    float pdfDir = 0.0f;
+    // a light subpath only matters to a camera subpath that it can be connected to
+    bool connects = false;
+    for (int t = 2; t <= nCam; t++) connects = connects || connectible(cp[t - 1]);
+    int nLight = inside && connects ? light_start(sv, lp, smp, maxBounce + 1, lightRay, beta, pdfDir) : 0;
+    nLight = walk(sv, nLight > 0, lightRay, beta, pdfDir, true, lp, nLight, maxBounce + 1, smp, kBlockLightWalk, lds, perm, nullptr, 0);
     Spec L = spec(0.0f);
-    for (int t = 2; t <= nCam; t++)
-        for (int s = 0; s <= nLight; s++) {
-            if (s + t - 2 > maxBounce) break;
-            L = L + connect(sv, lp, cp, s, t, smp, ts);
+    for (int t = 2; __ballot(t <= nCam); t++)
+        for (int s = 0; __ballot(t <= nCam && s <= nLight) && s + t - 2 <= maxBounce; s++) {
+            RayQuery q;
+            q.kind = kRayNone;
+            bool open = true;
+            Spec C = spec(0.0f);
+            if (t <= nCam && s <= nLight) {
+                C = connect(sv, lp, cp, sampled, s, t, smp, open, q.o, q.d);
+                if (!open) {
+                    q.kind = kRayShadow;
+                    q.tMax = 1 - SHADOW_EPS;
+                }
+            }
+            if (__ballot(!open) && trace_wave(sv, q, lds).blocked) C = spec(0.0f);
+            if (!isBlack(C)) L = L + C * mis_weight(sv, lp, cp, sampled, s, t);
         }
     return L;
 }
 
-// Four waves per SIMD (128 VGPRs): 32.4 ms per 4-spp frame of the 1M-triangle displaced sphere at
-// 1920x1080, against 38.0 ms at the three waves its natural 165 VGPRs allow and 34.3 ms at five.
+// A wave's 64 samples go through walks and strategies in step: their vertices, in private memory, are read at
+// the same index, and their rays are traced together (a ray at a time with every lane waiting for the longest,
+// and a light subpath for every sample: 4.18 ms for a 4-spp 641x361 frame of a 90k-triangle torus and 12.7 for
+// 16 spp, now 3.27 and 9.7; lanes that go on by themselves, as in whole paths: 7.2). It is bound by vector
+// instructions with a quarter of the lanes at work, as subpaths differ in length. Four waves per SIMD (128
+// VGPRs): 3.27 ms, 3.78 at three and 3.27 at five, where a spilling frame's memory grows.
 __global__ __launch_bounds__(256, 4) void k_bdpt(SceneView sv, RenderLaunch rl) {
-    __shared__ int stk[kShortStack * 256];
+    __shared__ int lds[4][kWaveTraceWords];
     __shared__ NoiseTables perm;
     noise_tables(perm, sv.perm, threadIdx.x, 256);
     __syncthreads();
@@ -407,8 +430,9 @@ __global__ __launch_bounds__(256, 4) void k_bdpt(SceneView sv, RenderLaunch rl) 
     const int px = (tile % tilesX) * kTileSide + (threadIdx.x & (kTileSide - 1));
     const int py = (tile / tilesX) * kTileSide + (threadIdx.x / kTileSide);
     const int sample = rl.s0 + blockIdx.y;
-    if (px >= W || py >= H || sample >= rl.s1) return;
-    Spec L = bdpt_radiance(sv, px, py, sample, rl, lds_stack(stk, threadIdx.x, 256), perm);
+    const bool inside = px < W && py < H && sample < rl.s1;
+    const Spec L = bdpt_radiance(sv, inside, px, py, sample, rl, lds[threadIdx.x >> 6], perm);
+    if (!inside) return;
     float* o = rl.sampleL + 3 * ((size_t)blockIdx.y * W * H + (size_t)py * W + px);
     o[0] = L.r; o[1] = L.g; o[2] = L.b;
 }

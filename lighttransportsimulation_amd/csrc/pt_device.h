@@ -12,11 +12,6 @@ struct Ray {
     float tMax;
 };
 
-struct Hit {
-    int leaf;   // leaf index of the closest triangle, -1 for a miss
-    float t, u, v, invDet;
-};
-
 struct SurfacePoint {
     V3 p, pError, wo, n;
     V2 uv;
@@ -79,22 +74,6 @@ LTS_D bool tri_hit(V3 p0, V3 p1, V3 p2, const Ray& r, float& t, float& u, float&
     return tri_mt(p0, p1, p2, r, kOneMinusEpsF, t, u, v, invDetOut) && t > 0 && t < r.tMax;
 }
 
-// The closest-hit acceptance of leaf `leaf` against the current closest hit (distance r.tMax, leaf
-// best): nearer, or exactly as near with a lower leaf index. BVH::intersect (BVH.cuh:365-398) keeps
-// the first triangle it meets at the closest distance, and its depth-first, left-first walk meets
-// the leaves in index order, so of several triangles at exactly that distance the lowest leaf wins;
-// this rule gives the same winner in any visiting order.
-LTS_D bool tri_hit_closest(V3 p0, V3 p1, V3 p2, const Ray& r, int leaf, int best, float& t, float& u, float& v,
-                           float& invDetOut) {
-    return tri_mt(p0, p1, p2, r, kOneMinusEpsF, t, u, v, invDetOut) && t > 0 && (t < r.tMax || (t == r.tMax && leaf < best));
-}
-
-// Triangle::simpleIntersect (shapes/Triangle.cu:50-84)
-LTS_D bool tri_occludes(V3 p0, V3 p1, V3 p2, const Ray& r) {
-    float t, u, v, invDet;
-    return tri_mt(p0, p2, p1, r, kOnePlusEpsF, t, u, v, invDet) && t > 0 && t < r.tMax;
-}
-
 // Bounds3::simpleIntersect (geometry/Bound.cuh:200-227); also returns the entry distance.
 LTS_D bool box_hit(const float* mn, const float* mx, const Ray& r, V3 inv, int nx, int ny, int nz, float& tEnter) {
     const float g3 = 1 + 2 * gammaN(3);
@@ -148,12 +127,6 @@ struct TraceStack {
 // LDS stack of thread `tid` in a block-wide array __shared__ int[kShortStack * blockSize].
 LTS_D TraceStack lds_stack(int* shared, int tid, int blockSize) { return TraceStack{shared + tid, blockSize}; }
 
-// Render-node fetches and triangle tests of one lane's traversals (counting launches only; the
-// timed kernels are instantiated without it).
-struct TraceTally {
-    unsigned long long nodes = 0, tris = 0;
-};
-
 // 1 / d by v_rcp_f32 (within 1 ulp) with its magnitude held to 2^100, for the node test only: a
 // zero direction component gives slab distances that are hugely negative or positive, never NaN.
 LTS_D float slab_inverse(float d) { return __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(d), -0x1p100f, 0x1p100f); }
@@ -187,7 +160,7 @@ LTS_D void trace_pop(TraceLane& l, TraceStack ts, const int* spill) {
 // One node of the 4-wide render tree (BVH::intersect / BVH::simpleIntersect, acceleration/BVH.cuh:331-398):
 // tests the boxes of its children, goes on to the nearest one hit and stacks the others. Every triangle
 // whose box the ray passes before its current tMax is reached, so the closest hit is the reference
-// traversal's in any order of visits (tri_hit_closest settles equal distances).
+// traversal's in any order of visits (ray_step settles equal distances).
 //
 // A child's planes are origin + q * 2^e with 8-bit q, and the builder encloses the child's box between
 // the exact planes (quantize_node). Their slab distances come as one fused multiply-add each,
@@ -320,10 +293,21 @@ LTS_D void ray_begin(TraceRay& t, int kind, V3 o, V3 d, float tMax, int best, co
     trace_begin(t.l, o, d, root, ts);
 }
 
-// One step of the wave: the node step for the lanes that hold a node, or the triangle step for those that
-// hold a triangle once they are half as many (kGateRatio). A shadow ray's triangle test
-// (Triangle::simpleIntersect) is the closest-hit test with the triangle's second and third corners
-// exchanged and wider margins.
+// One step of the wave: the node step for the lanes that hold a node, or the triangle step (fp64 cross
+// products) for those that hold a triangle once they are half as many (kGateRatio). The records were checked
+// when the scene was loaded (k_check_recs): children lie in range and after their node, so each traversal ends,
+// and no accepted tree needs more than kStack entries.
+//
+// A triangle becomes the closest hit when it is nearer, or exactly as near with a lower leaf index.
+// BVH::intersect (BVH.cuh:365-398) keeps the first triangle it meets at the closest distance, and its
+// depth-first, left-first walk meets the leaves in index order, so of several triangles at exactly that distance
+// the lowest leaf wins; this rule gives the same winner in any visiting order. A shadow ray's triangle test
+// (Triangle::simpleIntersect, shapes/Triangle.cu:50-84) is the closest-hit test with the triangle's second and
+// third corners exchanged and wider margins: it accepts points up to SHADOW_EPS outside the triangle's edges,
+// and the reference reaches a triangle only through its leaf's box test (BVH.cuh:343-348: the leaf node's
+// bounds, the primitive's own bounds). The render tree's quantized boxes are wider than that leaf box, so a
+// triangle the enlarged test accepts is also put to the leaf-box test. (The closest-hit test accepts only points
+// inside the triangle shrunk by SHADOW_EPS, which lie inside its bounds.)
 constexpr int kGateRatio = 2;
 
 template <bool kCount>
@@ -486,80 +470,58 @@ LTS_D void ray_finish_shared(TraceRay& t, TraceStack ts, int* spill) {
     t = c;
 }
 
-// What a traversal does at a triangle.
-enum TraceKind {
-    kTraceClosest,  // Triangle::intersect: keep the closest hit
-    kTraceShadow,   // Triangle::simpleIntersect within the leaf's box: any triangle ends the traversal
-    kTraceBeats     // Triangle::intersect: any triangle that would win the closest hit against `best` at r.tMax
+// A lane's ray for trace_wave, and its answer: the closest hit (leaf -1: none), or whether a light ray is blocked.
+struct RayQuery {
+    int kind;  // kRayNone: the lane has no ray
+    V3 o, d;
+    float tMax;
+};
+struct RayAnswer {
+    int leaf;
+    float t, u, v, invDet;
+    bool blocked;
 };
 
-// A whole traversal by every lane of the wave that calls it. The wave runs either the node step or the
-// triangle step: lanes that hold a triangle wait until kLeafGate of them do or no lane holds a node, so
-// the triangle test (fp64 cross products) runs for several lanes at once. The records were checked when
-// the scene was loaded (k_check_recs): children lie in range and after their node, so each traversal
-// ends, and no accepted tree needs more than kStack entries.
-constexpr int kLeafGate = 8;
-
-template <int kKind>
-LTS_D Hit traverse(const TraceRec* recs, int root, Ray& r, TraceStack ts, int best, TraceTally* tally) {
-    Hit h;
-    h.leaf = -1; h.t = h.u = h.v = h.invDet = 0;
+// Traces one ray of every lane of the wave, all lanes taking part (BVH::intersect, BVH::simpleIntersect,
+// acceleration/BVH.cuh:331-398): lanes whose ray has ended, or that have none, help the others. A function of
+// its own, so that its registers are not the caller's. ldsAddress: the wave's kWaveTraceWords words.
+constexpr int kWaveTraceWords = 64 * kShortStack + 16;
+__attribute__((noinline)) static __device__ void trace_wave(const TraceRec* recs, int root, const RayQuery* query, RayAnswer* answer,
+                                                            unsigned ldsAddress) {
+    const int lane = threadIdx.x & 63;
+    int* const lds = (int*)(__attribute__((address_space(3))) int*)ldsAddress;
+    const TraceStack ts{lds + lane, 64};
+    volatile uint8_t* const mark = reinterpret_cast<volatile uint8_t*>(lds + 64 * kShortStack);
     int spill[kStack - kShortStack];
-    TraceLane l;
-    trace_begin(l, r.o, r.d, root, ts);
-    while (l.cur != kTraceDone) {
-        const bool leafStep = l.cur < 0;
-        const unsigned long long waiting = __ballot(leafStep), walking = __ballot(!leafStep);
-        if (walking != 0 && __popcll(waiting) < kLeafGate) {
-            if (!leafStep) {
-                if (tally) tally->nodes++;
-                trace_node(l, recs, r.tMax, ts, spill);
+    TraceRay t;
+    ray_none(t, lane);
+    if (query->kind != kRayNone) ray_begin(t, query->kind, query->o, query->d, query->tMax, -1, recs, root, ts);
+    RayAnswer a;
+    a.leaf = -1; a.t = a.u = a.v = a.invDet = 0; a.blocked = false;
+    int wait = 0;
+    for (;;) {
+        const unsigned long long idle = __ballot(t.l.cur == kTraceDone);
+        if (idle == ~0ull || (__popcll(idle) >= kShareIdle && --wait < 0)) {
+            wait = kShareSteps;
+            ray_settle(t, lane);
+            const bool held = ray_held(t, lane, mark), free = t.l.cur == kTraceDone && !held;
+            if (free && t.kind != kRayNone) {
+                a.leaf = t.best; a.t = t.tMax; a.u = t.u; a.v = t.v; a.invDet = t.invDet;
+                a.blocked = t.mat != 0;
+                t.kind = kRayNone;
             }
-        } else if (leafStep) {
-            const TraceTri tr = trace_triangle(l, recs);
-            if (tally) tally->tris++;
-            float t, u, v, id;
-            if constexpr (kKind == kTraceShadow) {
-                if (tri_occludes(tr.p0, tr.p1, tr.p2, r) && leaf_box_passes(tr.p0, tr.p1, tr.p2, r)) { h.leaf = tr.leaf; break; }
-            } else if constexpr (kKind == kTraceBeats) {
-                if (tri_hit_closest(tr.p0, tr.p1, tr.p2, r, tr.leaf, best, t, u, v, id)) { h.leaf = tr.leaf; break; }
-            } else {
-                if (tri_hit_closest(tr.p0, tr.p1, tr.p2, r, tr.leaf, h.leaf, t, u, v, id)) {
-                    r.tMax = t;
-                    h.leaf = tr.leaf; h.t = t; h.u = u; h.v = v; h.invDet = id;
-                }
-            }
-            trace_pop(l, ts, spill);
+            if (idle == ~0ull) break;
+            ray_share(t, free, lane, ts);
         }
+        ray_step<false>(t, ts, spill, nullptr);
     }
-    return h;
+    *answer = a;
 }
-
-// Closest hit (BVH::intersect, acceleration/BVH.cuh:365-398); r.tMax becomes its distance.
-LTS_D Hit trace_closest(const SceneView& sv, Ray& r, TraceStack ts, unsigned long long* nodeCount, unsigned long long* triCount,
-                        TraceTally* tally = nullptr) {
-    if (nodeCount) {
-        TraceTally own;
-        const Hit h = traverse<kTraceClosest>(sv.recs, sv.root, r, ts, -1, &own);
-        atomicAdd(nodeCount, own.nodes);
-        atomicAdd(triCount, own.tris);
-        return h;
-    }
-    return traverse<kTraceClosest>(sv.recs, sv.root, r, ts, -1, tally);
-}
-
-// Any hit (BVH::simpleIntersect, acceleration/BVH.cuh:331-363), whether the ray is blocked before
-// r.tMax. kHitTest: the closest-hit question of an MIS ray, whether any leaf beats tieLeaf at r.tMax.
-// Otherwise a shadow ray. Triangle::simpleIntersect accepts points up to SHADOW_EPS outside the
-// triangle's edges, and the reference reaches a triangle only through its leaf's box test
-// (BVH.cuh:343-348: the leaf node's bounds, the primitive's own bounds). The render tree's quantized
-// boxes are wider than that leaf box, so a triangle the enlarged test accepts is also put to the
-// leaf-box test. (The closest-hit test accepts only points inside the triangle shrunk by SHADOW_EPS,
-// which lie inside its bounds.)
-template <bool kHitTest = false>
-LTS_D bool trace_any(const SceneView& sv, const Ray& ray, TraceStack ts, TraceTally* tally = nullptr, int tieLeaf = -1) {
-    Ray r = ray;
-    return traverse<kHitTest ? kTraceBeats : kTraceShadow>(sv.recs, sv.root, r, ts, tieLeaf, tally).leaf >= 0;
+LTS_D RayAnswer trace_wave(const SceneView& sv, const RayQuery& query, int* lds) {
+    RayQuery q = query;
+    RayAnswer a;
+    trace_wave(sv.recs, sv.root, &q, &a, (unsigned)(uintptr_t)(__attribute__((address_space(3))) int*)lds);
+    return a;
 }
 
 // Triangle::intersect interaction part + SurfaceInteraction constructor / setShaddingGeometry
@@ -1131,13 +1093,6 @@ LTS_D Spec sample_li(const SceneView& sv, const LightDesc& L, const SurfacePoint
     return light_le(L);
 }
 
-LTS_D bool unoccluded(const SceneView& sv, const SurfacePoint& it, const LightPoint& p1, TraceStack ts) {
-    V3 origin = offsetRayOrigin(it.p, it.pError, it.n, p1.p - it.p);
-    V3 target = offsetRayOrigin(p1.p, p1.pError, p1.n, origin - p1.p);
-    Ray r; r.o = origin; r.d = target - origin; r.tMax = 1 - SHADOW_EPS;
-    return !trace_any(sv, r, ts);
-}
-
 // Distribution1D::sampleDiscrete with the reference's search length (Sampling.cuh:155-188)
 LTS_D int sample_light(const SceneView& sv, float u, float* pdf) {
     int size = sv.nLights, off;
@@ -1161,7 +1116,7 @@ LTS_D int sample_light(const SceneView& sv, float u, float* pdf) {
 // triangle seen from its emitting side, or for the infinite light whether the ray escapes. A ray that
 // misses the light's triangle, or meets its back, never contributes. A ray that meets its front at t
 // reaches it unless some triangle would win the closest hit against it (nearer, or at exactly t with a
-// lower leaf index, tri_hit_closest), which an any-hit traversal bounded at tMax = t with tieLeaf
+// lower leaf index, ray_step), which an any-hit traversal bounded at tMax = t with tieLeaf
 // answers; the same t, u, v and 1/det come out of the triangle test whatever tMax is.
 LTS_D bool mis_ray(const SceneView& sv, const LightDesc& L, int li, const SurfacePoint& si, const Ray& r, bool sampledSpecular,
                    float scatteringPdf, float& weight, float& tMax, int& tieLeaf) {

@@ -105,20 +105,25 @@ hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, Tra
     return hipGetLastError();
 }
 
-// Closest hits of caller-given rays: the renderer's own traversal (trace_closest), one thread per
-// ray; a miss gives prim -1.
-__global__ __launch_bounds__(256) void k_trace_rays(SceneView sv, const float* __restrict__ origins, const float* __restrict__ dirs,
+// Closest hits of caller-given rays by the renderer's own traversal, one thread per ray; a miss gives prim -1.
+// 500000 rays at a 90k-triangle torus: 180 us with every lane waiting for its wave's longest ray, 162 with
+// trace_wave (201 without the bound on waves: 130 VGPRs).
+__global__ __launch_bounds__(256, 6) void k_trace_rays(SceneView sv, const float* __restrict__ origins, const float* __restrict__ dirs,
                                                     int stride, int n, int32_t* __restrict__ prim, float* __restrict__ tOut) {
-    __shared__ int stk[kShortStack * 256];
+    __shared__ int lds[4][kWaveTraceWords];
     const int i = blockIdx.x * 256 + threadIdx.x;
+    RayQuery q;
+    q.kind = kRayNone;
+    if (i < n) {
+        const float* o = origins + (size_t)stride * i;
+        const float* d = dirs + (size_t)stride * i;
+        q.kind = kRayClosest;
+        q.o = v3(o[0], o[1], o[2]);
+        q.d = v3(d[0], d[1], d[2]);
+        q.tMax = INFINITY;
+    }
+    const RayAnswer h = trace_wave(sv, q, lds[threadIdx.x >> 6]);
     if (i >= n) return;
-    Ray r;
-    const float* o = origins + (size_t)stride * i;
-    const float* d = dirs + (size_t)stride * i;
-    r.o = v3(o[0], o[1], o[2]);
-    r.d = v3(d[0], d[1], d[2]);
-    r.tMax = INFINITY;
-    const Hit h = trace_closest(sv, r, lds_stack(stk, threadIdx.x, 256), nullptr, nullptr);
     int p = -1;
     if (h.leaf >= 0) {
         V3 p0, p1, p2;

@@ -540,8 +540,7 @@ __global__ __launch_bounds__(kCollectBlock) void k_wf_nrc_scatter(const WfParams
 // (kGateRatio; measured before rays were shared: 29.5 ms of tracing per 64-spp frame of the 1M-triangle
 // displaced sphere at 1920x1080, 30.5 at a ratio of 1, 29.8 at 3, 31.1 at 6 and 38.0 without waiting; 43 ms
 // before both). Once no rays are left, a wave's free lanes help the others (ray_share). The lanes carry
-// rays of any kind: a shadow ray's triangle test (Triangle::simpleIntersect) is the closest-hit test with
-// the triangle's second and third corners exchanged and wider margins.
+// rays of any kind.
 // The launch asks for 6 waves per SIMD (80 VGPRs): 25.1 ms for that frame, 27.3 at 7 waves (72 VGPRs, spilling
 // in the loop), 26.9 at 5.
 // kCount: the counting instantiation, which also adds every lane's render-node fetches and

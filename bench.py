@@ -8,7 +8,7 @@ fixed seeds in the reference's own file formats (lighttransportsimulation_amd/sc
 Extra fields of the default run (the 1080p workload):
   roofline        the traversal kernel (k_wf_trace: path, shadow and MIS rays, one launch per bounce)
                   against HBM bandwidth. Algorithmic bytes are the kernel's own work on its own
-                  tree: 64 B per quantized 4-wide node fetch and 48 B per triangle test, counted on
+                  tree: 48 B per quantized 4-wide node fetch and 48 B per triangle test, counted on
                   the GPU for every ray kind of the same frame by the counting instantiation of the
                   kernel (an untimed run), over the kernel's device time per frame from HIP events.
                   `traffic` is the HBM bytes per frame that rocprofv3's FETCH_SIZE / WRITE_SIZE
@@ -40,7 +40,7 @@ METRIC = "Msamples/s & equal-time relMSE: cached vs plain path tracer, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
 # bytes the traversal kernel reads per render-node fetch (a quantized 4-wide node, four 16-byte
 # loads) and per triangle test (three 16-byte loads)
-NODE_BYTES, TRI_BYTES = 64, 48
+NODE_BYTES, TRI_BYTES = 48, 48
 # radix passes of the LBVH sort (10-bit digits over the 30-bit Morton codes)
 LBVH_RADIX_PASSES = 3
 
@@ -619,7 +619,7 @@ def main() -> int:
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": "k_wf_trace",
                 "kernel_ms_per_step": round(trav_ms, 3), "launches_per_step": n_launch,
                 "kernel_avg_launch_ms": round(trav_ms / n_launch, 3) if n_launch else None,
-                "algorithmic_bytes": "64 B per 4-wide node fetch + 48 B per triangle test, counted on the GPU for "
+                "algorithmic_bytes": "48 B per 4-wide node fetch + 48 B per triangle test, counted on the GPU for "
                                      "the same frame",
                 "algorithmic_bytes_per_sample": {k: round(v, 1) for k, v in per_sample.items()},
                 "node_fetches_per_sample": {k: round(n, 3) for k, (n, t) in counts.items()},

@@ -366,7 +366,9 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_scatter(const uint32_t* __
     __shared__ uint32_t scratch[kSortWaves];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int tile = xcd_tile(blockIdx.x, tiles);
-    for (int q = t; q < kSortWaves * kBins; q += kSortBlock) (&waveCnt[0][0])[q] = 0;
+    // A wave clears its own counters: its LDS operations execute in order, so it may count at once. Cleared by
+    // all threads together, a late wave could clear what another had counted already.
+    for (int q = lane; q < kBins; q += 64) waveCnt[wave][q] = 0;
     {  // the digits' bases in this tile: segment base (with the digit's base in the pass) + prefix in the segment
         const uint4 sb = reinterpret_cast<const uint4*>(segBase + (size_t)(tile / kSegTiles) * kBins)[t];
         const uint4 tb = reinterpret_cast<const uint4*>(counts + (size_t)tile * kBins)[t];

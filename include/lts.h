@@ -52,7 +52,12 @@ typedef struct lts_bvh_timing {
 /* Integrators. The megakernel and the wavefront are the plain path tracer: their samples are the same
  * bit for bit, and each runs the form that suits the size of its passes, whole paths in one launch up to
  * 2^22 samples of a scene and a wavefront of queues above. A wavefront for which a tuning option is set
- * (trace_block .. count_traversal below) runs as queues at any size. */
+ * (trace_block .. count_traversal below) runs as queues at any size.
+ * Device memory, kept by the context from render to render: 12 bytes for each sample of a pass, 28 for each
+ * pixel, and for queues 249 bytes of path state for each sample of a pass. The megakernel's queues take at
+ * most its automatic pass (2^28 / 12 samples: 5.6 GB; a longer spp_per_pass is cut to it, samples returned
+ * from more than that are traced as whole paths), and whole paths where the state finds no memory. A context
+ * gives its path state back when another of its calls finds none. */
 #define LTS_INTEGRATOR_MEGAKERNEL 0
 #define LTS_INTEGRATOR_WAVEFRONT 1
 #define LTS_INTEGRATOR_CACHED 2

@@ -122,12 +122,15 @@ int fail(lts_ctx* c, int code, const std::string& msg) {
     return code;
 }
 
+// A reported error is not left behind: the next kernel launch would report it again as its own.
 #define HIPCHK(ctx, expr)                                                                              \
     do {                                                                                               \
         hipError_t e_ = (expr);                                                                        \
-        if (e_ != hipSuccess)                                                                          \
+        if (e_ != hipSuccess) {                                                                        \
+            (void)hipGetLastError();                                                                   \
             return fail(ctx, e_ == hipErrorOutOfMemory ? LTS_E_NOMEM : LTS_E_HIP,                     \
                         std::string(#expr) + ": " + hipGetErrorString(e_));                            \
+        }                                                                                              \
     } while (0)
 
 template <typename T>
@@ -264,14 +267,33 @@ void film_advance(lts_ctx* c, const lts_render_params* p, int b1) {
     c->filmNext = b1;
 }
 
+// hipMalloc for c; when the device has no memory left, the path state that c holds between renders is given
+// back first. Not while a render uses that state: what a render needs besides it is allocated before it.
+hipError_t alloc_or_reclaim(lts_ctx* c, float** p, size_t floats) {
+    hipError_t e = hipMalloc((void**)p, floats * sizeof(float));
+    if (e != hipErrorOutOfMemory || c->wf.cap == 0) return e;
+    (void)hipGetLastError();
+    wf_release(c->wf);
+    return hipMalloc((void**)p, floats * sizeof(float));
+}
+
+// Runs a call that uses no path state, again without the context's when it finds no memory.
+template <typename F>
+int reclaiming(lts_ctx* c, F f) {
+    const int rc = f();
+    if (rc != LTS_E_NOMEM || !c || c->wf.cap == 0) return rc;
+    wf_release(c->wf);
+    return f();
+}
+
 int ensure_film(lts_ctx* c, size_t npix) {
     if (npix <= c->filmCap) return LTS_OK;
     if (c->film) (void)hipFree(c->film);
     if (c->rgb) (void)hipFree(c->rgb);
     c->film = c->rgb = nullptr;
     c->filmCap = 0;
-    HIPCHK(c, hipMalloc((void**)&c->film, npix * 4 * sizeof(float)));
-    HIPCHK(c, hipMalloc((void**)&c->rgb, npix * 3 * sizeof(float)));
+    HIPCHK(c, alloc_or_reclaim(c, &c->film, npix * 4));
+    HIPCHK(c, alloc_or_reclaim(c, &c->rgb, npix * 3));
     c->filmCap = npix;
     return LTS_OK;
 }
@@ -281,7 +303,7 @@ int ensure_samples(lts_ctx* c, size_t floats) {
     if (c->sampleL) (void)hipFree(c->sampleL);
     c->sampleL = nullptr;
     c->sampleCap = 0;
-    HIPCHK(c, hipMalloc((void**)&c->sampleL, floats * sizeof(float)));
+    HIPCHK(c, alloc_or_reclaim(c, &c->sampleL, floats));
     c->sampleCap = floats;
     c->sampleGen = next_buffer_generation();
     return LTS_OK;
@@ -315,6 +337,12 @@ int wf_run(lts_ctx* c, const WfTuning& t, int maxBounce, const NrcBuffers* nrc, 
         if (e == hipSuccess) e = e2;
         if (e == hipSuccess) e = hipGraphInstantiate(&c->wfExec, g, nullptr, nullptr, 0);
         if (g) (void)hipGraphDestroy(g);
+        if (e == hipErrorOutOfMemory) {  // no memory for the graph: the pass needs none
+            (void)hipGetLastError();
+            c->wfExec = nullptr;
+            HIPCHK(c, wf_enqueue_pass(c->wf, t, maxBounce, nrc, s, prof));
+            return LTS_OK;
+        }
         HIPCHK(c, e);
         c->wfKeyGen = c->wf.gen;
         c->wfKeyCacheGen = cacheGen;
@@ -502,7 +530,7 @@ bool wavefront_defaults(const lts_render_params* p) {
            !p->autotune && !p->profile_phases && !p->count_traversal;
 }
 
-// Samples of a wavefront pass. Automatic: 2^27 paths (about 36 GB of path state at 268 B per path). Each pass runs its
+// Samples of a wavefront pass. Automatic: 2^27 paths (33 GB of path state at 249 B per path). Each pass runs its
 // bounces as separate launches whose late ones hold few paths, so fewer, larger passes keep the
 // GPU busy: 2^24 -> 2^26 paths took the 1080p 64-spp frame from 585 to 756 Msamples/s, and
 // 2^26 -> 2^27 (the whole frame in one pass) from 1392 to 1524. The cached integrator takes the
@@ -540,30 +568,25 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
     pass = std::min(pass, b1 - b0);
     const size_t cap = totalPix * (size_t)pass;
     if (cap > (size_t)INT32_MAX) return fail(c, LTS_E_ARG, "pass holds more than 2^31 paths");
-    const bool realloc = cap > c->wf.cap || (int)scenes.size() > c->wf.maxScenes;
-    const hipError_t reserved = wf_reserve(c->wf, cap, (int)scenes.size());
-    if (reserved == hipErrorOutOfMemory && p->integrator == LTS_INTEGRATOR_MEGAKERNEL) {
-        (void)hipGetLastError();
-        return LTS_E_NOMEM;  // the caller has a form that needs no path state
-    }
-    HIPCHK(c, reserved);
-    if (realloc && c->wfExec) {
-        (void)hipGraphExecDestroy(c->wfExec);
-        c->wfExec = nullptr;
-    }
-    c->wf.matBins = std::min(maxMats, kWfMaxMatBins - 1) + 1;
     if ((rc = ensure_samples(c, cap * 3)) != LTS_OK) return rc;
-    c->wf.sampleBase = c->sampleL;
-    // training paths stay a minority of the pass (at most 1/8 of its paths) so most paths query
-    const int trainPaths = cached ? (int)std::max<size_t>(1, std::min<size_t>((size_t)c->nrcCfg.train_paths, cap / 8)) : 0;
-    if (cached) HIPCHK(c, wf_reserve_cache(c->wf, cap, trainPaths));
-    const NrcBuffers* nrc = cached ? &c->nrc : nullptr;
     std::vector<SceneView> views;
     for (lts_ctx* x : scenes) {
         views.push_back(x->scene.view);
         if ((rc = ensure_film(x, (size_t)x->scene.view.cam.width * x->scene.view.cam.height)) != LTS_OK)
             return fail(c, rc, x->err);
     }
+    const bool realloc = cap > c->wf.cap || (int)scenes.size() > c->wf.maxScenes;
+    HIPCHK(c, wf_reserve(c->wf, cap, (int)scenes.size()));
+    if (realloc && c->wfExec) {
+        (void)hipGraphExecDestroy(c->wfExec);
+        c->wfExec = nullptr;
+    }
+    c->wf.matBins = std::min(maxMats, kWfMaxMatBins - 1) + 1;
+    c->wf.sampleBase = c->sampleL;
+    // training paths stay a minority of the pass (at most 1/8 of its paths) so most paths query
+    const int trainPaths = cached ? (int)std::max<size_t>(1, std::min<size_t>((size_t)c->nrcCfg.train_paths, cap / 8)) : 0;
+    if (cached) HIPCHK(c, wf_reserve_cache(c->wf, cap, trainPaths));
+    const NrcBuffers* nrc = cached ? &c->nrc : nullptr;
     HIPCHK(c, hipMemcpyAsync(c->wf.scenes, views.data(), views.size() * sizeof(SceneView), hipMemcpyHostToDevice, s));
     if (b0 == 0)
         for (lts_ctx* x : scenes)
@@ -1042,12 +1065,12 @@ static int trace_rays_impl(lts_ctx* c, const float* rays, const float* dirs, int
 }
 
 int lts_trace_rays(lts_ctx* c, const float* rays, int32_t n, int32_t* prim, float* t) {
-    return guarded(c, [&] { return trace_rays_impl(c, rays, nullptr, n, prim, t); });
+    return guarded(c, [&] { return reclaiming(c, [&] { return trace_rays_impl(c, rays, nullptr, n, prim, t); }); });
 }
 
 int lts_trace_rays_split(lts_ctx* c, const float* origins, const float* directions, int32_t n, int32_t* prim, float* t) {
     if (!directions) return fail(c, LTS_E_ARG, "bad trace_rays arguments");
-    return guarded(c, [&] { return trace_rays_impl(c, origins, directions, n, prim, t); });
+    return guarded(c, [&] { return reclaiming(c, [&] { return trace_rays_impl(c, origins, directions, n, prim, t); }); });
 }
 
 int lts_render_tree_info(lts_ctx* c, int32_t* kind, int32_t* depth, int32_t* nodes4) {
@@ -1137,31 +1160,40 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
     sample_range(p, &b0, &b1);
     // samples of a pass; all of them where they are returned
     const bool wavefront = p->integrator == LTS_INTEGRATOR_WAVEFRONT;
-    int pass = wavefront ? wavefront_pass(p, npix)
-               : p->spp_per_pass > 0 ? p->spp_per_pass
-                                     : (int)std::max<size_t>(1, std::min<size_t>((size_t)(b1 - b0), (size_t)(1u << 28) / (npix * 12)));
+    const int automatic = (int)std::max<size_t>(1, std::min<size_t>((size_t)(b1 - b0), kWholePass / npix));
+    int pass = wavefront ? wavefront_pass(p, npix) : p->spp_per_pass > 0 ? p->spp_per_pass : automatic;
     if (sample_rgb) pass = b1 - b0;
     pass = std::min(pass, b1 - b0);
     const std::vector<lts_ctx*> one{c};
     if (p->integrator == LTS_INTEGRATOR_CACHED) return render_wavefront(c, one, p, &rgb_out, sample_rgb, st);
     // The plain path tracer has two forms with the same samples: whole paths in one launch, and the wavefront.
     // The size of the pass decides (kPathPass) for the megakernel, whose traversal counts are of whole paths,
-    // and for a wavefront whose tuning the caller leaves open. A megakernel pass stays whole where the path
-    // state finds no memory.
+    // and for a wavefront whose tuning the caller leaves open. The megakernel's queues hold at most an automatic
+    // pass (kWholePass samples, 5.6 GB of path state); where they find no memory, and for more samples than that
+    // returned from one pass, the pass stays whole and takes 12 bytes a sample.
     const bool small = npix * (size_t)pass <= kPathPass;
     if (wavefront && !(small && p->max_bounce > 0 && wavefront_defaults(p)))
         return render_wavefront(c, one, p, &rgb_out, sample_rgb, st);
+    if ((rc = film_continues(c, p, b0)) != LTS_OK) return rc;
+    const int queuePass = sample_rgb ? pass : std::min(pass, automatic);
     if (p->integrator == LTS_INTEGRATOR_MEGAKERNEL && !small && p->max_bounce > 0 && p->max_bounce <= kWfMaxBounce &&
-        !p->count_traversal && npix * (size_t)pass <= ((size_t)1 << 27)) {
+        !p->count_traversal && npix * (size_t)queuePass <= kWholePass) {
         lts_render_params q = *p;
-        q.spp_per_pass = pass;
+        q.spp_per_pass = queuePass;
         q.trace_block = q.persistent_blocks = q.tile_rows = q.autotune = q.profile_phases = 0;
         q.sort_materials = q.use_graph = -1;
-        rc = render_wavefront(c, one, &q, &rgb_out, sample_rgb, st);
-        if (rc == LTS_OK && st) st->trace_block = st->persistent_blocks = st->sort_materials = st->use_graph = st->tile_rows = st->spp_per_pass = 0;
-        if (rc != LTS_E_NOMEM) return rc;
+        // what both forms need, then the path state; once that is there the render's errors are its own
+        if ((rc = ensure_samples(c, npix * (size_t)queuePass * 3)) != LTS_OK) return rc;
+        if ((rc = ensure_film(c, npix)) != LTS_OK) return rc;
+        const hipError_t reserved = wf_reserve(c->wf, npix * (size_t)queuePass, 1);
+        if (reserved == hipSuccess) {
+            rc = render_wavefront(c, one, &q, &rgb_out, sample_rgb, st);
+            if (rc == LTS_OK && st) st->trace_block = st->persistent_blocks = st->sort_materials = st->use_graph = st->tile_rows = st->spp_per_pass = 0;
+            return rc;
+        }
+        (void)hipGetLastError();
+        if (reserved != hipErrorOutOfMemory) HIPCHK(c, reserved);
     }
-    if ((rc = film_continues(c, p, b0)) != LTS_OK) return rc;
     if ((rc = ensure_samples(c, npix * (size_t)pass * 3)) != LTS_OK) return rc;
     if ((rc = ensure_film(c, npix)) != LTS_OK) return rc;
     hipStream_t s = c->stream;
@@ -1474,15 +1506,15 @@ static int obj_to_bin_impl(const char* stem, int32_t* nTris) {
 // Entry points: host allocation failures and other exceptions become error codes, never
 // an exception crossing the C boundary.
 int lts_load_scene(lts_ctx* c, const char* dir, const char* scene, const char* subject, int32_t width, int32_t height) {
-    return guarded(c, [&] { return load_scene_impl(c, dir, scene, subject, width, height); });
+    return guarded(c, [&] { return reclaiming(c, [&] { return load_scene_impl(c, dir, scene, subject, width, height); }); });
 }
 
 int lts_bvh_build(lts_ctx* c, const float* tri, int32_t n, int32_t mode, lts_bvh_export* out, lts_bvh_timing* t) {
-    return guarded(c, [&] { return bvh_build_impl(c, tri, n, mode, out, t); });
+    return guarded(c, [&] { return reclaiming(c, [&] { return bvh_build_impl(c, tri, n, mode, out, t); }); });
 }
 
 int lts_bvh_build_device(lts_ctx* c, const float* dtri, int32_t n, int32_t mode, int32_t repeat, lts_bvh_timing* t) {
-    return guarded(c, [&] { return bvh_build_device_impl(c, dtri, n, mode, repeat, t); });
+    return guarded(c, [&] { return reclaiming(c, [&] { return bvh_build_device_impl(c, dtri, n, mode, repeat, t); }); });
 }
 
 int lts_mesh_transform(lts_ctx* c, const float* subject, float* points, int32_t n_points, float* normals, int32_t n_normals) {

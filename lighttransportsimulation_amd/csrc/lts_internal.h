@@ -120,6 +120,8 @@ hipError_t launch_paths(const SceneView& sv, const RenderLaunch& rl, int32_t* wo
 // 1.27/1.52, 3.7M 2.88/2.77, 7.4M 5.06/4.06; of a 256x256 Cornell box: 1.0M 1.52/2.08, 4.2M 4.74/5.03; of a
 // 1920x1080 frame of the 1M-triangle sphere: 2.1M 1.89/2.53, 4.1M 3.16/3.45, 8.3M 5.76/5.12).
 constexpr size_t kPathPass = (size_t)1 << 22;
+// Samples of an automatic megakernel or bidirectional pass: 256 MiB of radiance.
+constexpr size_t kWholePass = ((size_t)1 << 28) / 12;
 // Bidirectional path tracing (bdpt.hip), with the same sample layout and film.
 constexpr int kBdptMaxBounce = 8;
 hipError_t launch_bdpt(const SceneView& sv, const RenderLaunch& rl, hipStream_t stream);

@@ -54,6 +54,9 @@ typedef struct oracle_scene oracle_scene;
 // parseScene does. Returns NULL on failure (message via oracle_last_error()).
 oracle_scene* oracle_load_scene(const char* project_dir, const char* scene, const char* subject,
                                 int32_t width, int32_t height);
+// Pixels (w * h RGB bytes, top row first) of the JPEG file with exactly these bytes, for scene loads in a
+// process without the reference's decoder. The caller vouches that they are that decoder's.
+void oracle_add_jpeg_pixels(const uint8_t* file, int64_t bytes, int32_t w, int32_t h, const uint8_t* rgb);
 void oracle_free_scene(oracle_scene* s);
 const char* oracle_last_error(void);
 int32_t oracle_scene_info(const oracle_scene* s, int32_t* n_tris, int32_t* n_lights, int32_t* n_meshes);

@@ -107,7 +107,17 @@ static bool decodePPM(const std::vector<unsigned char>& b, int& w, int& h, std::
 
 // JPEG: the reference's own decoder, stb_image 2.27 (extern/stb_image.h), compiled by this
 // directory's Makefile into _ref/libstb_image.so beside _build/, and called through
-// stbi_load_from_memory with 3 components requested, as stbi_loadf does (ImageI.cuh:14).
+// stbi_load_from_memory with 3 components requested, as stbi_loadf does (ImageI.cuh:14). Without that
+// library, the pixels given to oracle_add_jpeg_pixels for the same file.
+struct JpegPixels {
+    std::vector<unsigned char> file, rgb;
+    int w, h;
+};
+static std::vector<JpegPixels> g_jpegPixels;
+extern "C" void oracle_add_jpeg_pixels(const uint8_t* file, int64_t bytes, int32_t w, int32_t h, const uint8_t* rgb) {
+    g_jpegPixels.push_back({std::vector<unsigned char>(file, file + bytes),
+                            std::vector<unsigned char>(rgb, rgb + 3 * (size_t)w * h), w, h});
+}
 static bool decodeJPEG(const std::vector<unsigned char>& b, int& w, int& h, std::vector<unsigned char>& rgb, std::string& err) {
     typedef unsigned char* (*LoadFn)(const unsigned char*, int, int*, int*, int*, int);
     typedef void (*FreeFn)(void*);
@@ -119,6 +129,15 @@ static bool decodeJPEG(const std::vector<unsigned char>& b, int& w, int& h, std:
         std::string dir(self.dli_fname);
         dir = dir.substr(0, dir.find_last_of('/'));
         void* lib = dlopen((dir + "/../_ref/libstb_image.so").c_str(), RTLD_NOW | RTLD_LOCAL);
+        if (!lib) {
+            for (const JpegPixels& p : g_jpegPixels)
+                if (p.file == b) {
+                    w = p.w;
+                    h = p.h;
+                    rgb = p.rgb;
+                    return true;
+                }
+        }
         if (!lib) { err = "JPEG needs oracle/_ref/libstb_image.so (built from the reference's extern/stb_image.h)"; return false; }
         release = (FreeFn)dlsym(lib, "stbi_image_free");
         load = (LoadFn)dlsym(lib, "stbi_load_from_memory");

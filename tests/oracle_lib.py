@@ -6,12 +6,17 @@ cpu_baseline leg load it, as the checker and as the host-core baseline.
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import hashlib
+import json
 import os
 
 import numpy as np
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(ROOT, "oracle", "_build", "liboracle.so")
+STB_PATH = os.path.join(ROOT, "oracle", "_ref", "libstb_image.so")
+GOLDEN = os.path.join(ROOT, "tests", "golden")
 
 _lib = None
 
@@ -48,6 +53,8 @@ def lib():
         L.oracle_sample.argtypes = [C.c_uint32, C.c_uint32, C.c_uint32, C.c_int32]
         L.oracle_load_scene.restype = C.c_void_p
         L.oracle_load_scene.argtypes = [C.c_char_p, C.c_char_p, C.c_char_p, C.c_int32, C.c_int32]
+        L.oracle_add_jpeg_pixels.argtypes = [C.c_char_p, C.c_int64, C.c_int32, C.c_int32, C.c_void_p]
+        L.oracle_add_jpeg_pixels.restype = None
         L.oracle_free_scene.argtypes = [C.c_void_p]
         L.oracle_last_error.restype = C.c_char_p
         L.oracle_scene_info.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
@@ -131,8 +138,34 @@ def philox(ctr, key) -> np.ndarray:
     return o
 
 
+@functools.cache
+def _add_pinned_jpegs():
+    """Where the reference's JPEG decoder is not built (it needs the reference tree), gives the oracle the
+    pixels of the one JPEG texture among the fixtures: decoded by the product, and the reference
+    decoder's bytes by their digest (golden/jpeg_stb_sha256.json)."""
+    if os.path.exists(STB_PATH):
+        return
+    from lighttransportsimulation_amd import LtsError, load_image
+    name = "res/blackDragon.jpg"
+    try:
+        linear = load_image(os.path.join(GOLDEN, name))
+    except LtsError:
+        return  # no product library to ask
+    lut = np.float32(np.float64(np.arange(256, dtype=np.float32) / np.float32(255)) ** np.float64(np.float32(2.2)))
+    rgb = np.ascontiguousarray(np.searchsorted(lut, linear).astype(np.uint8)[::-1])
+    h, w, _ = rgb.shape
+    with open(os.path.join(GOLDEN, "jpeg_stb_sha256.json")) as f:
+        pinned = json.load(f)[name]
+    if f"{w}x{h}:" + hashlib.sha256(rgb.tobytes()).hexdigest()[:32] != pinned:
+        raise RuntimeError(f"{name} does not decode to the reference decoder's bytes")
+    with open(os.path.join(GOLDEN, name), "rb") as f:
+        data = f.read()
+    lib().oracle_add_jpeg_pixels(data, len(data), w, h, _p(rgb))
+
+
 class OracleScene:
     def __init__(self, project_dir: str, scene: str, subject: str, width: int, height: int):
+        _add_pinned_jpegs()
         d = project_dir if project_dir.endswith("/") else project_dir + "/"
         h = lib().oracle_load_scene(d.encode(), scene.encode(), (subject or "").encode(), width, height)
         if not h:

@@ -72,7 +72,8 @@ LTS_D void work_next(WorkDeal<T>& q, int waves, int resident, int32_t* work) {
     auto start = [&](int s, int c) { return (T)(((min((int)gridDim.x, resident) - s + kWfWorkSegments - 1) / kWfWorkSegments) * waves + c) * q.chunk; };
     auto take = [&](int s, T at) {
         q.next = s * segLen + at;
-        q.end = at < segLen ? min(q.next + q.chunk, q.n) : q.next;
+        // a segment's last chunk ends with it: what lies behind is another wave's
+        q.end = at < segLen ? min(q.next + min((T)q.chunk, segLen - at), q.n) : q.next;
         return q.next < q.end;
     };
     if (q.open >> kWfWorkSegments) {

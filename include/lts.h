@@ -139,7 +139,8 @@ typedef struct lts_stats {
     double msamples_per_s;  /* samples / (render_ms + resolve_ms)                   */
     int64_t node_visits;    /* count_traversal: render-node fetches of the path rays */
     int64_t tri_tests;
-    int32_t trace_block;    /* wavefront tuning that was used                      */
+    int32_t trace_block;    /* wavefront of queues: tuning that was used (all four 0 where the   */
+                            /*    render ran as whole paths, and for the megakernel)             */
     int32_t persistent_blocks;
     int32_t sort_materials;
     int32_t use_graph;

@@ -1238,12 +1238,7 @@ static int render_impl(lts_ctx* c, const lts_render_params* p, float* rgb_out, f
         st->samples = (int64_t)npix * (b1 - b0);
         st->msamples_per_s = (renderMs + resolveMs) > 0 ? st->samples / ((renderMs + resolveMs) * 1e3) : 0;
         if (wavefront) {
-            const WfTuning t;
-            st->trace_block = t.traceBlock;
-            st->persistent_blocks = t.persistentBlocks;
-            st->sort_materials = t.sortMaterials;
-            st->use_graph = t.useGraph;
-            st->tile_rows = t.tileRows;
+            st->tile_rows = kPathRows;
             st->spp_per_pass = pass;
         }
         if (rl.counters) {

@@ -114,6 +114,7 @@ struct RenderLaunch {
 // Whole paths in one launch (paths.hip). work, other: kPathWork counters each; the launch takes work cleared
 // and clears other, so a context's launches alternate between two sets.
 constexpr int kPathWork = 128;
+constexpr int kPathRows = 8;  // band height of their path order
 hipError_t launch_paths(const SceneView& sv, const RenderLaunch& rl, int32_t* work, int32_t* other, hipStream_t stream);
 // Passes of at most this many samples of one scene run as whole paths, larger ones as wavefront passes
 // (device ms, whole paths / wavefront, of a 1280x720 frame of a 360k-triangle displaced sphere: 0.92M samples

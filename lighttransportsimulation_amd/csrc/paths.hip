@@ -36,7 +36,7 @@ LTS_D bool film_path(const SceneView& sv, const RenderLaunch& rl, long k, int& p
     const int n = rl.s1 - rl.s0, j = (int)(g / n) * 64 + (int)(k & 63);
     sample = rl.s0 + (int)(g % n);
     if (j >= sv.cam.width * sv.cam.height) return false;
-    pixel = band_pixel(j, sv.cam.width, sv.cam.height, 8);
+    pixel = band_pixel(j, sv.cam.width, sv.cam.height, kPathRows);
     return true;
 }
 

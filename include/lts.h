@@ -79,7 +79,8 @@ typedef struct lts_render_params {
                           /* 2^27 paths per pass; megakernel: 2^28 / 12 B)          */
     /* wavefront of queues only (0 / -1 = default or the autotuned value) */
     int32_t trace_block;        /* block size of the persistent traversal kernels: 64, 128, 256 */
-    int32_t persistent_blocks;  /* grid of the persistent traversal kernels                     */
+    int32_t persistent_blocks;  /* grid of the persistent traversal kernels; at most the          */
+                                /*    workgroups resident at once are launched (1536 of 256)     */
     int32_t sort_materials;     /* -1 default (on), 0 off, 1 shade in material order            */
     int32_t use_graph;          /* -1 default (on), 0 off: capture each pass in a hipGraph       */
     int32_t autotune;           /* 1: time candidate tunings on this scene before rendering:    */

@@ -477,10 +477,15 @@ int autotune(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_render_p
         WfTuning t = cur; t.traceBlock = tb;
         if ((rc = consider(t)) != LTS_OK) return rc;
     }
+    // grids as they are launched: those above the resident workgroups are one candidate
+    cur.persistentBlocks = wf_trace_grid(cur.traceBlock, cur.persistentBlocks);
     const WfTuning afterBlock = cur;
+    int timed = 0;
     for (int pb : {512, 1024, 2048, 4096, 8192}) {
-        if (pb == afterBlock.persistentBlocks) continue;
-        WfTuning t = afterBlock; t.persistentBlocks = pb;
+        const int grid = wf_trace_grid(afterBlock.traceBlock, pb);
+        if (grid == afterBlock.persistentBlocks || grid == timed) continue;
+        timed = grid;
+        WfTuning t = afterBlock; t.persistentBlocks = grid;
         if ((rc = consider(t)) != LTS_OK) return rc;
     }
     {
@@ -496,7 +501,8 @@ int autotune(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_render_p
     }
     // The search compares single passes, so a choice can win by noise: time it against the starting
     // tuning again, two passes each, and keep the starting tuning unless the choice is faster.
-    const WfTuning start = *best;
+    WfTuning start = *best;
+    start.persistentBlocks = wf_trace_grid(start.traceBlock, start.persistentBlocks);
     if (cur.traceBlock != start.traceBlock || cur.persistentBlocks != start.persistentBlocks ||
         cur.sortMaterials != start.sortMaterials || cur.tileRows != start.tileRows) {
         double msStart = 0, msCur = 0;

@@ -191,7 +191,7 @@ constexpr int kMaxTileRows = 64;
 
 struct WfTuning {
     int traceBlock = 256;         // block size of the persistent traversal kernels (64, 128, 256)
-    int persistentBlocks = 2048;  // grid of the traversal kernels, at most the workgroups resident at once
+    int persistentBlocks = 2048;  // grid of the traversal kernels, at most the workgroups resident at once (wf_trace_grid)
     int sweepBlocks = 2048;       // grid of the generate / shade / finalize sweeps
     int sortMaterials = 1;        // shade in material order within chunks of the queue
     int useGraph = 1;             // capture the pass in a hipGraph and replay it
@@ -249,6 +249,8 @@ struct WfProfile { hipEvent_t ev[kWfPhaseEvents]; };
 // rays (the megakernel uses the first two, for its path rays).
 constexpr int kTraceCounters = 6;
 
+// Workgroups of traceBlock threads in a trace launch of grid persistentBlocks.
+int wf_trace_grid(int traceBlock, int persistentBlocks);
 hipError_t wf_reserve(WfBuffers& b, size_t cap, int maxScenes);
 hipError_t wf_reserve_cache(WfBuffers& b, size_t cap, int trainCap);
 void wf_release(WfBuffers& b);

@@ -684,6 +684,8 @@ __global__ void k_wf_fill(int32_t* p, int n, int32_t v) {
 
 }  // namespace
 
+int wf_trace_grid(int traceBlock, int persistentBlocks) { return std::min(persistentBlocks, resident_blocks(traceBlock)); }
+
 hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce, const NrcBuffers* nrc, hipStream_t s,
                            const WfProfile* prof, unsigned long long* traceCounts) {
     auto mark = [&](int i) {
@@ -707,7 +709,7 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
         const int32_t* ext = bounce > 0 ? b.queue[bounce & 1] : nullptr;
         int32_t* work = bounce0 + kWfCountsPerBounce * bounce + kWfWorkBase;
         auto launch = [&](auto kernel, int bs) {
-            kernel<<<std::min(t.persistentBlocks, resident_blocks(bs)), bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, bins, b.matBins, b.shadows, shadowCount,
+            kernel<<<wf_trace_grid(bs, t.persistentBlocks), bs, 0, s>>>(b.scenes, b.rays, b.hits, ext, extCount, bins, b.matBins, b.shadows, shadowCount,
                                                      b.mis, misCount, b.shadowQ, b.misQ, b.nee, work, traceCounts);
         };
         const bool counting = traceCounts != nullptr;

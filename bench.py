@@ -38,8 +38,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Msamples/s & equal-time relMSE: cached vs plain path tracer, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
-# bytes the traversal kernel reads per render-node fetch (a quantized 4-wide node, four 16-byte
-# loads) and per triangle test (three 16-byte loads)
+# bytes the traversal kernel reads per render-node fetch (a quantized 4-wide node) and per triangle test: a
+# record of three 16-byte loads either way
 NODE_BYTES, TRI_BYTES = 48, 48
 # radix passes of the LBVH sort (10-bit digits over the 30-bit Morton codes)
 LBVH_RADIX_PASSES = 3

@@ -44,8 +44,9 @@ typedef struct lts_bvh_export {
 
 typedef struct lts_bvh_timing {
     double total_ms;   /* bounds -> pack, device time of the whole build           */
-    double sort_ms;    /* the four radix-sort passes                               */
-    double bounds_ms;  /* primitive bounds + scene-bound reduction + Morton codes  */
+    double sort_ms;    /* the three radix-sort passes; 0 for up to 16384 triangles, which one  */
+                       /* launch boxes, codes and sorts                                        */
+    double bounds_ms;  /* primitive bounds + scene-bound reduction + Morton codes; that launch */
     double tree_ms;    /* Karras hierarchy + bottom-up refit + node packing        */
 } lts_bvh_timing;
 
@@ -76,7 +77,8 @@ typedef struct lts_render_params {
     int32_t stratified;   /* 1: film sample per Sampler::stratifiedSample          */
     int32_t integrator;   /* LTS_INTEGRATOR_*                                      */
     int32_t spp_per_pass; /* samples per pass; 0 = automatic (wavefront and cached: */
-                          /* 2^27 paths per pass; megakernel: 2^28 / 12 B)          */
+                          /* 2^27 paths per pass; megakernel and bidirectional:     */
+                          /* 2^28 / 12 samples)                                     */
     /* wavefront of queues only (0 / -1 = default or the autotuned value) */
     int32_t trace_block;        /* block size of the persistent traversal kernels: 64, 128, 256 */
     int32_t persistent_blocks;  /* grid of the persistent traversal kernels; at most the          */

@@ -1,5 +1,5 @@
 // Bidirectional path tracing for gfx950: one thread per (pixel, sample), launched and gathered onto
-// the film exactly as the plain megakernel is (render.hip).
+// the film exactly as the plain path tracer's (render.hip).
 //
 // The reference has a bidirectional integrator (intergrators/BidirectionalPathIntegrator.cuh:1-665)
 // that its author disabled as not functional (LightTransportSimulation.cu:116-121): the light walk

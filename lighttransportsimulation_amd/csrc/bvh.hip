@@ -581,7 +581,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_small_sort(const float* __restr
 #pragma unroll
             for (int j = 0; j < kSmallRows; j++) {
                 const uint32_t d = (key[j] >> shift) & (kSmallBins - 1);
-                const uint32_t at = start[d] + cnt[wave][d] + rank[j];  // below 256 times the busy waves
+                const uint32_t at = start[d] + cnt[wave][d] + rank[j];  // below 64 kSmallRows times the busy waves
                 sKeys[at] = key[j];
                 sVals[at] = (uint16_t)val[j];
             }

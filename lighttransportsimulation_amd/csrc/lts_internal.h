@@ -109,7 +109,7 @@ struct RenderLaunch {
     int s0, s1;          // sample range of this pass
     float* sampleL;      // [s1 - s0][H][W][3] radiance of the pass
     float* film;         // [H][W][4] rgb + weight, accumulated across passes
-    unsigned long long* counters;  // optional [2]: node visits, triangle tests
+    unsigned long long* counters;  // optional [kTraceCounters]: node fetches and triangle tests of path, shadow and MIS rays
 };
 // Whole paths in one launch (paths.hip). work, other: kPathWork counters each; the launch takes work cleared
 // and clears other, so a context's launches alternate between two sets.
@@ -246,7 +246,7 @@ constexpr int kWfBounceBase = 32;
 constexpr int kWfPhaseEvents = 8 * kWfMaxBounce + 4;
 struct WfProfile { hipEvent_t ev[kWfPhaseEvents]; };
 // Traversal counters of a context: render-node fetches and triangle tests of path, shadow and MIS
-// rays (the megakernel uses the first two, for its path rays).
+// rays.
 constexpr int kTraceCounters = 6;
 
 // Workgroups of traceBlock threads in a trace launch of grid persistentBlocks.

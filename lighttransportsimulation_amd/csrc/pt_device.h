@@ -1,4 +1,4 @@
-// Path-tracer device routines shared by the megakernel and the wavefront kernels.
+// Path-tracer device routines shared by the whole-path, wavefront and bidirectional kernels.
 // Each routine restates a reference routine (tierChampion/LightTransportSimulation/src) with
 // the same fp32 evaluation order; see lts_device.h for the arithmetic conventions.
 #pragma once

@@ -3,13 +3,14 @@
 // The reference integrator (intergrators/PathTracingIntegrator.cuh:38-104 with estimateDirect,
 // IntegratorHelper.cuh:51-125) is cut at its three ray casts:
 //   extend   closest hit of every live path ray                     (persistent)
-//   shade    (by default in material order within chunks of the queue) emission, BSDF, light sample + MIS-BSDF sample (NEE set-up), continuation, roulette;
-//            appends one shadow ray and one MIS ray per path at most
+//   shade    (by default in material order within chunks of the queue) emission, BSDF, light sample + MIS-BSDF
+//            sample (NEE set-up), continuation, roulette; appends one shadow ray and one MIS ray per path at
+//            most; first completes the paths that ended at the bounce before
 //   shadow   any hit of the shadow rays                             (persistent, in extend's launch)
 //   mis      whether an MIS-BSDF ray reaches its light              (persistent, in extend's launch)
-//   finalize L += beta * ((Ld_light + Ld_bsdf) / p_pick), the reference's order of additions;
-//            terminated paths write their radiance
-// Each path's arithmetic is the megakernel's, so the image does not depend on queue order.
+//   finalize L += beta * ((Ld_light + Ld_bsdf) / p_pick), the reference's order of additions, for the paths that
+//            ended at the last bounce
+// Each path's arithmetic is that of whole paths (paths.hip), so the image does not depend on queue order or form.
 // Every count lives in device memory and is reset by kernels, so the bounce loop of a pass is
 // captured once in a hipGraph and replayed.
 #include <algorithm>

@@ -674,14 +674,13 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
         resolveMs += ms_between(c->ev[6], c->ev[7]);
         launches++;
         if (prof && p->max_bounce > 0) {
-            // the pass's first trace, then per bounce: sort, shade, trace, finalize
+            // the pass's first trace, then per bounce: shade, trace, finalize
             phase[LTS_PHASE_EXTEND] += ms_between(prof->ev[8 * kWfMaxBounce + 3], prof->ev[0]);
             for (int b = 0; b < p->max_bounce; b++) {
                 const hipEvent_t* e = prof->ev + 8 * b;
-                phase[LTS_PHASE_SORT] += ms_between(e[0], e[1]);
-                phase[LTS_PHASE_SHADE] += ms_between(e[1], e[2]);
-                phase[LTS_PHASE_EXTEND] += ms_between(e[2], e[3]);
-                phase[LTS_PHASE_FINALIZE] += ms_between(e[3], e[4]);
+                phase[LTS_PHASE_SHADE] += ms_between(e[0], e[1]);
+                phase[LTS_PHASE_EXTEND] += ms_between(e[1], e[2]);
+                phase[LTS_PHASE_FINALIZE] += ms_between(e[2], e[3]);
             }
             if (cached) {
                 const hipEvent_t* e = prof->ev + 8 * kWfMaxBounce;
@@ -718,10 +717,7 @@ int render_wavefront(lts_ctx* c, const std::vector<lts_ctx*>& scenes, const lts_
         if (prof && p->max_bounce > 0) {
             const int64_t perBounce = launches * p->max_bounce;
             st->phase_launches[LTS_PHASE_EXTEND] = perBounce + launches;
-            st->phase_launches[LTS_PHASE_SORT] = 0;
             st->phase_launches[LTS_PHASE_SHADE] = perBounce;
-            st->phase_launches[LTS_PHASE_SHADOW] = 0;
-            st->phase_launches[LTS_PHASE_MIS] = 0;
             st->phase_launches[LTS_PHASE_FINALIZE] = launches;
             st->phase_launches[LTS_PHASE_CACHE_INFER] = cached ? launches : 0;
             st->phase_launches[LTS_PHASE_CACHE_TRAIN] = cached ? launches * c->nrc.steps : 0;
@@ -1001,16 +997,16 @@ static int load_scene_impl(lts_ctx* c, const char* dir, const char* scene, const
     std::vector<ShadeTri> shadeLeaf(n);
     for (int k = 0; k < n; k++) shadeLeaf[k] = H.shade[perm[k]];
     HIPCHK(c, upload(&S.shade, shadeLeaf.data(), shadeLeaf.size(), s));
-    HIPCHK(c, launch_tri_materials(S.bvh.tris, S.shade, n, S.bvh.recs, nodes4 + n, s));
+    HIPCHK(c, launch_rec_materials(S.shade, n, S.bvh.recs, nodes4 + n, s));
     std::vector<LightDesc> lights = H.lights;
     for (LightDesc& L : lights)
         if (L.kind == 0) L.leaf = leafOf[L.prim];
     HIPCHK(c, upload(&S.lights, lights.data(), lights.size(), s));
     SceneView& v = S.view;
-    v.tris = S.bvh.tris; v.nodes = S.bvh.nodes; v.recs = S.bvh.recs; v.shade = S.shade; v.mats = S.mats; v.texs = S.texs;
+    v.tris = S.bvh.tris; v.recs = S.bvh.recs; v.shade = S.shade; v.mats = S.mats; v.texs = S.texs;
     v.mips = S.mips; v.mipData = S.mipData; v.lights = S.lights; v.lfunc = S.lfunc; v.lcdf = S.lcdf;
     v.funcInt = H.funcInt; v.nLights = (int)H.lights.size(); v.nPrim = n; v.infiniteLight = H.infiniteLight;
-    v.root = n == 1 ? INT32_MIN : 0;
+    v.root = n == 1 ? kTraceLeaf : 0;
     v.perm = c->perm;
     v.cam = H.cam;
     std::memcpy(v.filter, H.filter, sizeof(v.filter));

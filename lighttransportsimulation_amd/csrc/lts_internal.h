@@ -131,9 +131,9 @@ hipError_t launch_film_clear(float* film, int npix, hipStream_t stream);
 // ray i: origin at origins[stride i ..], direction at dirs[stride i ..]
 hipError_t launch_trace_rays(const SceneView& sv, const float* origins, const float* dirs, int stride, int n, int32_t* prim,
                              float* t, hipStream_t stream);
-// The material of each of the n leaves of a loaded scene (shade is in leaf order) into its triangle and
-// its render record (nRecs records).
-hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t stream);
+// The material of each of the n leaves of a loaded scene (shade is in leaf order) into its render record
+// (nRecs records).
+hipError_t launch_rec_materials(const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t stream);
 hipError_t launch_get_render(const SceneView& sv, const float* film, float* rgb, hipStream_t stream);
 // plain copy of `bytes` (a multiple of 16) with 16-byte vector loads and stores
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
@@ -239,8 +239,8 @@ constexpr int kWfGlobalBase = 0;   // [0] cache queries
 constexpr int kWfBounceBase = 32;
 
 // Optional phase timing: events recorded between the kernels of a pass launched directly (not
-// captured). ev[8 kWfMaxBounce + 3] precedes the pass's first trace; bounce b uses ev[8b + 0..4]:
-// two before shading, after shading, after the trace of the next path rays with this bounce's shadow
+// captured). ev[8 kWfMaxBounce + 3] precedes the pass's first trace; bounce b uses ev[8b + 0..3]:
+// before shading, after shading, after the trace of the next path rays with this bounce's shadow
 // and MIS rays, after the last bounce's finalize; the cached integrator's tail uses
 // ev[8 kWfMaxBounce + 0..2]: before inference, after inference, after the training steps.
 constexpr int kWfPhaseEvents = 8 * kWfMaxBounce + 4;

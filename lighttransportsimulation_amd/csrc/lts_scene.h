@@ -19,8 +19,7 @@ struct alignas(16) TriLeaf {
     float p1y, p1z, p2x, p2y;
     float p2z;
     int32_t prim;  // primitive number (global triangle order of the scene)
-    int32_t mat;   // material of the primitive (scenes; 0 after a standalone build)
-    int32_t pad1;
+    int32_t pad[2];
 };
 
 struct alignas(16) BvhNode {
@@ -47,6 +46,8 @@ struct alignas(16) TraceRec {
 };
 static_assert(sizeof(TraceRec) == 48, "TraceRec layout");
 constexpr int kRecUnits = 3;  // 16-byte units of a record
+// A traversal's stack entry is a record's offset in 16-byte units, with the sign bit set for a triangle.
+constexpr int kTraceLeaf = INT32_MIN;
 
 struct alignas(16) ShadeTri {
     float n[9];    // vertex normals (valid when hasN)
@@ -111,8 +112,7 @@ struct CameraDesc {
 // Everything the integrator kernels read, by device pointer.
 struct SceneView {
     const TriLeaf* tris;
-    const BvhNode* nodes;
-    const TraceRec* recs;    // 4-wide collapse of `nodes` with its triangles, root at 0 (used by the traversal)
+    const TraceRec* recs;    // render tree: 4-wide nodes and triangles, root at 0 (used by the traversal)
     const ShadeTri* shade;   // per BVH leaf: shade[k] belongs to the triangle tris[k]
     const MatDesc* mats;
     const TexDesc* texs;

@@ -111,8 +111,6 @@ constexpr int kStack = kTraceStack;
 // entries of a 256-lane block (22528 B) plus the 256 B of ray_held's marks let 7 trace blocks (7
 // waves per SIMD) share a CU's 160 KB of LDS.
 constexpr int kShortStack = 22;
-// A stack entry is a record's offset in 16-byte units, with the sign bit set for a triangle.
-constexpr int kTraceLeaf = INT32_MIN;
 constexpr int kTraceDone = -1;  // bottom of the stack: the traversal has ended
 
 // Traversal stack of one lane: entries [0, kShortStack) in LDS (entry e at lds[e * stride], so the

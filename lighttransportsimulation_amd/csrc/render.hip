@@ -7,14 +7,11 @@ namespace lts {
 
 namespace {
 
-__global__ __launch_bounds__(256) void k_tri_materials(TriLeaf* __restrict__ tris, const ShadeTri* __restrict__ shade, int n,
-                                                       TraceRec* __restrict__ recs, int nRecs) {
+__global__ __launch_bounds__(256) void k_rec_materials(const ShadeTri* __restrict__ shade, int n, TraceRec* __restrict__ recs, int nRecs) {
     const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k < n) tris[k].mat = shade[k].mat;
-    if (k < nRecs) {
-        const uint32_t leaf = recs[k].w[11];
-        if (leaf < (uint32_t)n) recs[k].w[10] = (uint32_t)shade[leaf].mat;
-    }
+    if (k >= nRecs) return;
+    const uint32_t leaf = recs[k].w[11];
+    if (leaf < (uint32_t)n) recs[k].w[10] = (uint32_t)shade[leaf].mat;
 }
 
 // Pixel (x, y) gathers, for each sample in order and each owner pixel (ox, oy) with ox in
@@ -98,10 +95,9 @@ hipError_t launch_film_gather(const SceneView& sv, const RenderLaunch& rl, hipSt
     return hipGetLastError();
 }
 
-hipError_t launch_tri_materials(TriLeaf* tris, const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t s) {
-    if (n < 1) return hipSuccess;
-    const int m = nRecs > n ? nRecs : n;
-    k_tri_materials<<<(m + 255) / 256, 256, 0, s>>>(tris, shade, n, recs, nRecs);
+hipError_t launch_rec_materials(const ShadeTri* shade, int n, TraceRec* recs, int nRecs, hipStream_t s) {
+    if (nRecs < 1) return hipSuccess;
+    k_rec_materials<<<(nRecs + 255) / 256, 256, 0, s>>>(shade, n, recs, nRecs);
     return hipGetLastError();
 }
 

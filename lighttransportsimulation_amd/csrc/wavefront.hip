@@ -727,7 +727,6 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
         int32_t* cnt = bounce0 + kWfCountsPerBounce * bounce;
         int32_t* nxt = cnt + kWfCountsPerBounce;
         mark(8 * bounce + 0);
-        mark(8 * bounce + 1);
         {
             auto shade = cached ? (bounce == 0 ? k_wf_shade<true, true> : k_wf_shade<true, false>)
                                 : (bounce == 0 ? k_wf_shade<false, true> : k_wf_shade<false, false>);
@@ -736,12 +735,12 @@ hipError_t wf_enqueue_pass(const WfBuffers& b, const WfTuning& t, int maxBounce,
                                                   cnt + 1, b.mis, cnt + 2, cached ? b.qRaw : nullptr, b.qMeta, qCount, b.tRec, b.tRaw,
                                                   b.done[q], cnt + 3, b.shadowQ, b.misQ);
         }
-        mark(8 * bounce + 2);
+        mark(8 * bounce + 1);
         // the next bounce's path rays (none after the last bounce) with this bounce's shadow and MIS rays
         trace(bounce + 1, nxt, cnt + 1, cnt + 2);
-        mark(8 * bounce + 3);
+        mark(8 * bounce + 2);
         if (bounce + 1 == maxBounce) k_wf_finalize<<<gridAll, 256, 0, s>>>(b.params, b.slots, b.paths, b.nee, b.done[q], cnt + 3);
-        mark(8 * bounce + 4);
+        mark(8 * bounce + 3);
     }
     if (cached) {
         mark(8 * kWfMaxBounce + 0);

@@ -417,8 +417,9 @@ LTS_D Spec bdpt_radiance(const SceneView& sv, bool inside, int px, int py, int s
 // the same index, and their rays are traced together (a ray at a time with every lane waiting for the longest,
 // and a light subpath for every sample: 4.18 ms for a 4-spp 641x361 frame of a 90k-triangle torus and 12.7 for
 // 16 spp, now 3.27 and 9.7; lanes that go on by themselves, as in whole paths: 7.2). It is bound by vector
-// instructions with a quarter of the lanes at work, as subpaths differ in length. Four waves per SIMD (128
-// VGPRs): 3.27 ms, 3.78 at three and 3.27 at five, where a spilling frame's memory grows.
+// instructions (0.46 per SIMD per 4 cycles) and private memory (half of the wave time waits on memory) with 24 %
+// of the lanes at work, as subpaths differ in length. Four waves per SIMD (128 VGPRs): 3.27 ms, 3.78 at three
+// and 3.27 at five, where a spilling frame's memory grows.
 __global__ __launch_bounds__(256, 4) void k_bdpt(SceneView sv, RenderLaunch rl) {
     __shared__ int lds[4][kWaveTraceWords];
     __shared__ NoiseTables perm;

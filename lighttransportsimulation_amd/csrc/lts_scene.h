@@ -2,7 +2,8 @@
 //
 // HBM layout of one loaded scene:
 //   tris     TriLeaf[n]   48 B  vertices in BVH leaf order (leaf k = k-th primitive in Morton order)
-//   nodes    BvhNode[n-1] 64 B  both child boxes + child indices (unified index space)
+//   nodes    BvhNode[n-1] 64 B  both child boxes + child indices (unified index space), for the build
+//   recs     TraceRec[..] 48 B  the render tree: 4-wide nodes and triangles, level by level
 //   shade    ShadeTri[n]  80 B  per leaf: normals, uvs, material, light (read once per hit)
 //   lights   LightDesc[L]       area lights in global triangle order, infinite light last
 //   mats/texs/mips              material, texture and mip-pyramid descriptors
